@@ -349,6 +349,21 @@ int warp_amd_normalize_dirichlet_projector(int scalar_size, int block_dim, int n
                                            const int* row_counts, const int* columns, void* values,
                                            void* fixed_values, void* stream);
 
+/* Dirichlet projection of a compact square matrix by a block-diagonal
+ * projector P (replaces the copies, products and sums of
+ * project_system_matrix, warp/_src/fem/dirichlet.py:93-104, where they keep
+ * the topology).  _check: out[0] (device) = rows of P that hold anything but
+ * one diagonal block, plus rows whose diagonal block A lacks; out[1] = blocks
+ * of A.  _blocks, valid for out[0] == 0: A := (I - P) A (I - P) + P in place,
+ * block_dim 1, 2 or 3, every product and sum rounded in the order of the
+ * general route; blocks with neither factor are not touched.  nnz only
+ * chooses the lanes per row. */
+int warp_amd_bsr_project_check(int nrow, const int* a_offsets, const int* a_columns, const int* p_offsets,
+                               const int* p_columns, int* out, void* stream);
+int warp_amd_bsr_project_blocks(int scalar_size, int block_dim, int nrow, int64_t nnz, const int* a_offsets,
+                                const int* a_columns, void* a_values, const int* p_offsets, const void* p_values,
+                                void* stream);
+
 /* x[0..n) *= alpha, fp32 (4) or fp64 (8) (bsr_scale's value kernel). */
 int warp_amd_scale_values(int scalar_size, int64_t n, void* x, double alpha, void* stream);
 

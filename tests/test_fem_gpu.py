@@ -113,3 +113,71 @@ def test_projected_system_solves_with_cg(device):
     res = sparse.bsr_mv(A, x, alpha=-1.0)
     res += rhs
     assert float(res.norm() / rhs.norm()) < 1e-5
+
+
+@pytest.mark.parametrize("case", ["diagonal", "off_diagonal", "missing_diagonal", "empty_projector"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("br", [1, 2, 3])
+def test_projection_in_place_equals_general_route(device, br, dtype, case, monkeypatch):
+    """A block-diagonal projector on A's diagonal takes the in-place pass; it and
+    every other projector give the values of the general products and sums
+    (same operations, same order: equal, not close), NaN and infinities kept."""
+    from warp_amd.fem import dirichlet
+
+    g = torch.Generator().manual_seed(7 * br)
+    n = 67
+    rows = torch.arange(n).repeat_interleave(9)
+    cols = (rows + torch.randint(-20, 21, rows.shape, generator=g)).clamp(0, n - 1)
+    diag = torch.arange(n) if case != "missing_diagonal" else torch.arange(0)
+    if case == "missing_diagonal":
+        rows, cols = rows[rows != cols], cols[rows != cols]
+    rows, cols = torch.cat([rows, diag]), torch.cat([cols, diag])
+    vals = torch.randn((rows.numel(), br, br), generator=g, dtype=torch.float64).to(dtype)
+    vals[5, 0, 0], vals[6, 0, 0], vals[7] = float("inf"), float("nan"), 0.0
+    keep = torch.nonzero(torch.rand(n, generator=g) < 0.4).reshape(-1)
+    pcols = keep.clone()
+    if case == "off_diagonal":
+        pcols[0] = (pcols[0] + 1) % n
+    pvals = torch.randn((keep.numel(), br, br), generator=g, dtype=torch.float64).to(dtype)
+    btype = wa.types.type_to_scalar(dtype) if br == 1 else wa.matrix((br, br), wa.types.type_to_scalar(dtype))
+
+    def build(r, c, v):
+        M = sparse.bsr_zeros(n, n, btype, device=device)
+        v = v.reshape(-1) if br == 1 else v
+        sparse.bsr_set_from_triplets(M, r.to(torch.int32).to(device), c.to(torch.int32).to(device),
+                                     v.contiguous().to(device))
+        return M
+
+    results = []
+    for general in (False, True):
+        A, P = build(rows, cols, vals), build(keep, pcols, pvals)
+        if case == "empty_projector":
+            P = sparse.bsr_zeros(n, n, btype, device=device)
+        if general:
+            monkeypatch.setattr(dirichlet, "_project_in_place", lambda A, P: False)
+        else:
+            probe = build(rows, cols, vals)
+            assert dirichlet._project_in_place(probe, P) == (case == "diagonal")
+        fem.project_system_matrix(A, P)
+        nnz = A.nnz_sync()
+        results.append((A.offsets.cpu(), A.columns[:nnz].cpu(), A.values[:nnz].cpu(), A.nnz))
+    (o0, c0, v0, n0), (o1, c1, v1, n1) = results
+    assert n0 == n1 and torch.equal(o0, o1) and torch.equal(c0, c1)
+    torch.testing.assert_close(v0, v1, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1029])
+def test_copy_and_rescale_vector_tails(device, n, shift, dtype):
+    """Value copies at the remainders of the 16-byte pass and at storage that is not 16-byte aligned."""
+    btype = wa.types.type_to_scalar(dtype)
+    A = sparse.bsr_identity(n, btype, device=device)
+    store = torch.randn(n + shift + 5, dtype=dtype, device=device)
+    A.values = store[shift:shift + n]
+    before = store.clone()
+    C = sparse.bsr_copy(3.0 * A)
+    assert torch.equal(C.values[:n], 3.0 * A.values[:n])
+    sparse.bsr_axpy(sparse.bsr_identity(n, btype, device=device), A, alpha=2.0, beta=0.5)
+    assert torch.equal(A.values[:n], 0.5 * before[shift:shift + n] + 2.0)
+    assert torch.equal(store[shift + n:], before[shift + n:]) and torch.equal(store[:shift], before[:shift])

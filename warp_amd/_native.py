@@ -131,6 +131,8 @@ _SIGNATURES = {
     "warp_amd_bsr_diag_topology": (c_int, [c_int, c_int, c_ptr, c_ptr, c_ptr]),
     "warp_amd_axpby": (c_int, [c_int, c_i64, c_f64, c_ptr, c_f64, c_ptr, c_ptr]),
     "warp_amd_normalize_dirichlet_projector": (c_int, [c_int, c_int, c_int] + [c_ptr] * 6),
+    "warp_amd_bsr_project_check": (c_int, [c_int] + [c_ptr] * 6),
+    "warp_amd_bsr_project_blocks": (c_int, [c_int, c_int, c_int, c_i64] + [c_ptr] * 6),
     "warp_amd_bsr_residual_workspace_size": (c_size, [c_int]),
     "warp_amd_bsr_residual_f32_f64": (c_int, [c_int, c_int, c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_size, c_ptr]),
     "warp_amd_bsr_residual_f32_f64_noalloc": (c_int, [c_int, c_int, c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr]),

@@ -7,6 +7,7 @@
 // built by the triplet assembly (one triplet per destination sub-block).
 #include "common.h"
 
+#include <algorithm>
 #include <climits>
 
 namespace wa {
@@ -833,6 +834,193 @@ template <typename S> __global__ __launch_bounds__(kBlock) void rescale_kernel(i
     }
 }
 
+// The same two passes over one scalar type in 16-byte vectors: one vector per
+// thread, and the n % kV last scalars by the first threads.  Bound by HBM;
+// what limits a 4-byte-per-lane pass is the request rate.  On the 64.7M
+// scalars of the 64^3 elasticity matrix (518 MB moved): 139 us at 4 bytes per
+// lane, 87 with plain 16-byte accesses (8 vectors per thread: 130), 79 us
+// (6.5 TB/s) with non-temporal ones, which keep the once-touched stream from
+// displacing what the next kernel reads.
+template <typename S> struct Vec16 {
+    static constexpr int kV = 16 / (int)sizeof(S);
+    typedef S type __attribute__((ext_vector_type(16 / sizeof(S))));
+};
+
+template <typename S>
+__global__ __launch_bounds__(kBlock) void copy_scaled_vec_kernel(int64_t n, const S* __restrict__ src, S scale,
+                                                                S* __restrict__ dst)
+{
+    typedef typename Vec16<S>::type V;
+    constexpr int kV = Vec16<S>::kV;
+    const int64_t nv = n / kV;
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < nv) {
+        V v = __builtin_nontemporal_load(reinterpret_cast<const V*>(src) + i);
+#pragma unroll
+        for (int k = 0; k < kV; ++k)
+            v[k] = scale * v[k];
+        __builtin_nontemporal_store(v, reinterpret_cast<V*>(dst) + i);
+    }
+    if (i < n - nv * kV)
+        dst[nv * kV + i] = scale * src[nv * kV + i];
+}
+
+template <typename S>
+__global__ __launch_bounds__(kBlock) void rescale_vec_kernel(int64_t n, S* __restrict__ x, S beta)
+{
+#pragma clang fp contract(off)
+    typedef typename Vec16<S>::type V;
+    constexpr int kV = Vec16<S>::kV;
+    const S zero = S(0);
+    const int64_t nv = n / kV;
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < nv) {
+        V v = __builtin_nontemporal_load(reinterpret_cast<const V*>(x) + i);
+#pragma unroll
+        for (int k = 0; k < kV; ++k)
+            v[k] = zero + beta * v[k];
+        __builtin_nontemporal_store(v, reinterpret_cast<V*>(x) + i);
+    }
+    if (i < n - nv * kV)
+        x[nv * kV + i] = zero + beta * x[nv * kV + i];
+}
+
+// Workgroups of a vector pass over n scalars (at least one, for the tail).
+template <typename S> unsigned vec_blocks(int64_t n)
+{
+    return (unsigned)std::max<int64_t>(1, ceil_div(n / Vec16<S>::kV, kBlock));
+}
+
+inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// Block-diagonal projectors ---------------------------------------------------
+
+// out[0] += rows of P that hold anything but one diagonal block, plus rows
+// whose diagonal block is missing from A; out[1] = blocks of A.
+__global__ __launch_bounds__(kBlock) void project_check_kernel(int nrow, const int* __restrict__ a_offsets,
+                                                              const int* __restrict__ a_columns,
+                                                              const int* __restrict__ p_offsets,
+                                                              const int* __restrict__ p_columns, int* __restrict__ out)
+{
+    __shared__ int lds_count;
+    if (threadIdx.x == 0)
+        lds_count = 0;
+    __syncthreads();
+    const int r = blockIdx.x * kBlock + threadIdx.x;
+    if (r < nrow) {
+        const int pb = p_offsets[r], np = p_offsets[r + 1] - pb;
+        if (np != 0 && (np != 1 || p_columns[pb] != r || find_block(a_offsets, nullptr, a_columns, r, r) < 0))
+            atomicAdd(&lds_count, 1);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (lds_count)
+            atomicAdd(out, lds_count);
+        if (blockIdx.x == 0)
+            out[1] = a_offsets[nrow];
+    }
+}
+
+// A := (I - P) A (I - P) + P in place for a block-diagonal P, G lanes per row
+// of A.  A block (r, c) changes only where P holds (r, r) or (c, c): the pass
+// reads A's columns (and P's offsets, which stay in L2) and touches the values
+// of those blocks alone.  Each goes through the operations of the general
+// route, rounded one by one in its order: c = (0 + a) - P_r a, + P_r on the
+// diagonal, then - c P_c (oracle order of bsr_mm; an absent factor contributes
+// + 0 * -1).  Copy and projection of the 64^3 elasticity system with two
+// constrained faces: 1867 us by products, copies and sums of whole matrices,
+// 282 us so (the copy and the right-hand side's product are most of it).
+template <typename S, int BR, int G>
+__global__ __launch_bounds__(kBlock) void project_blocks_kernel(int nrow, const int* __restrict__ a_offsets,
+                                                               const int* __restrict__ a_columns,
+                                                               S* __restrict__ a_values,
+                                                               const int* __restrict__ p_offsets,
+                                                               const S* __restrict__ p_values)
+{
+#pragma clang fp contract(off)
+    const int64_t row = (int64_t)blockIdx.x * (kBlock / G) + threadIdx.x / G;
+    if (row >= nrow)
+        return;
+    const int r = (int)row;
+    const int lane = threadIdx.x % G;
+    const int pr = p_offsets[r];
+    const bool has_r = p_offsets[r + 1] > pr;
+    const int end = a_offsets[r + 1];
+    for (int b = a_offsets[r] + lane; b < end; b += G) {
+        const int c = a_columns[b];
+        if (c < 0 || c >= nrow)
+            continue;
+        const int pc = p_offsets[c];
+        const bool has_c = p_offsets[c + 1] > pc;
+        if (!has_r && !has_c)
+            continue;
+        S* blk = a_values + (size_t)b * (BR * BR);
+        S left[BR * BR], v[BR * BR];
+#pragma unroll
+        for (int e = 0; e < BR * BR; ++e) {
+            v[e] = blk[e];
+            left[e] = S(0);
+        }
+        if (has_r) {
+            const S* m = p_values + (size_t)pr * (BR * BR);
+#pragma unroll
+            for (int i = 0; i < BR; ++i)
+#pragma unroll
+                for (int j = 0; j < BR; ++j) {
+                    S prod = m[i * BR] * v[j];
+#pragma unroll
+                    for (int k = 1; k < BR; ++k)
+                        prod = prod + m[i * BR + k] * v[k * BR + j];
+                    left[i * BR + j] = left[i * BR + j] + prod;
+                }
+        }
+#pragma unroll
+        for (int e = 0; e < BR * BR; ++e)
+            v[e] = (S(0) + v[e]) + S(-1) * left[e];
+        S out[BR * BR];
+#pragma unroll
+        for (int e = 0; e < BR * BR; ++e)
+            out[e] = S(0) + v[e];
+        if (c == r) {
+            const S* m = p_values + (size_t)pr * (BR * BR);
+#pragma unroll
+            for (int e = 0; e < BR * BR; ++e)
+                out[e] += m[e];
+        }
+        if (has_c) {
+            const S* m = p_values + (size_t)pc * (BR * BR);
+#pragma unroll
+            for (int i = 0; i < BR; ++i)
+#pragma unroll
+                for (int j = 0; j < BR; ++j) {
+                    S prod = v[i * BR] * m[j];
+#pragma unroll
+                    for (int k = 1; k < BR; ++k)
+                        prod = prod + v[i * BR + k] * m[k * BR + j];
+                    const S acc = S(0) + prod;
+                    out[i * BR + j] = (S(0) + out[i * BR + j]) + S(-1) * acc;
+                }
+        }
+#pragma unroll
+        for (int e = 0; e < BR * BR; ++e)
+            blk[e] = out[e];
+    }
+}
+
+template <typename S, int BR>
+void launch_project(int nrow, int lanes, const int* a_offsets, const int* a_columns, void* a_values,
+                    const int* p_offsets, const void* p_values, hipStream_t s)
+{
+#define WA_PROJECT(G)                                                                                                 \
+    project_blocks_kernel<S, BR, G><<<(unsigned)ceil_div(nrow, kBlock / G), kBlock, 0, s>>>(                          \
+        nrow, a_offsets, a_columns, static_cast<S*>(a_values), p_offsets, static_cast<const S*>(p_values))
+    if (lanes >= 32)
+        WA_PROJECT(32);
+    else
+        WA_PROJECT(8);
+#undef WA_PROJECT
+}
+
 // Number of pairs (rows[i], cols[i]), rows[i] >= 0, with no block in the
 // matrix, added to *missing (one atomic per workgroup).
 __global__ __launch_bounds__(kBlock) void count_missing_kernel(int64_t n, const int* __restrict__ rows,
@@ -1047,6 +1235,16 @@ WA_API int warp_amd_copy_scaled_values(int src_scalar_size, int dst_scalar_size,
     WA_REQUIRE(src && dst, "copy_scaled_values: null array");
     const unsigned grid = (unsigned)wa::ceil_div(n, wa::kBlock);
     hipStream_t s = wa::as_stream(stream);
+    if (src_scalar_size == dst_scalar_size && wa::aligned16(src) && wa::aligned16(dst)) {
+        if (src_scalar_size == 4)
+            wa::copy_scaled_vec_kernel<float><<<wa::vec_blocks<float>(n), wa::kBlock, 0, s>>>(
+                n, static_cast<const float*>(src), (float)scale, static_cast<float*>(dst));
+        else
+            wa::copy_scaled_vec_kernel<double><<<wa::vec_blocks<double>(n), wa::kBlock, 0, s>>>(
+                n, static_cast<const double*>(src), scale, static_cast<double*>(dst));
+        WA_LAUNCH_CHECK();
+        return wa::kOk;
+    }
 #define WA_COPY(SS, DS)                                                                                               \
     wa::copy_scaled_kernel<SS, DS><<<grid, wa::kBlock, 0, s>>>(n, static_cast<const SS*>(src), (SS)scale,             \
                                                                static_cast<DS*>(dst))
@@ -1072,10 +1270,64 @@ WA_API int warp_amd_rescale_values(int scalar_size, int64_t n, void* x, double b
     WA_REQUIRE(x != nullptr, "rescale_values: null array");
     const unsigned grid = (unsigned)wa::ceil_div(n, wa::kBlock);
     hipStream_t s = wa::as_stream(stream);
+    if (wa::aligned16(x)) {
+        if (scalar_size == 4)
+            wa::rescale_vec_kernel<float><<<wa::vec_blocks<float>(n), wa::kBlock, 0, s>>>(n, static_cast<float*>(x),
+                                                                                       (float)beta);
+        else
+            wa::rescale_vec_kernel<double><<<wa::vec_blocks<double>(n), wa::kBlock, 0, s>>>(
+                n, static_cast<double*>(x), beta);
+        WA_LAUNCH_CHECK();
+        return wa::kOk;
+    }
     if (scalar_size == 4)
         wa::rescale_kernel<float><<<grid, wa::kBlock, 0, s>>>(n, static_cast<float*>(x), (float)beta);
     else
         wa::rescale_kernel<double><<<grid, wa::kBlock, 0, s>>>(n, static_cast<double*>(x), beta);
+    WA_LAUNCH_CHECK();
+    return wa::kOk;
+}
+
+WA_API int warp_amd_bsr_project_check(int nrow, const int* a_offsets, const int* a_columns, const int* p_offsets,
+                                      const int* p_columns, int* out, void* stream)
+{
+    WA_REQUIRE(nrow > 0, "bsr_project_check: invalid row count %d", nrow);
+    WA_REQUIRE(a_offsets && a_columns && p_offsets && p_columns && out, "bsr_project_check: null array");
+    hipStream_t s = wa::as_stream(stream);
+    WA_TRY(wa::launch_fill_i32(out, 2, 0, s));
+    wa::project_check_kernel<<<(unsigned)wa::ceil_div(nrow, wa::kBlock), wa::kBlock, 0, s>>>(
+        nrow, a_offsets, a_columns, p_offsets, p_columns, out);
+    WA_LAUNCH_CHECK();
+    return wa::kOk;
+}
+
+WA_API int warp_amd_bsr_project_blocks(int scalar_size, int block_dim, int nrow, int64_t nnz, const int* a_offsets,
+                                       const int* a_columns, void* a_values, const int* p_offsets,
+                                       const void* p_values, void* stream)
+{
+    WA_REQUIRE(nrow > 0 && block_dim >= 1 && block_dim <= 3, "bsr_project_blocks: unsupported shape (%d rows, %d)",
+               nrow, block_dim);
+    WA_REQUIRE(scalar_size == 4 || scalar_size == 8, "bsr_project_blocks: values must be fp32 or fp64");
+    WA_REQUIRE(a_offsets && a_columns && a_values && p_offsets && p_values, "bsr_project_blocks: null array");
+    hipStream_t s = wa::as_stream(stream);
+    // a lane per block of a mean row: 32 lanes from 16 blocks on (27-block rows), 8 below (7 and 9)
+    const int lanes = nnz > (int64_t)16 * nrow ? 32 : 8;
+#define WA_PROJECT_DIM(S, BR)                                                                                         \
+    case BR: wa::launch_project<S, BR>(nrow, lanes, a_offsets, a_columns, a_values, p_offsets, p_values, s); break;
+    if (scalar_size == 4) {
+        switch (block_dim) {
+            WA_PROJECT_DIM(float, 1)
+            WA_PROJECT_DIM(float, 2)
+            WA_PROJECT_DIM(float, 3)
+        }
+    } else {
+        switch (block_dim) {
+            WA_PROJECT_DIM(double, 1)
+            WA_PROJECT_DIM(double, 2)
+            WA_PROJECT_DIM(double, 3)
+        }
+    }
+#undef WA_PROJECT_DIM
     WA_LAUNCH_CHECK();
     return wa::kOk;
 }

@@ -68,8 +68,47 @@ def project_system_rhs(system_matrix: BsrMatrix, system_rhs: torch.Tensor, proje
     bsr_mv(A=projector_matrix, x=rhs_tmp, y=system_rhs, alpha=-1.0, beta=1.0)
 
 
+def _project_in_place(A: BsrMatrix, P: BsrMatrix) -> bool:
+    """The projection of a compact ``A`` by a block-diagonal ``P`` whose blocks all lie on ``A``'s diagonal: the
+    topology stays, and only the blocks of constrained rows and columns are read and written.  False, with nothing
+    done, where that does not hold; the check reads two counts back, so never under graph capture."""
+    if (
+        A is P
+        or A.row_counts is not None
+        or P.row_counts is not None
+        or A.block_shape != P.block_shape
+        or A.block_shape not in ((1, 1), (2, 2), (3, 3))
+        or A.scalar_type != P.scalar_type
+        or A.scalar_type.torch_dtype not in (torch.float32, torch.float64)
+        or not A.nrow == A.ncol == P.nrow == P.ncol
+        or A.values.device != P.values.device
+        or min(A.nrow, int(A.nnz), int(P.nnz)) == 0
+        or not (A.values.is_contiguous() and P.values.is_contiguous())
+        or A.values.data_ptr() == P.values.data_ptr()
+    ):
+        return False
+    _require_gpu(A.device, "project_system_matrix")
+    if torch.cuda.is_current_stream_capturing():
+        return False
+    out = torch.empty(2, dtype=torch.int32, device=A.device)
+    stream = _native.stream_of(A.device)
+    a_off, a_col, p_off = _native.ptr(A.offsets), _native.ptr(A.columns), _native.ptr(P.offsets)
+    _native.call("warp_amd_bsr_project_check", A.nrow, a_off, a_col, p_off, _native.ptr(P.columns),
+                 _native.ptr(out), stream)
+    foreign, nnz = out.tolist()
+    if foreign or nnz > min(A.columns.numel(), A.values.shape[0]):
+        return False
+    A.nnz, A._nnz_pending = nnz, False
+    A.values[nnz:].zero_()
+    _native.call("warp_amd_bsr_project_blocks", A.scalar_type.size, A.block_shape[0], A.nrow, nnz, a_off, a_col,
+                 _native.ptr(A.values), p_off, _native.ptr(P.values), stream)
+    return True
+
+
 def project_system_matrix(system_matrix: BsrMatrix, projector_matrix: BsrMatrix) -> None:
     """``A = (I - P) A (I - P) + P`` in place (dirichlet.py:93-104)."""
+    if _project_in_place(system_matrix, projector_matrix):
+        return
     complement_system = bsr_copy(system_matrix)
     bsr_mm(x=projector_matrix, y=system_matrix, z=complement_system, alpha=-1.0, beta=1.0)
     bsr_assign(dest=system_matrix, src=complement_system)
