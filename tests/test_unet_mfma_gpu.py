@@ -270,3 +270,27 @@ def test_pack_input_bf16_vs_torch_rounding(device, nvox, offset):
     torch.cuda.synchronize()
     want = torch.stack([(r_h[offset:] * 0.37).float().to(torch.bfloat16), k_h[offset:].to(torch.bfloat16)], 1)
     assert torch.equal(out.cpu(), want.view(torch.int16).reshape(-1))
+
+
+@pytest.mark.parametrize("accumulate", [0, 8])
+@pytest.mark.parametrize("ci,co", [(1, 16), (16, 32)])
+def test_conv_f32_output_alignment(device, ci, co, accumulate):
+    """FP32 outputs through 16-byte stores (aligned) and 4-byte stores (an output shifted by one float): same bits."""
+    m = 12
+    rng = np.random.default_rng(3 * ci + co)
+    x = _bf16_tensor(rng.standard_normal((m, m, m, ci)), device)
+    W = torch.tensor(rng.standard_normal((27, ci, co)).astype(np.float32), device=device)
+    wsw = torch.empty(_native.lib().warp_amd_conv3_mfma_weight_size(ci, co), dtype=torch.uint8, device=device)
+    s = _native.stream_of(device)
+    _native.call("warp_amd_conv3_mfma_swizzle", ci, co, 0, _native.ptr(W), _native.ptr(wsw), s)
+    base = torch.tensor(rng.standard_normal(m**3 * co).astype(np.float32), device=device)
+    outs = []
+    for shift in (0, 1):
+        store = torch.full((m**3 * co + 8,), 7.0, dtype=torch.float32, device=device)
+        y = store[shift:shift + m**3 * co]
+        y.copy_(base)
+        _native.call("warp_amd_conv3_mfma", m, ci, co, 0, _native.ptr(x), None, _native.ptr(wsw), None, 4 | accumulate,
+                     None, _native.ptr(y), None, s)
+        assert torch.all(store[:shift] == 7.0) and torch.all(store[shift + m**3 * co:] == 7.0)
+        outs.append(y.clone())
+    assert torch.equal(outs[0], outs[1])
