@@ -740,6 +740,10 @@ int warp_amd_unet_pack_input_bf16(int64_t nvox, const double* r, const float* lo
  * rounded as the forward rounds it); dy: FP32 [m^3][cout], rounded to BF16; FP32
  * accumulation; per-workgroup partials in the workspace added in a fixed order.
  * Channel pairs: 2-16, 16-32, 32-64, 64-64, 64-32, 32-16, 16-1. */
+size_t warp_amd_conv3_mfma_wgrad_bf16_workspace_size(int m, int cin, int cout);
+int warp_amd_conv3_mfma_wgrad_bf16(int m, int cin, int cout, int in_mode, const void* x, const void* coarse,
+                                   const void* dy, float* dW, float* db, void* workspace, size_t workspace_bytes,
+                                   void* stream);
 size_t warp_amd_conv3_mfma_wgrad_workspace_size(int m, int cin, int cout);
 int warp_amd_conv3_mfma_wgrad(int m, int cin, int cout, int in_mode, const void* x, const void* coarse,
                               const float* dy, float* dW, float* db, void* workspace, size_t workspace_bytes,

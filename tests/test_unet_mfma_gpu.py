@@ -294,3 +294,41 @@ def test_conv_f32_output_alignment(device, ci, co, accumulate):
         assert torch.all(store[:shift] == 7.0) and torch.all(store[shift + m**3 * co:] == 7.0)
         outs.append(y.clone())
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("ci,co,m,up", [(2, 16, 100, False), (16, 1, 100, True), (16, 1, 100, False), (16, 32, 60, False),
+                                        (32, 16, 52, True), (64, 64, 44, False), (16, 32, 4, False), (2, 16, 4, False)])
+def test_wgrad_bf16_many_tiles(device, ci, co, m, up):
+    """Weight gradients from a BF16 dy where every workgroup walks several
+    tiles (and at the smallest grid), tiles reaching past the grid included,
+    against float64 sums over the same BF16 operands: FP32 accumulation of at
+    most 2e6 products, error within 2e-5 of the sum of absolute products."""
+    g = torch.Generator(device=device).manual_seed(ci + co + m)
+
+    def field(side, ch):
+        return torch.randn((side, side, side, ch), generator=g, device=device).to(torch.bfloat16)
+
+    x, dy = field(m, ci), field(m, co)
+    coarse = field(m // 2, ci) if up else None
+    xin = x
+    if up:
+        fine = coarse.float().repeat_interleave(2, 0).repeat_interleave(2, 1).repeat_interleave(2, 2)
+        xin = (x.float() + fine).to(torch.bfloat16)
+    xp = torch.nn.functional.pad(xin.double(), (0, 0, 1, 1, 1, 1, 1, 1))
+    d = dy.double().reshape(-1, co)
+    want, size = [], []
+    for t in range(27):
+        dz, ddy, dx = t // 9, (t // 3) % 3, t % 3
+        xs = xp[dz:dz + m, ddy:ddy + m, dx:dx + m].reshape(-1, ci)
+        want.append(xs.T @ d)
+        size.append(xs.abs().T @ d.abs())
+    want, size = torch.stack(want), torch.stack(size)
+    nbytes = _native.lib().warp_amd_conv3_mfma_wgrad_bf16_workspace_size(m, ci, co)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    dW = torch.full((27, ci, co), float("nan"), device=device)
+    db = torch.full((co,), float("nan"), device=device)
+    _native.call("warp_amd_conv3_mfma_wgrad_bf16", m, ci, co, 1 if up else 0, _native.ptr(x), _native.ptr(coarse),
+                 _native.ptr(dy), _native.ptr(dW), _native.ptr(db), _native.ptr(ws), ws.numel(),
+                 _native.stream_of(device))
+    assert bool(((dW.double() - want).abs() <= 2e-5 * size + 1e-30).all())
+    assert bool(((db.double() - d.sum(0)).abs() <= 2e-5 * d.abs().sum(0) + 1e-30).all())

@@ -191,6 +191,11 @@ _SIGNATURES = {
         c_int,
         [c_int, c_int, c_int, c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_size, c_ptr],
     ),
+    "warp_amd_conv3_mfma_wgrad_bf16_workspace_size": (c_size, [c_int, c_int, c_int]),
+    "warp_amd_conv3_mfma_wgrad_bf16": (
+        c_int,
+        [c_int, c_int, c_int, c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_size, c_ptr],
+    ),
     "warp_amd_relu_mask_bf16": (c_int, [c_i64, c_ptr, c_ptr, c_ptr, c_ptr]),
     "warp_amd_f32_to_bf16": (c_int, [c_i64, c_ptr, c_ptr, c_ptr]),
     "warp_amd_bf16_to_f32": (c_int, [c_i64, c_ptr, c_ptr, c_ptr]),

@@ -29,6 +29,7 @@
 // several taps into one 8-wide k slot: k = tap * CI + ci.
 #include "common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace wa {
@@ -780,99 +781,208 @@ __global__ void pack_input_bf16_x4_kernel(int64_t nquad, const double* __restric
 //   dW[t][ci][co] = sum_v x~[v + d_t][ci] dy[v][co],   db[co] = sum_v dy[v][co]
 //
 // with x~ the layer input as the forward saw it (x, or x + upsample(coarse)
-// rounded to BF16) and dy the FP32 output gradient, rounded to BF16 for the
-// MFMA (v_mfma_f32_16x16x32_bf16, FP32 accumulation).  GEMM per workgroup
-// tile of 8 x 8 x 4 voxels: C[g][co] += A[g][k] B[k][co], k = 32 voxels (four
-// x rows of 8), rows g = (tap, input channel) with g = t * CI + ci, and row
-// 27 * CI a row of ones whose C row is db.  A lane's A operand is the 8
-// voxels of one x row of the input shifted by its row's tap; three copies of
-// the halo pre-shifted by dx = -1, 0, 1 (copy s holds halo x = s .. s + 7)
-// keep that read 16-byte aligned.  Its B operand is the same 8 voxels of dy
-// for one output channel (dy staged channel-major).  Rows are cut in blocks
-// of 16: for CI >= 16 one block per tap and 16-channel group (workgroups
-// split the channel groups) plus the ones block in group 0; for CI <= 2 the
-// 27 * CI + 1 rows in order.  The four waves of a workgroup take every fourth
-// row block.  Workgroups are persistent over their tiles, sum in registers,
-// and write one partial [27 * CI + 1][CO_pad] each; wgrad_sum_kernel adds
-// the partials in a fixed order.
-constexpr int kWgXS = 6 * 10 * 8 * 2 + 16;  // bytes per (copy, channel) of the shifted halo (+16 padding)
-constexpr int kWgDS = 32 * 8 * 2 + 16;       // bytes per output channel of the dy tile (+16 padding)
-constexpr int kWgMaxSlots = 256;             // workgroups per channel group
+// rounded to BF16) and dy the output gradient in BF16
+// (v_mfma_f32_16x16x32_bf16, FP32 accumulation).  The sum runs over voxels, so
+// both operands need 8 voxels of one channel per lane where memory holds the
+// channels of one voxel: the tiles lie in LDS as they lie in memory and
+// ds_read_b64_tr_b16 transposes on the way to the registers (a group of 16
+// lanes reads 4 voxels x 16 channels, lane n receives channel n of the four).
+// A tap is then only another voxel offset.  Storing them transposed instead
+// took three copies of the halo, each pre-shifted by one voxel, in 2-byte LDS
+// stores.
+//
+// k order: k block kb covers the tile's x rows 4 kb .. 4 kb + 3; lane group q
+// holds voxels 4 (q % 2) .. + 3 of row 4 kb + q / 2 and of row 4 kb + 2 + q / 2,
+// so that one read instruction covers consecutive voxels.
+//
+// Workgroups are persistent over their 8 x 8 x 4 tiles, load the next tile
+// into registers while the MFMAs of the current one run, sum in registers and
+// write one partial each; wgrad_sum_kernel adds the partials in a fixed order.
+// Kernel time per layer of the 128^3 network, before (three shifted copies,
+// every load waited for in turn, at most 256 workgroups) and now, in us:
+// 16 -> 1 245 / 28.6, 2 -> 16 151 / 27.7, 32 -> 16 45 / 21.4, 16 -> 32 45 / 17.5,
+// 32 -> 64 22 / 14.7, 64 -> 32 21 / 14.3, 64 -> 64 18 / 12.1; the sums of the
+// partials 46 / 10.6 on average.  The first and last layer now read their 75 MB
+// at 2.7 TB/s, the others are bound by the latency of one tile at one or two
+// workgroups per compute unit.
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 
-__host__ __device__ constexpr int wg_channels(int ci) { return ci >= 16 ? 16 : ci; }
-__host__ __device__ constexpr int wg_groups(int ci) { return ci >= 16 ? ci / 16 : 1; }
-__host__ __device__ constexpr int wg_row_blocks(int ci) { return ci >= 16 ? 28 : (27 * ci + 1 + 15) / 16; }
-__host__ __device__ constexpr int wg_rows(int ci) { return 27 * ci + 1; }
-
-template <int CI, int CO, int IN>
-__global__ __launch_bounds__(kBlock) void conv3_wgrad_mfma_kernel(int m, const unsigned short* __restrict__ x,
-                                                                  const unsigned short* __restrict__ coarse,
-                                                                  const float* __restrict__ dy, int nslots,
-                                                                  float* __restrict__ partial)
+__device__ __forceinline__ bf16x4 lds_read_tr(const unsigned char* p)
 {
-    constexpr int CH = wg_channels(CI);
-    constexpr int NCG = wg_groups(CI);
-    constexpr int NRB = wg_row_blocks(CI);
-    constexpr int RBW = (NRB + 3) / 4;  // row blocks per wave
-    constexpr int CBN = c_blocks(CO);
-    constexpr int COP = 16 * CBN;
-    constexpr int ROWS = wg_rows(CI);
-    constexpr int kXBytes = 3 * CH * kWgXS;
-    constexpr int kDyOff = kXBytes;
-    constexpr int kBytes = kDyOff + COP * kWgDS;
-    static_assert(kBytes <= 160 * 1024, "LDS budget");
-    __shared__ __attribute__((aligned(16))) unsigned char smem[kBytes];
-    unsigned char* xs = smem;
-    unsigned char* dys = smem + kDyOff;
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_bf16x4*)p);
+}
 
-    const int cg = (int)blockIdx.x % NCG;  // channel group: input channels 16 cg .. (CI >= 16)
-    const int slot = (int)blockIdx.x / NCG;
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const int ln = lane % 16, kq = lane / 16;
-    const int tiles_x = (m + kTX - 1) / kTX;
-    const int tiles_xy = tiles_x * tiles_x;
-    const int ntiles = tiles_xy * (m / kTZ);
-    const int mh = m / 2;
+__device__ __forceinline__ mfma_bf16x8 join8(bf16x4 lo, bf16x4 hi)
+{
+    return __builtin_bit_cast(mfma_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
 
-    // padded output channels stay zero in the dy tile
-    for (int i = threadIdx.x; i < (COP - CO) * (kWgDS / 4); i += kBlock)
-        reinterpret_cast<unsigned*>(dys + CO * kWgDS)[i] = 0u;
+constexpr int kWgTile = kTX * kTY * kTZ;  // voxels of a tile
+constexpr int kWgKB = kWgTile / 32;       // k blocks of a tile
 
-    // the lane's row in each of its row blocks: kind 0 = weight row (A from the
-    // shifted halo), 1 = the ones row, 2 = padding; byte offset of its A rows
-    int kind[RBW], aoff[RBW], grow[RBW];
+__host__ __device__ constexpr int wg_groups(int ci) { return ci >= 16 ? ci / 16 : 1; }
+__host__ __device__ constexpr int wg_rows(int ci) { return 27 * ci + 1; }
+// columns of a partial
+__host__ __device__ constexpr int wg_cols(int co) { return co == 1 ? 1 : 16 * c_blocks(co); }
+// bytes per voxel of the dy tile: 32 bytes of padding from 32 channels on, so
+// that the four voxels of a lane group fall on different banks
+__host__ __device__ constexpr int wg_dy_stride(int co) { return 2 * co + (co > 16 ? 32 : 0); }
+
+// Workgroups (= partials) per channel group.  First and last layer: as many as
+// fit the chip (their partials are a few KB); the others one or two per compute
+// unit (their partials are up to 0.4 MB each).
+__host__ __device__ constexpr int wg_max_slots(int ci, int co)
+{
+    return (ci < 16 || co == 1) ? 2048 : (ci == 16 ? 512 : 256);
+}
+
+struct WgTiles {
+    int tiles_x, tiles_xy, ntiles;
+    __device__ __forceinline__ explicit WgTiles(int m)
+    {
+        tiles_x = (m + kTX - 1) / kTX;
+        tiles_xy = tiles_x * tiles_x;
+        ntiles = tiles_xy * (m / kTZ);
+    }
+    __device__ __forceinline__ void origin(int t, int& X0, int& Y0, int& Z0) const
+    {
+        X0 = (t % tiles_x) * kTX;
+        Y0 = ((t / tiles_x) % tiles_x) * kTY;
+        Z0 = (t / tiles_xy) * kTZ;
+    }
+};
+
+// A tile of [m^3][C] BF16 voxels (C = channels taken: 8 per item), between its
+// global loads and its LDS stores.  HALO: with the one-voxel halo.  Voxels
+// outside the grid load an in-range one and store zeros.
+template <int C, bool HALO, int IN> struct WgStage {
+    static constexpr int SX = HALO ? kHX : kTX, SY = HALO ? kHY : kTY, SZ = HALO ? kHZ : kTZ;
+    static constexpr int QPV = C / 8;
+    static constexpr int TOTAL = SX * SY * SZ * QPV;
+    static constexpr int ITERS = (TOTAL + kBlock - 1) / kBlock;
+    bf16x8 v[ITERS];
+    bf16x8 cv[IN == kInUpAdd ? ITERS : 1];
+    unsigned in;  // bit u: item u is inside the grid
+
+    // `stride` channels per voxel in memory, of which C from channel c0 on
+    __device__ __forceinline__ void load(int m, int X0, int Y0, int Z0, const unsigned short* __restrict__ x,
+                                         const unsigned short* __restrict__ coarse, int stride, int c0)
+    {
+        const int mh = m / 2;
+        in = 0;
 #pragma unroll
-    for (int j = 0; j < RBW; ++j) {
-        const int rb = wave + 4 * j;
-        int g = -1, k = 2;
-        if (rb < NRB) {
-            if constexpr (CI >= 16) {
-                if (rb < 27) {
-                    g = rb * CI + 16 * cg + ln;
-                    k = 0;
-                } else if (cg == 0 && ln == 0) {
-                    g = 27 * CI;
-                    k = 1;
-                }
-            } else {
-                const int gg = 16 * rb + ln;
-                if (gg < 27 * CI) {
-                    g = gg;
-                    k = 0;
-                } else if (gg == 27 * CI) {
-                    g = gg;
-                    k = 1;
+        for (int u = 0; u < ITERS; ++u) {
+            const int c = min(u * kBlock + (int)threadIdx.x, TOTAL - 1);
+            const int hv = c / QPV, od = c % QPV;
+            const int gx = X0 - (HALO ? 1 : 0) + hv % SX;
+            const int gy = Y0 - (HALO ? 1 : 0) + (hv / SX) % SY;
+            const int gz = Z0 - (HALO ? 1 : 0) + hv / (SX * SY);
+            if (gx >= 0 && gx < m && gy >= 0 && gy < m && gz >= 0 && gz < m)
+                in |= 1u << u;
+            const int cx = min(max(gx, 0), m - 1), cy = min(max(gy, 0), m - 1), cz = min(max(gz, 0), m - 1);
+            v[u] = load8(x + ((size_t)(cz * m + cy) * m + cx) * stride + c0 + 8 * od);
+            if constexpr (IN == kInUpAdd)
+                cv[u] = load8(coarse + ((size_t)((cz >> 1) * mh + (cy >> 1)) * mh + (cx >> 1)) * stride + c0 + 8 * od);
+        }
+    }
+
+    template <int STRIDE> __device__ __forceinline__ void store(unsigned char* lds) const
+    {
+#pragma unroll
+        for (int u = 0; u < ITERS; ++u) {
+            const int c = u * kBlock + threadIdx.x;
+            if (c < TOTAL) {
+                bf16x8 w = v[u];
+                if constexpr (IN == kInUpAdd)
+                    w = add8(w, cv[u]);
+                *reinterpret_cast<bf16x8*>(lds + (c / QPV) * STRIDE + 16 * (c % QPV)) = (in >> u) & 1u ? w : zero8();
+            }
+        }
+    }
+};
+
+// Halo words of a field with one 2- or 4-byte word per voxel, stored as three
+// copies of each of its NC 2-byte channels: copy s holds halo x = s .. s + 7 of
+// every halo row, [s][channel][hz * 10 + hy][8], so that the four voxels of a
+// lane's operand are an aligned 8-byte read whatever the tap's shift in x.
+template <int NC> struct WgPlanes {
+    static constexpr int kBytes = 3 * NC * kHY * kHZ * 16;
+    static constexpr int ITERS = (kHalo + kBlock - 1) / kBlock;
+    unsigned v[ITERS];
+
+    __device__ __forceinline__ void load(int m, int X0, int Y0, int Z0, const unsigned short* __restrict__ x)
+    {
+#pragma unroll
+        for (int u = 0; u < ITERS; ++u) {
+            const int hv = min(u * kBlock + (int)threadIdx.x, kHalo - 1);
+            const int gx = X0 - 1 + hv % kHX, gy = Y0 - 1 + (hv / kHX) % kHY, gz = Z0 - 1 + hv / (kHX * kHY);
+            const bool in = gx >= 0 && gx < m && gy >= 0 && gy < m && gz >= 0 && gz < m;
+            const int cx = min(max(gx, 0), m - 1), cy = min(max(gy, 0), m - 1), cz = min(max(gz, 0), m - 1);
+            const size_t g = (size_t)(cz * m + cy) * m + cx;
+            const unsigned w = NC == 2 ? reinterpret_cast<const unsigned*>(x)[g] : (unsigned)x[g];
+            v[u] = in ? w : 0u;
+        }
+    }
+
+    __device__ __forceinline__ void store(unsigned char* lds) const
+    {
+#pragma unroll
+        for (int u = 0; u < ITERS; ++u) {
+            const int hv = u * kBlock + threadIdx.x;
+            if (hv < kHalo) {
+                const int hx = hv % kHX, row = hv / kHX;  // row = hz * 10 + hy
+#pragma unroll
+                for (int s = 0; s < 3; ++s) {
+                    const int xl = hx - s;
+                    if (xl >= 0 && xl < 8) {
+#pragma unroll
+                        for (int c = 0; c < NC; ++c)
+                            *reinterpret_cast<unsigned short*>(lds + ((s * NC + c) * kHY * kHZ + row) * 16 + 2 * xl) =
+                                (unsigned short)(v[u] >> (16 * c));
+                    }
                 }
             }
         }
-        kind[j] = k;
-        grow[j] = g;
-        aoff[j] = 0;
-        if (k == 0) {
-            const int t = g / CI, c = (g % CI) - (CI >= 16 ? 16 * cg : 0);
-            const int dz = t / 9, dyy = (t / 3) % 3, s = t % 3;  // halo offsets (d + 1)
-            aoff[j] = (s * CH + c) * kWgXS + (dz * 10 + dyy) * 16;
-        }
+    }
+};
+
+// Halo row of x row R = 4 kb + 2 half (+ q / 2) of the tile, z * 10 + y.
+__host__ __device__ constexpr int wg_halo_row(int kb, int half) { return (kb / 2) * kHY + (4 * kb + 2 * half) % 8; }
+
+// CI >= 16, CO >= 16: rows g = tap * CI + ci in blocks of one tap and the 16
+// channels of this workgroup's group, plus a block of ones (db) in group 0; the
+// four waves take every fourth row block.
+template <int CI, int CO, int IN>
+__global__ __launch_bounds__(kBlock) void conv3_wgrad_mfma_kernel(int m, const unsigned short* __restrict__ x,
+                                                                  const unsigned short* __restrict__ coarse,
+                                                                  const unsigned short* __restrict__ dy, int nslots,
+                                                                  float* __restrict__ partial)
+{
+    constexpr int NRB = 28;
+    constexpr int RBW = NRB / 4;  // row blocks per wave
+    constexpr int CBN = c_blocks(CO);
+    constexpr int COP = wg_cols(CO);
+    constexpr int ROWS = wg_rows(CI);
+    constexpr int DS = wg_dy_stride(CO);
+    constexpr int kDyOff = kHalo * 32;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kDyOff + kWgTile * DS];
+    unsigned char* xs = smem;
+    unsigned char* dys = smem + kDyOff;
+
+    const int cg = (int)blockIdx.x / nslots;  // channel group: input channels 16 cg ..
+    const int slot = (int)blockIdx.x % nslots;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int ln = lane % 16, kq = lane / 16;
+    const WgTiles tiles(m);
+
+    // the lane's byte offset within a read of four voxels x 16 channels
+    const int abase = ((kq / 2) * kHX + 4 * (kq % 2) + ln / 4) * 32 + (ln % 4) * 8;
+    const int bbase = (4 * kq + ln / 4) * DS + (ln % 4) * 8;
+    int aoff[RBW];
+#pragma unroll
+    for (int j = 0; j < RBW; ++j) {
+        const int t = min(wave + 4 * j, 26);
+        aoff[j] = abase + (((t / 9) * kHY + (t / 3) % 3) * kHX + t % 3) * 32;
     }
     f32x4 acc[RBW][CBN];
 #pragma unroll
@@ -880,109 +990,42 @@ __global__ __launch_bounds__(kBlock) void conv3_wgrad_mfma_kernel(int m, const u
 #pragma unroll
         for (int cb = 0; cb < CBN; ++cb)
             acc[j][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bf16x8 ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    const bf16x8 ones8 = {0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    const mfma_bf16x8 ones = __builtin_bit_cast(mfma_bf16x8, ones8);
 
-    for (TileWalk walk(ntiles, slot, nslots); walk.t < walk.end; walk.t += walk.step) {
-        const int t2 = walk.t;
-        const int X0 = (t2 % tiles_x) * kTX;
-        const int Y0 = ((t2 / tiles_x) % tiles_x) * kTY;
-        const int Z0 = (t2 / tiles_xy) * kTZ;
+    TileWalk walk(tiles.ntiles, slot, nslots);
+    WgStage<16, true, IN> sx;
+    WgStage<CO, false, kInPlain> sd;
+    if (walk.t < walk.end) {
+        int X0, Y0, Z0;
+        tiles.origin(walk.t, X0, Y0, Z0);
+        sx.load(m, X0, Y0, Z0, x, coarse, CI, 16 * cg);
+        sd.load(m, X0, Y0, Z0, dy, nullptr, CO, 0);
+    }
+    for (; walk.t < walk.end; walk.t += walk.step) {
         __syncthreads();  // the previous tile's reads are done
-        // shifted halo copies of the group's CH input channels
-        if constexpr (CI >= 16) {
-            constexpr int ITEMS = kHalo * 2;  // (voxel, channel octet)
-            for (int it = threadIdx.x; it < ITEMS; it += kBlock) {
-                const int hv = it >> 1, od = it & 1;
-                const int hx = hv % kHX, hy = (hv / kHX) % kHY, hz = hv / (kHX * kHY);
-                const int gx = X0 - 1 + hx, gy = Y0 - 1 + hy, gz = Z0 - 1 + hz;
-                bf16x8 v = zero8();
-                if (gx >= 0 && gx < m && gy >= 0 && gy < m && gz >= 0 && gz < m) {
-                    const size_t g = (size_t)(gz * m + gy) * m + gx;
-                    v = load8(x + g * CI + 16 * cg + 8 * od);
-                    if constexpr (IN == kInUpAdd)
-                        v = add8(v, load8(coarse + ((size_t)((gz >> 1) * mh + (gy >> 1)) * mh + (gx >> 1)) * CI +
-                                          16 * cg + 8 * od));
-                }
-#pragma unroll
-                for (int sft = 0; sft < 3; ++sft) {
-                    const int xl = hx - sft;
-                    if (xl >= 0 && xl < 8) {
-#pragma unroll
-                        for (int c = 0; c < 8; ++c)
-                            *reinterpret_cast<unsigned short*>(xs + (sft * CH + 8 * od + c) * kWgXS +
-                                                               (hz * 10 + hy) * 16 + 2 * xl) = (unsigned short)v[c];
-                    }
-                }
-            }
-        } else {
-            for (int hv = threadIdx.x; hv < kHalo; hv += kBlock) {
-                const int hx = hv % kHX, hy = (hv / kHX) % kHY, hz = hv / (kHX * kHY);
-                const int gx = X0 - 1 + hx, gy = Y0 - 1 + hy, gz = Z0 - 1 + hz;
-                unsigned u = 0u;
-                if (gx >= 0 && gx < m && gy >= 0 && gy < m && gz >= 0 && gz < m) {
-                    const size_t g = (size_t)(gz * m + gy) * m + gx;
-                    u = CI == 2 ? reinterpret_cast<const unsigned*>(x)[g] : (unsigned)x[g];
-                }
-#pragma unroll
-                for (int sft = 0; sft < 3; ++sft) {
-                    const int xl = hx - sft;
-                    if (xl >= 0 && xl < 8) {
-#pragma unroll
-                        for (int c = 0; c < CI; ++c)
-                            *reinterpret_cast<unsigned short*>(xs + (sft * CH + c) * kWgXS + (hz * 10 + hy) * 16 +
-                                                               2 * xl) = (unsigned short)(u >> (16 * c));
-                    }
-                }
-            }
-        }
-        // dy tile, channel-major BF16: dys[co][z * 8 + y][x]
-        {
-            constexpr int QPV = CO >= 4 ? CO / 4 : 1;  // 4-channel quads per voxel
-            constexpr int ITEMS = kTX * kTY * kTZ * QPV;
-            for (int it = threadIdx.x; it < ITEMS; it += kBlock) {
-                const int vl = it / QPV, qd = it % QPV;
-                const int lx = vl % 8, ly = (vl / 8) % 8, lz = vl / 64;
-                const int gx = X0 + lx, gy = Y0 + ly, gz = Z0 + lz;
-                const bool in = gx < m && gy < m;
-                const size_t g = in ? (size_t)(gz * m + gy) * m + gx : 0;
-                unsigned char* row = dys + (lz * 8 + ly) * 16 + 2 * lx;
-                if constexpr (CO >= 4) {
-                    const float4 d = in ? *reinterpret_cast<const float4*>(dy + g * CO + 4 * qd)
-                                        : float4{0.f, 0.f, 0.f, 0.f};
-                    const unsigned p0 = pack_bf16x2(d.x, d.y), p1 = pack_bf16x2(d.z, d.w);
-                    *reinterpret_cast<unsigned short*>(row + (4 * qd + 0) * kWgDS) = (unsigned short)p0;
-                    *reinterpret_cast<unsigned short*>(row + (4 * qd + 1) * kWgDS) = (unsigned short)(p0 >> 16);
-                    *reinterpret_cast<unsigned short*>(row + (4 * qd + 2) * kWgDS) = (unsigned short)p1;
-                    *reinterpret_cast<unsigned short*>(row + (4 * qd + 3) * kWgDS) = (unsigned short)(p1 >> 16);
-                } else {
-#pragma unroll
-                    for (int c = 0; c < CO; ++c) {
-                        const float d = in ? dy[g * CO + c] : 0.0f;
-                        *reinterpret_cast<unsigned short*>(row + c * kWgDS) = (unsigned short)pack_bf16x2(d, 0.0f);
-                    }
-                }
-            }
-        }
+        sx.template store<32>(xs);
+        sd.template store<DS>(dys);
         __syncthreads();
+        if (walk.t + walk.step < walk.end) {  // the next tile, in flight during the MFMAs
+            int X0, Y0, Z0;
+            tiles.origin(walk.t + walk.step, X0, Y0, Z0);
+            sx.load(m, X0, Y0, Z0, x, coarse, CI, 16 * cg);
+            sd.load(m, X0, Y0, Z0, dy, nullptr, CO, 0);
+        }
 #pragma unroll
-        for (int kb = 0; kb < 8; ++kb) {
-            const int R = 4 * kb + kq;  // x row of the tile: y = R % 8, z = R / 8
-            const int rofs = ((R / 8) * 10 + (R % 8)) * 16;
+        for (int kb = 0; kb < kWgKB; ++kb) {
             mfma_bf16x8 b[CBN];
 #pragma unroll
             for (int cb = 0; cb < CBN; ++cb)
-                b[cb] = __builtin_bit_cast(mfma_bf16x8,
-                                           *reinterpret_cast<const bf16x8*>(dys + (16 * cb + ln) * kWgDS + R * 16));
+                b[cb] = join8(lds_read_tr(dys + bbase + (32 * kb) * DS + 32 * cb),
+                              lds_read_tr(dys + bbase + (32 * kb + 16) * DS + 32 * cb));
 #pragma unroll
             for (int j = 0; j < RBW; ++j) {
-                if (wave + 4 * j >= NRB)
-                    continue;  // wave-uniform
-                bf16x8 av = zero8();
-                if (kind[j] == 0)
-                    av = *reinterpret_cast<const bf16x8*>(xs + aoff[j] + rofs);
-                else if (kind[j] == 1)
-                    av = ones;
-                const mfma_bf16x8 a = __builtin_bit_cast(mfma_bf16x8, av);
+                mfma_bf16x8 a = join8(lds_read_tr(xs + aoff[j] + wg_halo_row(kb, 0) * kHX * 32),
+                                      lds_read_tr(xs + aoff[j] + wg_halo_row(kb, 1) * kHX * 32));
+                if (j == RBW - 1 && wave == 3)  // row block 27
+                    a = ones;
 #pragma unroll
                 for (int cb = 0; cb < CBN; ++cb)
                     acc[j][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[cb], acc[j][cb], 0, 0, 0);
@@ -993,21 +1036,10 @@ __global__ __launch_bounds__(kBlock) void conv3_wgrad_mfma_kernel(int m, const u
 #pragma unroll
     for (int j = 0; j < RBW; ++j) {
         const int rb = wave + 4 * j;
-        if (rb >= NRB)
-            continue;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            // the row held in C row 4 kq + i of this block (same mapping as the A rows)
             const int r = 4 * kq + i;
-            int g = -1;
-            if constexpr (CI >= 16) {
-                if (rb < 27)
-                    g = rb * CI + 16 * cg + r;
-                else if (cg == 0 && r == 0)
-                    g = 27 * CI;
-            } else {
-                g = 16 * rb + r < ROWS ? 16 * rb + r : -1;
-            }
+            const int g = rb < 27 ? rb * CI + 16 * cg + r : (cg == 0 && r == 0 ? 27 * CI : -1);
             if (g >= 0) {
 #pragma unroll
                 for (int cb = 0; cb < CBN; ++cb)
@@ -1017,42 +1049,253 @@ __global__ __launch_bounds__(kBlock) void conv3_wgrad_mfma_kernel(int m, const u
     }
 }
 
-// dW[row * CO + co] (rows < 27 * CI) and db[co] (row 27 * CI) = sum over the slots in order
-__global__ __launch_bounds__(kBlock) void wgrad_sum_kernel(int rows, int co, int cop, int nslots,
+// First layer (2 input channels, 16 output channels): the 54 rows (tap, ci)
+// and the row of ones in order, one block of 16 per wave; their operands from
+// the shifted planes of x, dy transposed on the read as above.
+template <int CO>
+__global__ __launch_bounds__(kBlock) void conv3_wgrad_ci2_kernel(int m, const unsigned short* __restrict__ x,
+                                                                const unsigned short* __restrict__ dy, int nslots,
+                                                                float* __restrict__ partial)
+{
+    static_assert(CO == 16, "one block of output channels");
+    constexpr int ROWS = wg_rows(2);
+    constexpr int DS = wg_dy_stride(CO);
+    constexpr int kDyOff = WgPlanes<2>::kBytes;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kDyOff + kWgTile * DS];
+    unsigned char* xs = smem;
+    unsigned char* dys = smem + kDyOff;
+    const int slot = (int)blockIdx.x;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int ln = lane % 16, kq = lane / 16;
+    const WgTiles tiles(m);
+    const int g = 16 * wave + ln;  // this lane's row
+    const int tap = min(g / 2, 26);
+    const int aoff = ((((tap % 3) * 2 + g % 2) * kHZ + tap / 9) * kHY + (tap / 3) % 3 + kq / 2) * 16 + (kq % 2) * 8;
+    const int bbase = (4 * kq + ln / 4) * DS + (ln % 4) * 8;
+    const short fill = g == 54 ? (short)0x3f80 : (short)0;  // the row of ones; zeros below it
+    const bf16x4 constant = {fill, fill, fill, fill};
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+
+    TileWalk walk(tiles.ntiles, slot, nslots);
+    WgPlanes<2> sx;
+    WgStage<CO, false, kInPlain> sd;
+    if (walk.t < walk.end) {
+        int X0, Y0, Z0;
+        tiles.origin(walk.t, X0, Y0, Z0);
+        sx.load(m, X0, Y0, Z0, x);
+        sd.load(m, X0, Y0, Z0, dy, nullptr, CO, 0);
+    }
+    for (; walk.t < walk.end; walk.t += walk.step) {
+        __syncthreads();
+        sx.store(xs);
+        sd.template store<DS>(dys);
+        __syncthreads();
+        if (walk.t + walk.step < walk.end) {
+            int X0, Y0, Z0;
+            tiles.origin(walk.t + walk.step, X0, Y0, Z0);
+            sx.load(m, X0, Y0, Z0, x);
+            sd.load(m, X0, Y0, Z0, dy, nullptr, CO, 0);
+        }
+#pragma unroll
+        for (int kb = 0; kb < kWgKB; ++kb) {
+            const mfma_bf16x8 b =
+                join8(lds_read_tr(dys + bbase + (32 * kb) * DS), lds_read_tr(dys + bbase + (32 * kb + 16) * DS));
+            bf16x4 lo = *reinterpret_cast<const bf16x4*>(xs + aoff + wg_halo_row(kb, 0) * 16);
+            bf16x4 hi = *reinterpret_cast<const bf16x4*>(xs + aoff + wg_halo_row(kb, 1) * 16);
+            if (g >= 54)
+                lo = hi = constant;
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(join8(lo, hi), b, acc, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 16 * wave + 4 * kq + i;
+        if (r < ROWS)
+            partial[((size_t)slot * ROWS + r) * CO + ln] = acc[i];
+    }
+}
+
+// Last layer (16 input channels, one output channel): with
+// dW[t][ci] = sum_u x~[u][ci] dy[u - d_t] the rows are the 16 channels, the
+// columns the 27 taps (two blocks) and x needs no halo; dy's shifts come from
+// its planes.  db is the centre tap's column under rows of ones.  The waves
+// split the tile's k blocks and are added in LDS.
+template <int IN>
+__global__ __launch_bounds__(kBlock) void conv3_wgrad_co1_kernel(int m, const unsigned short* __restrict__ x,
+                                                                const unsigned short* __restrict__ coarse,
+                                                                const unsigned short* __restrict__ dy, int nslots,
+                                                                float* __restrict__ partial)
+{
+    constexpr int CI = 16;
+    constexpr int ROWS = wg_rows(CI);
+    constexpr int kDyOff = kWgTile * 32;
+    constexpr int kRed = 4 * 3 * kWave * 16;  // the waves' accumulators, over the tiles
+    constexpr int kTiles = kDyOff + WgPlanes<1>::kBytes;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kTiles > kRed ? kTiles : kRed];
+    unsigned char* xs = smem;
+    unsigned char* dys = smem + kDyOff;
+    const int slot = (int)blockIdx.x;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int ln = lane % 16, kq = lane / 16;
+    const WgTiles tiles(m);
+    const int abase = (4 * kq + ln / 4) * 32 + (ln % 4) * 8;
+    int boff[2];
+#pragma unroll
+    for (int nb = 0; nb < 2; ++nb) {
+        const int t = min(16 * nb + ln, 26);
+        boff[nb] = (((2 - t % 3) * kHZ + 2 - t / 9) * kHY + 2 - (t / 3) % 3 + kq / 2) * 16 + (kq % 2) * 8;
+    }
+    const bf16x4 zero4 = {0, 0, 0, 0};
+    const bf16x8 ones8 = {0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    const mfma_bf16x8 ones = __builtin_bit_cast(mfma_bf16x8, ones8);
+    f32x4 acc[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+        acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    TileWalk walk(tiles.ntiles, slot, nslots);
+    WgStage<CI, false, IN> sx;
+    WgPlanes<1> sd;
+    if (walk.t < walk.end) {
+        int X0, Y0, Z0;
+        tiles.origin(walk.t, X0, Y0, Z0);
+        sx.load(m, X0, Y0, Z0, x, coarse, CI, 0);
+        sd.load(m, X0, Y0, Z0, dy);
+    }
+    for (; walk.t < walk.end; walk.t += walk.step) {
+        __syncthreads();
+        sx.template store<32>(xs);
+        sd.store(dys);
+        __syncthreads();
+        if (walk.t + walk.step < walk.end) {
+            int X0, Y0, Z0;
+            tiles.origin(walk.t + walk.step, X0, Y0, Z0);
+            sx.load(m, X0, Y0, Z0, x, coarse, CI, 0);
+            sd.load(m, X0, Y0, Z0, dy);
+        }
+#pragma unroll
+        for (int kk = 0; kk < kWgKB / 4; ++kk) {
+            const int kb = wave * (kWgKB / 4) + kk;  // both k blocks of a wave lie in the slice z = wave
+            const mfma_bf16x8 a =
+                join8(lds_read_tr(xs + abase + (32 * kb) * 32), lds_read_tr(xs + abase + (32 * kb + 16) * 32));
+            const unsigned char* drow = dys + (wave * kHY + 4 * kk) * 16;
+            mfma_bf16x8 b[2];
+#pragma unroll
+            for (int nb = 0; nb < 2; ++nb) {
+                bf16x4 lo = *reinterpret_cast<const bf16x4*>(drow + boff[nb]);
+                bf16x4 hi = *reinterpret_cast<const bf16x4*>(drow + boff[nb] + 32);
+                if (16 * nb + ln >= 27)
+                    lo = hi = zero4;
+                b[nb] = join8(lo, hi);
+            }
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[0], acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[1], acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, b[0], acc[2], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+    f32x4* red = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+        red[(j * 4 + wave) * kWave + lane] = acc[j];
+    __syncthreads();
+    if (wave < 3) {  // wave j adds accumulator j of the four waves
+        f32x4 s = red[(wave * 4) * kWave + lane];
+#pragma unroll
+        for (int w = 1; w < 4; ++w)
+            s += red[(wave * 4 + w) * kWave + lane];
+        float* out = partial + (size_t)slot * ROWS;
+        if (wave < 2) {
+            const int t = 16 * wave + ln;
+            if (t < 27) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    out[t * CI + 4 * kq + i] = s[i];
+            }
+        } else if (ln == 13 && kq == 0) {
+            out[27 * CI] = s[0];
+        }
+    }
+}
+
+// dW[row * CO + co] (rows < 27 * CI) and db[co] (row 27 * CI): 16 consecutive
+// outputs per workgroup, SL threads each, thread s adding the partials s,
+// s + SL, ... in order and a tree the SL sums.  (One thread per output summed
+// its 256 partials one load after another: 5-100 us a layer, now 3-17.)
+template <int SL>
+__global__ __launch_bounds__(16 * SL) void wgrad_sum_kernel(int rows, int co, int cop, int nslots,
                                                            const float* __restrict__ partial, float* __restrict__ dW,
                                                            float* __restrict__ db)
 {
-    const int idx = blockIdx.x * kBlock + threadIdx.x;
-    if (idx >= rows * co)
-        return;
-    const int g = idx / co, c = idx % co;
+    __shared__ float red[SL][17];
+    const int col = threadIdx.x % 16, sl = threadIdx.x / 16;
+    const int idx = (int)blockIdx.x * 16 + col;
+    const bool on = idx < rows * co;
+    const int g = on ? idx / co : 0, c = on ? idx % co : 0;
+    const float* p = partial + (size_t)g * cop + c;
+    const size_t step = (size_t)rows * cop;
     float s = 0.0f;
-    for (int k = 0; k < nslots; ++k)
-        s += partial[((size_t)k * rows + g) * cop + c];
-    if (g < rows - 1)
-        dW[(size_t)g * co + c] = s;
-    else
-        db[c] = s;
+    int k = sl;
+    for (; k + 7 * SL < nslots; k += 8 * SL) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            v[u] = p[(size_t)(k + u * SL) * step];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            s += v[u];
+    }
+    for (; k < nslots; k += SL)
+        s += p[(size_t)k * step];
+    red[sl][col] = s;
+    __syncthreads();
+#pragma unroll
+    for (int w = SL / 2; w > 0; w >>= 1) {
+        if (sl < w)
+            red[sl][col] += red[sl + w][col];
+        __syncthreads();
+    }
+    if (sl == 0 && on) {
+        if (g < rows - 1)
+            dW[(size_t)g * co + c] = red[0][col];
+        else
+            db[c] = red[0][col];
+    }
+}
+
+inline int wgrad_slots(int m, int ci, int co)
+{
+    const int txy = (m + kTX - 1) / kTX;
+    const int64_t tiles = (int64_t)txy * txy * (m / kTZ);
+    return (int)std::min<int64_t>(tiles, wg_max_slots(ci, co));
 }
 
 template <int CI, int CO>
-int launch_wgrad(int m, int in_mode, const unsigned short* x, const unsigned short* coarse, const float* dy,
+int launch_wgrad(int m, int in_mode, const unsigned short* x, const unsigned short* coarse, const unsigned short* dy,
                  float* dW, float* db, float* partial, hipStream_t s)
 {
-    const int txy = (m + kTX - 1) / kTX;
-    const int tiles = txy * txy * (m / kTZ);
-    const int nslots = tiles < kWgMaxSlots ? tiles : kWgMaxSlots;
-    const unsigned grid = (unsigned)(nslots * wg_groups(CI));
-    if (in_mode == kInUpAdd) {
-        if constexpr (CI >= 16)
-            conv3_wgrad_mfma_kernel<CI, CO, kInUpAdd><<<grid, kBlock, 0, s>>>(m, x, coarse, dy, nslots, partial);
+    const int nslots = wgrad_slots(m, CI, CO);
+    if constexpr (CO == 1) {
+        if (in_mode == kInUpAdd)
+            conv3_wgrad_co1_kernel<kInUpAdd><<<nslots, kBlock, 0, s>>>(m, x, coarse, dy, nslots, partial);
+        else
+            conv3_wgrad_co1_kernel<kInPlain><<<nslots, kBlock, 0, s>>>(m, x, coarse, dy, nslots, partial);
+    } else if constexpr (CI == 2) {
+        conv3_wgrad_ci2_kernel<CO><<<nslots, kBlock, 0, s>>>(m, x, dy, nslots, partial);
     } else {
-        conv3_wgrad_mfma_kernel<CI, CO, kInPlain><<<grid, kBlock, 0, s>>>(m, x, coarse, dy, nslots, partial);
+        const unsigned grid = (unsigned)(nslots * wg_groups(CI));
+        if (in_mode == kInUpAdd)
+            conv3_wgrad_mfma_kernel<CI, CO, kInUpAdd><<<grid, kBlock, 0, s>>>(m, x, coarse, dy, nslots, partial);
+        else
+            conv3_wgrad_mfma_kernel<CI, CO, kInPlain><<<grid, kBlock, 0, s>>>(m, x, coarse, dy, nslots, partial);
     }
     WA_LAUNCH_CHECK();
     const int rows = wg_rows(CI);
-    wgrad_sum_kernel<<<(unsigned)ceil_div(rows * CO, kBlock), kBlock, 0, s>>>(rows, CO, 16 * c_blocks(CO), nslots,
-                                                                           partial, dW, db);
+    const unsigned sums = (unsigned)ceil_div(rows * CO, 16);
+    if (nslots >= 128)
+        wgrad_sum_kernel<64><<<sums, 1024, 0, s>>>(rows, CO, wg_cols(CO), nslots, partial, dW, db);
+    else
+        wgrad_sum_kernel<16><<<sums, 256, 0, s>>>(rows, CO, wg_cols(CO), nslots, partial, dW, db);
     WA_LAUNCH_CHECK();
     return kOk;
 }
@@ -1202,40 +1445,46 @@ bool wgrad_pair_supported(int ci, int co)
 }
 }  // namespace
 
-// Bytes of workspace of warp_amd_conv3_mfma_wgrad on an m^3 grid.
+// Bytes of workspace of warp_amd_conv3_mfma_wgrad_bf16 on an m^3 grid: the workgroups' partials.
+WA_API size_t warp_amd_conv3_mfma_wgrad_bf16_workspace_size(int m, int cin, int cout)
+{
+    if (m <= 0)
+        return 0;
+    return sizeof(float) * (size_t)wa::wgrad_slots(m, cin, cout) * wa::wg_rows(cin) * wa::wg_cols(cout);
+}
+
+// The same of warp_amd_conv3_mfma_wgrad: the partials and dy in BF16.
 WA_API size_t warp_amd_conv3_mfma_wgrad_workspace_size(int m, int cin, int cout)
 {
     if (m <= 0)
         return 0;
-    const int64_t txy = wa::ceil_div(m, wa::kTX);
-    const int64_t tiles = txy * txy * (m / wa::kTZ);
-    const int64_t slots = tiles < wa::kWgMaxSlots ? tiles : wa::kWgMaxSlots;
-    return sizeof(float) * (size_t)slots * wa::wg_rows(cin) * 16 * wa::c_blocks(cout);
+    return warp_amd_conv3_mfma_wgrad_bf16_workspace_size(m, cin, cout) + 16 + sizeof(short) * (size_t)m * m * m * cout;
 }
 
 // Weight and bias gradients of a BF16 (cin -> cout) 3x3x3 convolution on an
 // m^3 grid (m a multiple of 4): dW[27][cin][cout] = sum_v x~[v + d_t][ci]
 // dy[v][co], db[cout] = sum_v dy[v][co], both overwritten.  x: BF16 layer
 // input [m^3][cin] (in_mode 1: x + upsample(coarse), as the forward formed
-// it); dy: FP32 [m^3][cout], rounded to BF16; FP32 accumulation, partial
-// sums per workgroup added in a fixed order (deterministic).
-WA_API int warp_amd_conv3_mfma_wgrad(int m, int cin, int cout, int in_mode, const void* x, const void* coarse,
-                                     const float* dy, float* dW, float* db, void* workspace, size_t workspace_bytes,
-                                     void* stream)
+// it); dy: BF16 [m^3][cout]; FP32 accumulation, partial sums per workgroup
+// added in a fixed order (deterministic).  x, coarse and dy 16-byte aligned.
+WA_API int warp_amd_conv3_mfma_wgrad_bf16(int m, int cin, int cout, int in_mode, const void* x, const void* coarse,
+                                          const void* dy, float* dW, float* db, void* workspace,
+                                          size_t workspace_bytes, void* stream)
 {
     WA_REQUIRE(wgrad_pair_supported(cin, cout), "conv3_mfma_wgrad: unsupported channel pair %d -> %d", cin, cout);
     WA_REQUIRE(m >= 4 && m % 4 == 0, "conv3_mfma_wgrad: grid side %d must be a positive multiple of 4", m);
     WA_REQUIRE(in_mode == 0 || (in_mode == 1 && cin >= 16 && coarse), "conv3_mfma_wgrad: bad input mode");
     WA_REQUIRE(x && dy && dW && db, "conv3_mfma_wgrad: null array");
-    WA_REQUIRE(workspace && workspace_bytes >= warp_amd_conv3_mfma_wgrad_workspace_size(m, cin, cout),
+    WA_REQUIRE(workspace && workspace_bytes >= warp_amd_conv3_mfma_wgrad_bf16_workspace_size(m, cin, cout),
                "conv3_mfma_wgrad: workspace too small");
     const unsigned short* xi = static_cast<const unsigned short*>(x);
     const unsigned short* ci = static_cast<const unsigned short*>(coarse);
+    const unsigned short* di = static_cast<const unsigned short*>(dy);
     float* pw = static_cast<float*>(workspace);
     hipStream_t s = wa::as_stream(stream);
 #define WA_WGRAD_CASE(A, B)                                                                                      \
     if (cin == A && cout == B)                                                                                   \
-        return wa::launch_wgrad<A, B>(m, in_mode, xi, ci, dy, dW, db, pw, s);
+        return wa::launch_wgrad<A, B>(m, in_mode, xi, ci, di, dW, db, pw, s);
     WA_WGRAD_CASE(2, 16)
     WA_WGRAD_CASE(16, 32)
     WA_WGRAD_CASE(32, 64)
@@ -1245,6 +1494,22 @@ WA_API int warp_amd_conv3_mfma_wgrad(int m, int cin, int cout, int in_mode, cons
     WA_WGRAD_CASE(16, 1)
 #undef WA_WGRAD_CASE
     return wa::kErrUnsupported;
+}
+
+// The same with dy FP32 [m^3][cout], rounded to BF16 in the workspace first.
+WA_API int warp_amd_conv3_mfma_wgrad(int m, int cin, int cout, int in_mode, const void* x, const void* coarse,
+                                     const float* dy, float* dW, float* db, void* workspace, size_t workspace_bytes,
+                                     void* stream)
+{
+    WA_REQUIRE(wgrad_pair_supported(cin, cout), "conv3_mfma_wgrad: unsupported channel pair %d -> %d", cin, cout);
+    WA_REQUIRE(m >= 4 && m % 4 == 0, "conv3_mfma_wgrad: grid side %d must be a positive multiple of 4", m);
+    WA_REQUIRE(x && dy && dW && db, "conv3_mfma_wgrad: null array");
+    WA_REQUIRE(workspace && workspace_bytes >= warp_amd_conv3_mfma_wgrad_workspace_size(m, cin, cout),
+               "conv3_mfma_wgrad: workspace too small");
+    const size_t parts = warp_amd_conv3_mfma_wgrad_bf16_workspace_size(m, cin, cout);
+    void* h = reinterpret_cast<void*>(wa::align_up((uintptr_t)workspace + parts, 16));
+    WA_TRY(warp_amd_f32_to_bf16((int64_t)m * m * m * cout, dy, h, stream));
+    return warp_amd_conv3_mfma_wgrad_bf16(m, cin, cout, in_mode, x, coarse, h, dW, db, workspace, parts, stream);
 }
 
 // out = y > 0 ? dy : 0 with y BF16 (the ReLU of a BF16 forward), dy and out FP32

@@ -205,30 +205,33 @@ class UNet:
                          _native.ptr(t), s)
             self._wsw_t[name] = t
 
+    def _dy_bf16(self, name, dy):
+        """A layer's FP32 output gradient in BF16, the operand of its weight and input gradients."""
+        _, co, _, lvl = LAYER_INDEX[name]
+        h = self._hbuf("gy_" + name, lvl, co)
+        _native.call("warp_amd_f32_to_bf16", h.numel(), _native.ptr(dy), _native.ptr(h), self._s())
+        return h
+
     def _wgrad_bf16(self, name, x, dy, coarse=None):
-        """dW, db of a layer on MFMA from its BF16 input (x + upsample(coarse) for decoders) and FP32 dy."""
+        """dW, db of a layer on MFMA from its BF16 input (x + upsample(coarse) for decoders) and BF16 dy."""
         ci, co, _, lvl = LAYER_INDEX[name]
         n = self.side(lvl)
-        ws_bytes = self._lib.warp_amd_conv3_mfma_wgrad_workspace_size(n, ci, co)
+        ws_bytes = self._lib.warp_amd_conv3_mfma_wgrad_bf16_workspace_size(n, ci, co)
         t = self._buf.get("wgrad_mfma_ws")
         if t is None or t.numel() < ws_bytes:
             t = torch.empty(ws_bytes, dtype=torch.uint8, device=self.dev)
             self._buf["wgrad_mfma_ws"] = t
         _native.call(
-            "warp_amd_conv3_mfma_wgrad", n, ci, co, 1 if coarse is not None else 0, _native.ptr(x),
+            "warp_amd_conv3_mfma_wgrad_bf16", n, ci, co, 1 if coarse is not None else 0, _native.ptr(x),
             _native.ptr(coarse) if coarse is not None else None, _native.ptr(dy), _native.ptr(self.grads[name + ".W"]),
             _native.ptr(self.grads[name + ".b"]), _native.ptr(t), t.numel(), self._s(),
         )
 
     def _bwd_data_bf16(self, name, dy, dx):
-        """dx = the input gradient of a layer (FP32) from its FP32 output gradient dy, on MFMA."""
+        """dx = the input gradient of a layer (FP32) from its BF16 output gradient dy, on MFMA."""
         ci, co, _, lvl = LAYER_INDEX[name]
-        n = self.side(lvl)
-        s = self._s()
-        h = self._hbuf("gy_" + name, lvl, co)
-        _native.call("warp_amd_f32_to_bf16", h.numel(), _native.ptr(dy), _native.ptr(h), s)
-        _native.call("warp_amd_conv3_mfma", n, co, ci, 0, _native.ptr(h), None, _native.ptr(self._wsw_t[name]), None,
-                     4, None, _native.ptr(dx), None, s)
+        _native.call("warp_amd_conv3_mfma", self.side(lvl), co, ci, 0, _native.ptr(dy), None,
+                     _native.ptr(self._wsw_t[name]), None, 4, None, _native.ptr(dx), None, self._s())
 
     def _relu_bf16(self, y_bf16, dy, out):
         _native.call("warp_amd_relu_mask_bf16", dy.numel(), _native.ptr(y_bf16), _native.ptr(dy), _native.ptr(out),
@@ -254,45 +257,46 @@ class UNet:
         a3 = H("a3", 3, 64)
         b2, b1 = H("b2", 2, 32), H("b1", 1, 16)
         # d0 (linear): input a0 + up(b1)
-        self._wgrad_bf16("d0", a0, dout, coarse=b1)
+        dy = self._dy_bf16("d0", dout)
+        self._wgrad_bf16("d0", a0, dy, coarse=b1)
         da0 = B("da0", 0, 16)
-        self._bwd_data_bf16("d0", dout, da0)
+        self._bwd_data_bf16("d0", dy, da0)
         # d1: input a1 + up(b2), output b1
         g1 = B("g1", 1, 16)
         _native.call("warp_amd_up2_bwd_f32", self.side(1), 16, _native.ptr(da0), _native.ptr(g1), s)
-        dy = self._relu_bf16(b1, g1, B("m1", 1, 16))
+        dy = self._dy_bf16("d1", self._relu_bf16(b1, g1, B("m1", 1, 16)))
         self._wgrad_bf16("d1", a1, dy, coarse=b2)
         da1 = B("da1", 1, 32)
         self._bwd_data_bf16("d1", dy, da1)
         # d2: input a2 + up(a3), output b2
         g2 = B("g2", 2, 32)
         _native.call("warp_amd_up2_bwd_f32", self.side(2), 32, _native.ptr(da1), _native.ptr(g2), s)
-        dy = self._relu_bf16(b2, g2, B("m2", 2, 32))
+        dy = self._dy_bf16("d2", self._relu_bf16(b2, g2, B("m2", 2, 32)))
         self._wgrad_bf16("d2", a2, dy, coarse=a3)
         da2 = B("da2", 2, 64)
         self._bwd_data_bf16("d2", dy, da2)
         # e3: input p2, output a3
         g3 = B("g3", 3, 64)
         _native.call("warp_amd_up2_bwd_f32", self.side(3), 64, _native.ptr(da2), _native.ptr(g3), s)
-        dy = self._relu_bf16(a3, g3, B("m3", 3, 64))
+        dy = self._dy_bf16("e3", self._relu_bf16(a3, g3, B("m3", 3, 64)))
         self._wgrad_bf16("e3", p2, dy)
         dp2 = B("dp2", 3, 64)
         self._bwd_data_bf16("e3", dy, dp2)
         _native.call("warp_amd_pool2_bwd_f32", self.side(2), 64, _native.ptr(dp2), _native.ptr(da2), 1, s)
         # e2: input p1, output a2
-        dy = self._relu_bf16(a2, da2, B("m2b", 2, 64))
+        dy = self._dy_bf16("e2", self._relu_bf16(a2, da2, B("m2b", 2, 64)))
         self._wgrad_bf16("e2", p1, dy)
         dp1 = B("dp1", 2, 32)
         self._bwd_data_bf16("e2", dy, dp1)
         _native.call("warp_amd_pool2_bwd_f32", self.side(1), 32, _native.ptr(dp1), _native.ptr(da1), 1, s)
         # e1: input p0, output a1
-        dy = self._relu_bf16(a1, da1, B("m1b", 1, 32))
+        dy = self._dy_bf16("e1", self._relu_bf16(a1, da1, B("m1b", 1, 32)))
         self._wgrad_bf16("e1", p0, dy)
         dp0 = B("dp0", 1, 16)
         self._bwd_data_bf16("e1", dy, dp0)
         _native.call("warp_amd_pool2_bwd_f32", self.side(0), 16, _native.ptr(dp0), _native.ptr(da0), 1, s)
         # e0: input (BF16 network input), output a0
-        dy = self._relu_bf16(a0, da0, B("m0", 0, 16))
+        dy = self._dy_bf16("e0", self._relu_bf16(a0, da0, B("m0", 0, 16)))
         self._wgrad_bf16("e0", self._inp_bf16, dy)
 
     def _layer_grads(self, name, x, y, dy, masked):
