@@ -733,12 +733,21 @@ int warp_amd_bf16_to_f32(int64_t count, const void* in, float* out, void* stream
 /* BF16 network input [nvox][2] = (r * inv_scale, standardized log k) */
 int warp_amd_unet_pack_input_bf16(int64_t nvox, const double* r, const float* logk_std, const double* inv_scale,
                                   void* out, void* stream);
+/* Output gradient of a layer in BF16 for the training backward (no reference
+ * counterpart), zero where the layer's BF16 output y is not positive.
+ * up2: the sum of the FP32 gradient d [(2n)^3][ch] over the 8 children of
+ * each of n^3 voxels.  pool2: d [n^3][ch] + dp [(n/2)^3][ch] / 8, dp the
+ * gradient of the 2x2x2 average.  ch a multiple of 8, arrays 16-byte aligned. */
+int warp_amd_relu_up2_bwd_bf16(int n, int ch, const float* d, const void* y, void* out, void* stream);
+int warp_amd_relu_pool2_bwd_bf16(int n, int ch, const float* d, const float* dp, const void* y, void* out,
+                                 void* stream);
+
 /* Weight and bias gradients of a BF16 (cin -> cout) convolution on MFMA (no
  * reference counterpart; training of the learned preconditioner):
  * dW[27][cin][cout] = sum_v x~[v + d_t][ci] dy[v][co], db[cout] = sum_v dy[v][co],
  * both overwritten.  x: the layer's BF16 input (in_mode 1: x + upsample(coarse),
- * rounded as the forward rounds it); dy: FP32 [m^3][cout], rounded to BF16; FP32
- * accumulation; per-workgroup partials in the workspace added in a fixed order.
+ * rounded as the forward rounds it); dy: [m^3][cout], BF16 (_bf16) or FP32 and
+ * rounded to BF16 in the workspace; FP32 accumulation; per-workgroup partials in the workspace added in a fixed order.
  * Channel pairs: 2-16, 16-32, 32-64, 64-64, 64-32, 32-16, 16-1. */
 size_t warp_amd_conv3_mfma_wgrad_bf16_workspace_size(int m, int cin, int cout);
 int warp_amd_conv3_mfma_wgrad_bf16(int m, int cin, int cout, int in_mode, const void* x, const void* coarse,

@@ -332,3 +332,32 @@ def test_wgrad_bf16_many_tiles(device, ci, co, m, up):
                  _native.stream_of(device))
     assert bool(((dW.double() - want).abs() <= 2e-5 * size + 1e-30).all())
     assert bool(((db.double() - d.sum(0)).abs() <= 2e-5 * d.abs().sum(0) + 1e-30).all())
+
+
+@pytest.mark.parametrize("n,ch", [(2, 16), (6, 8), (10, 32), (4, 64)])
+def test_fused_output_gradients_vs_torch(device, n, ch):
+    """The decoder / encoder output gradients (resampling adjoint, skip sum, ReLU
+    mask, one BF16 rounding) equal torch's in the same order, zeros, negative
+    zeros and NaN of the mask included."""
+    g = torch.Generator(device=device).manual_seed(n * ch)
+
+    def rnd(*shape):
+        return torch.randn(shape, generator=g, device=device)
+
+    y = rnd(n, n, n, ch).to(torch.bfloat16)
+    y.view(-1)[:4] = torch.tensor([0.0, -0.0, float("nan"), float("inf")], dtype=torch.bfloat16, device=device)
+    s = _native.stream_of(device)
+    out = torch.empty((n, n, n, ch), dtype=torch.bfloat16, device=device)
+    fine = rnd(2 * n, 2 * n, 2 * n, ch)
+    _native.call("warp_amd_relu_up2_bwd_bf16", n, ch, _native.ptr(fine), _native.ptr(y), _native.ptr(out), s)
+    total = torch.zeros((n, n, n, ch), device=device)
+    for k in range(8):
+        total = total + fine[k >> 2::2, (k >> 1) & 1::2, k & 1::2]
+    want = torch.where(y.float() > 0, total, torch.zeros_like(total)).to(torch.bfloat16)
+    assert torch.equal(out, want)
+    skip, dp = rnd(n, n, n, ch), rnd(n // 2, n // 2, n // 2, ch)
+    _native.call("warp_amd_relu_pool2_bwd_bf16", n, ch, _native.ptr(skip), _native.ptr(dp), _native.ptr(y),
+                 _native.ptr(out), s)
+    up = dp.repeat_interleave(2, 0).repeat_interleave(2, 1).repeat_interleave(2, 2)
+    total = skip + 0.125 * up
+    assert torch.equal(out, torch.where(y.float() > 0, total, torch.zeros_like(total)).to(torch.bfloat16))

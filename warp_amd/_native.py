@@ -196,6 +196,8 @@ _SIGNATURES = {
         c_int,
         [c_int, c_int, c_int, c_int, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_ptr, c_size, c_ptr],
     ),
+    "warp_amd_relu_up2_bwd_bf16": (c_int, [c_int, c_int] + [c_ptr] * 4),
+    "warp_amd_relu_pool2_bwd_bf16": (c_int, [c_int, c_int] + [c_ptr] * 5),
     "warp_amd_relu_mask_bf16": (c_int, [c_i64, c_ptr, c_ptr, c_ptr, c_ptr]),
     "warp_amd_f32_to_bf16": (c_int, [c_i64, c_ptr, c_ptr, c_ptr]),
     "warp_amd_bf16_to_f32": (c_int, [c_i64, c_ptr, c_ptr, c_ptr]),

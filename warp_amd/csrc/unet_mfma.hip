@@ -1300,6 +1300,77 @@ int launch_wgrad(int m, int in_mode, const unsigned short* x, const unsigned sho
     return kOk;
 }
 
+// A layer's output gradient in BF16, formed where its parts meet: the adjoint
+// of the resampling, the skip sum and the ReLU mask of the layer's stored
+// output y, rounded once.  FP32 sums in the order of the separate passes.
+// Bound by HBM: these passes used to write and read FP32 gradients between
+// them (pool2_bwd, relu_mask, f32_to_bf16, up2_bwd: 460 us a training gradient
+// at 128^3).
+
+// out = y > 0 ? sum of d over the 8 children : 0 (decoder layers; the adjoint
+// of upsampling).  n: coarse side; one thread per coarse voxel and four channels.
+__global__ __launch_bounds__(kBlock) void relu_up2_bwd_kernel(int n, int ch, const float* __restrict__ d,
+                                                              const unsigned short* __restrict__ y,
+                                                              unsigned short* __restrict__ out)
+{
+    const int q4 = ch / 4;
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= (int64_t)n * n * n * q4)
+        return;
+    const int c = (int)(i % q4);
+    const int64_t p = i / q4;
+    const int px = (int)(p % n), py = (int)((p / n) % n), pz = (int)(p / ((int64_t)n * n));
+    const int64_t nf = 2 * n;
+    f32x4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const int64_t f = 2 * px + (k & 1) + nf * (2 * py + ((k >> 1) & 1) + nf * (2 * pz + (k >> 2)));
+        v[k] = reinterpret_cast<const f32x4*>(d)[f * q4 + c];
+    }
+    const bf16x4 yv = reinterpret_cast<const bf16x4*>(y)[i];
+    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        s += v[k];
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        s[e] = bf2f((unsigned short)yv[e]) > 0.0f ? s[e] : 0.0f;
+    const unsigned st[2] = {pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])};
+    reinterpret_cast<bf16x4*>(out)[i] = __builtin_bit_cast(bf16x4, st);
+}
+
+// out = y > 0 ? d + dp / 8 : 0 (encoder layers; dp: gradient of the 2x2x2
+// average).  nf: fine side; one thread per voxel and eight channels.
+__global__ __launch_bounds__(kBlock) void relu_pool2_bwd_kernel(int nf, int ch, const float* __restrict__ d,
+                                                                const float* __restrict__ dp,
+                                                                const unsigned short* __restrict__ y,
+                                                                unsigned short* __restrict__ out)
+{
+    const int q8 = ch / 8;
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= (int64_t)nf * nf * nf * q8)
+        return;
+    const int c = (int)(i % q8);
+    const int64_t f = i / q8;
+    const int fx = (int)(f % nf), fy = (int)((f / nf) % nf), fz = (int)(f / ((int64_t)nf * nf));
+    const int64_t nc = nf / 2;
+    const int64_t p = fx / 2 + nc * (fy / 2 + nc * (fz / 2));
+    const f32x4* dv = reinterpret_cast<const f32x4*>(d) + 2 * i;
+    const f32x4* pv = reinterpret_cast<const f32x4*>(dp) + 2 * (p * q8 + c);
+    const f32x4 d0 = __builtin_nontemporal_load(dv), d1 = __builtin_nontemporal_load(dv + 1);
+    const f32x4 p0 = pv[0], p1 = pv[1];
+    const bf16x8 yv = reinterpret_cast<const bf16x8*>(y)[i];
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float g = (e < 4 ? d0[e % 4] : d1[e % 4]) + 0.125f * (e < 4 ? p0[e % 4] : p1[e % 4]);
+        s[e] = bf2f((unsigned short)yv[e]) > 0.0f ? g : 0.0f;
+    }
+    const unsigned st[4] = {pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3]), pack_bf16x2(s[4], s[5]),
+                            pack_bf16x2(s[6], s[7])};
+    reinterpret_cast<bf16x8*>(out)[i] = __builtin_bit_cast(bf16x8, st);
+}
+
 // BF16 ReLU mask of an FP32 gradient: out = y > 0 ? dy : 0 (y BF16)
 __global__ __launch_bounds__(kBlock) void relu_mask_bf16_kernel(int64_t count, const unsigned short* __restrict__ y,
                                                                 const float* __restrict__ dy, float* __restrict__ out)
@@ -1520,6 +1591,39 @@ WA_API int warp_amd_relu_mask_bf16(int64_t count, const void* y, const float* dy
     wa::relu_mask_bf16_kernel<<<(unsigned)wa::ceil_div(count, wa::kBlock), wa::kBlock, 0, wa::as_stream(stream)>>>(
         count, static_cast<const unsigned short*>(y), dy, out
     );
+    WA_LAUNCH_CHECK();
+    return wa::kOk;
+}
+
+// BF16 output gradient of a decoder layer: out [n^3][ch] = y > 0 ? the sum of
+// d [(2n)^3][ch] over each voxel's 8 children : 0.  ch a multiple of 8, arrays
+// 16-byte aligned.
+WA_API int warp_amd_relu_up2_bwd_bf16(int n, int ch, const float* d, const void* y, void* out, void* stream)
+{
+    WA_REQUIRE(n > 0 && ch > 0 && ch % 8 == 0, "relu_up2_bwd: unsupported shape (side %d, %d channels)", n, ch);
+    WA_REQUIRE(d && y && out, "relu_up2_bwd: null array");
+    WA_REQUIRE(((uintptr_t)d | (uintptr_t)y | (uintptr_t)out) % 16 == 0, "relu_up2_bwd: arrays must be 16-byte aligned");
+    const int64_t count = (int64_t)n * n * n * (ch / 4);
+    wa::relu_up2_bwd_kernel<<<(unsigned)wa::ceil_div(count, wa::kBlock), wa::kBlock, 0, wa::as_stream(stream)>>>(
+        n, ch, d, static_cast<const unsigned short*>(y), static_cast<unsigned short*>(out));
+    WA_LAUNCH_CHECK();
+    return wa::kOk;
+}
+
+// BF16 output gradient of an encoder layer: out [n^3][ch] = y > 0 ? d + the
+// gradient dp [(n/2)^3][ch] of its 2x2x2 average / 8 : 0.  n even, ch a
+// multiple of 8, arrays 16-byte aligned.
+WA_API int warp_amd_relu_pool2_bwd_bf16(int n, int ch, const float* d, const float* dp, const void* y, void* out,
+                                        void* stream)
+{
+    WA_REQUIRE(n > 0 && n % 2 == 0 && ch > 0 && ch % 8 == 0, "relu_pool2_bwd: unsupported shape (side %d, %d channels)",
+               n, ch);
+    WA_REQUIRE(d && dp && y && out, "relu_pool2_bwd: null array");
+    WA_REQUIRE(((uintptr_t)d | (uintptr_t)dp | (uintptr_t)y | (uintptr_t)out) % 16 == 0,
+               "relu_pool2_bwd: arrays must be 16-byte aligned");
+    const int64_t count = (int64_t)n * n * n * (ch / 8);
+    wa::relu_pool2_bwd_kernel<<<(unsigned)wa::ceil_div(count, wa::kBlock), wa::kBlock, 0, wa::as_stream(stream)>>>(
+        n, ch, d, dp, static_cast<const unsigned short*>(y), static_cast<unsigned short*>(out));
     WA_LAUNCH_CHECK();
     return wa::kOk;
 }

@@ -205,11 +205,28 @@ class UNet:
                          _native.ptr(t), s)
             self._wsw_t[name] = t
 
+    # A layer's output gradient in BF16, the operand of its weight and input gradients.
     def _dy_bf16(self, name, dy):
-        """A layer's FP32 output gradient in BF16, the operand of its weight and input gradients."""
+        """... from its FP32 form."""
         _, co, _, lvl = LAYER_INDEX[name]
         h = self._hbuf("gy_" + name, lvl, co)
         _native.call("warp_amd_f32_to_bf16", h.numel(), _native.ptr(dy), _native.ptr(h), self._s())
+        return h
+
+    def _dy_up(self, name, y, dfine):
+        """... of a layer whose output y is upsampled into an input with FP32 gradient dfine."""
+        _, co, _, lvl = LAYER_INDEX[name]
+        h = self._hbuf("gy_" + name, lvl, co)
+        _native.call("warp_amd_relu_up2_bwd_bf16", self.side(lvl), co, _native.ptr(dfine), _native.ptr(y),
+                     _native.ptr(h), self._s())
+        return h
+
+    def _dy_pool(self, name, y, dskip, dpool):
+        """... of a layer whose output y feeds a skip (FP32 gradient dskip) and a pooling (dpool)."""
+        _, co, _, lvl = LAYER_INDEX[name]
+        h = self._hbuf("gy_" + name, lvl, co)
+        _native.call("warp_amd_relu_pool2_bwd_bf16", self.side(lvl), co, _native.ptr(dskip), _native.ptr(dpool),
+                     _native.ptr(y), _native.ptr(h), self._s())
         return h
 
     def _wgrad_bf16(self, name, x, dy, coarse=None):
@@ -233,11 +250,6 @@ class UNet:
         _native.call("warp_amd_conv3_mfma", self.side(lvl), co, ci, 0, _native.ptr(dy), None,
                      _native.ptr(self._wsw_t[name]), None, 4, None, _native.ptr(dx), None, self._s())
 
-    def _relu_bf16(self, y_bf16, dy, out):
-        _native.call("warp_amd_relu_mask_bf16", dy.numel(), _native.ptr(y_bf16), _native.ptr(dy), _native.ptr(out),
-                     self._s())
-        return out
-
     def backward_bf16(self, dout: torch.Tensor) -> None:
         """Gradients of all parameters (into self.grads) for dL/dout after :meth:`forward_bf16`.
 
@@ -246,11 +258,10 @@ class UNet:
         same way) and the output gradients rounded to BF16; input gradients
         by the MFMA convolution with flipped weights (FP32 out); ReLU masks
         from the stored BF16 activations; pooling / upsampling adjoints and
-        the skip sums in FP32."""
+        the skip sums in FP32, rounded to BF16 once per layer."""
         if getattr(self, "_wsw_t", None) is None:
             self.sync_bf16_flipped()
         H, B = self._hbuf, self.buf
-        s = self._s()
         a0, p0 = H("a0", 0, 16), H("p0", 1, 16)
         a1, p1 = H("a1", 1, 32), H("p1", 2, 32)
         a2, p2 = H("a2", 2, 64), H("p2", 3, 64)
@@ -262,41 +273,32 @@ class UNet:
         da0 = B("da0", 0, 16)
         self._bwd_data_bf16("d0", dy, da0)
         # d1: input a1 + up(b2), output b1
-        g1 = B("g1", 1, 16)
-        _native.call("warp_amd_up2_bwd_f32", self.side(1), 16, _native.ptr(da0), _native.ptr(g1), s)
-        dy = self._dy_bf16("d1", self._relu_bf16(b1, g1, B("m1", 1, 16)))
+        dy = self._dy_up("d1", b1, da0)
         self._wgrad_bf16("d1", a1, dy, coarse=b2)
         da1 = B("da1", 1, 32)
         self._bwd_data_bf16("d1", dy, da1)
         # d2: input a2 + up(a3), output b2
-        g2 = B("g2", 2, 32)
-        _native.call("warp_amd_up2_bwd_f32", self.side(2), 32, _native.ptr(da1), _native.ptr(g2), s)
-        dy = self._dy_bf16("d2", self._relu_bf16(b2, g2, B("m2", 2, 32)))
+        dy = self._dy_up("d2", b2, da1)
         self._wgrad_bf16("d2", a2, dy, coarse=a3)
         da2 = B("da2", 2, 64)
         self._bwd_data_bf16("d2", dy, da2)
         # e3: input p2, output a3
-        g3 = B("g3", 3, 64)
-        _native.call("warp_amd_up2_bwd_f32", self.side(3), 64, _native.ptr(da2), _native.ptr(g3), s)
-        dy = self._dy_bf16("e3", self._relu_bf16(a3, g3, B("m3", 3, 64)))
+        dy = self._dy_up("e3", a3, da2)
         self._wgrad_bf16("e3", p2, dy)
         dp2 = B("dp2", 3, 64)
         self._bwd_data_bf16("e3", dy, dp2)
-        _native.call("warp_amd_pool2_bwd_f32", self.side(2), 64, _native.ptr(dp2), _native.ptr(da2), 1, s)
         # e2: input p1, output a2
-        dy = self._dy_bf16("e2", self._relu_bf16(a2, da2, B("m2b", 2, 64)))
+        dy = self._dy_pool("e2", a2, da2, dp2)
         self._wgrad_bf16("e2", p1, dy)
         dp1 = B("dp1", 2, 32)
         self._bwd_data_bf16("e2", dy, dp1)
-        _native.call("warp_amd_pool2_bwd_f32", self.side(1), 32, _native.ptr(dp1), _native.ptr(da1), 1, s)
         # e1: input p0, output a1
-        dy = self._dy_bf16("e1", self._relu_bf16(a1, da1, B("m1b", 1, 32)))
+        dy = self._dy_pool("e1", a1, da1, dp1)
         self._wgrad_bf16("e1", p0, dy)
         dp0 = B("dp0", 1, 16)
         self._bwd_data_bf16("e1", dy, dp0)
-        _native.call("warp_amd_pool2_bwd_f32", self.side(0), 16, _native.ptr(dp0), _native.ptr(da0), 1, s)
         # e0: input (BF16 network input), output a0
-        dy = self._dy_bf16("e0", self._relu_bf16(a0, da0, B("m0", 0, 16)))
+        dy = self._dy_pool("e0", a0, da0, dp0)
         self._wgrad_bf16("e0", self._inp_bf16, dy)
 
     def _layer_grads(self, name, x, y, dy, masked):
