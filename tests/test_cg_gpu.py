@@ -449,3 +449,48 @@ def test_segmented_dot_known_answers(device):
     bo = np.concatenate([[0], np.cumsum(sizes)])
     ref = np.array([math.fsum(x[s:e] * y[s:e]) for s, e in zip(bo[:-1], bo[1:])])
     np.testing.assert_allclose(got, ref, rtol=1e-12, atol=1e-12)
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("prec", ["diag", "id"])
+@pytest.mark.parametrize("dtype,n", [(torch.float32, 89), (torch.float64, 89), (torch.float64, 45)])
+def test_cg_vector_update_and_wave_spmv(device, dtype, n, prec, shift):
+    """Unfused scalar systems: the 16-byte update with its tail (odd n^3), wave
+    tiles from 2^19 FP64 rows on, the scalar update for an x that is not 16-byte
+    aligned.  Twelve iterations against the same recurrence in float64 torch.
+    Bound: rounding grows by at most the condition number (about 1e4 here) per
+    iteration's unit roundoff, 12 * 1e4 * 1.1e-16 = 1.3e-11 in FP64; FP32 stays
+    well below that (1e-6), and one wrong entry of N gives N^-1/2 > 1e-3."""
+    from warp_amd import problems
+
+    g = torch.Generator(device=device).manual_seed(n)
+    k = torch.exp(torch.randn((n, n, n), generator=g, device=device))
+    off, col, val = problems.fv7_poisson(k)
+    N = n**3
+    A = sparse.bsr_zeros(N, N, wa.types.type_to_scalar(dtype), device=device)
+    A.offsets, A.columns, A.values, A.nnz = off, col, val.to(dtype), col.numel()
+    b = torch.randn(N, generator=g, device=device, dtype=dtype)
+    store = torch.zeros(N + 8, dtype=dtype, device=device)
+    x = store[shift:shift + N]
+    it, _, _ = linear.cg(A, b, x, tol=1e-14, atol=0.0, maxiter=12, M=linear.preconditioner(A, prec))
+    assert it == 12 and float(store[N + shift:].abs().max()) == 0.0
+    rows = torch.repeat_interleave(torch.arange(N, device=device), (off[1:] - off[:-1]).long())
+    v64, c64 = val.double(), col.long()
+
+    def mv(u):
+        return torch.zeros(N, dtype=torch.float64, device=device).index_add(0, rows, v64 * u[c64])
+
+    inv = 1.0 / v64[rows == c64] if prec == "diag" else torch.ones(N, dtype=torch.float64, device=device)
+    xs = torch.zeros(N, dtype=torch.float64, device=device)
+    r = b.double()
+    z = inv * r
+    p, rz = z, r @ z
+    for _ in range(12):
+        q = mv(p)
+        a = rz / (p @ q)
+        xs, r = xs + a * p, r - a * q
+        z = inv * r
+        rz, old = r @ z, rz
+        p = z + (rz / old) * p
+    rel = float((x.double() - xs).norm() / xs.norm())
+    assert rel < (2e-5 if dtype == torch.float32 else 1.3e-11), rel

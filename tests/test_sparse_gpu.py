@@ -1521,3 +1521,35 @@ def test_bsr_mv_transpose_symmetric_pattern_is_deterministic(device, bshape, dty
     DB = _dense_of(B)
     if not np.array_equal(DB != 0, (DB != 0).T):
         assert not sparse._mirror_symmetric(B)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_bsr_mv_wave_tiles_equal_lane_groups(device, dtype, shift):
+    """Large scalar matrices (wave tiles) against four lanes per row (tile_size=4):
+    the same order per row, so the same bits.  Empty rows, rows far above a
+    tile's LDS image, a ragged last tile, alpha / beta, both traversal
+    directions, arrays that are not 16-byte aligned (the lane groups there)."""
+    nrow = (1 << 21) + 37 if dtype == torch.float32 else (1 << 18) + 37
+    g = torch.Generator(device=device).manual_seed(5)
+    counts = torch.randint(0, 12, (nrow,), generator=g, device=device)
+    counts[1000:1003] = 700
+    counts[5000:5200] = 0
+    counts[-1] = 3
+    off = torch.zeros(nrow + 1, dtype=torch.int64, device=device)
+    off[1:] = torch.cumsum(counts, 0)
+    nnz = int(off[-1])
+    assert 4 < nnz / nrow < 7.25
+    cols = torch.randint(0, nrow, (nnz + 8,), generator=g, device=device).to(torch.int32)
+    vals = torch.randn(nnz + 8, generator=g, device=device, dtype=dtype)
+    A = sparse.bsr_zeros(nrow, nrow, wa.types.type_to_scalar(dtype), device=device)
+    A.offsets, A.columns, A.values, A.nnz = off.to(torch.int32), cols[shift:], vals[shift:], nnz
+    x = torch.randn(nrow, generator=g, device=device, dtype=dtype)
+    y0 = torch.randn(nrow, generator=g, device=device, dtype=dtype)
+    for alpha, beta in ((1.0, 0.0), (-0.5, 2.0), (1.0, 0.0)):
+        want, got = y0.clone(), y0.clone()
+        sparse.bsr_mv(A, x, want, alpha=alpha, beta=beta, tile_size=4)
+        sparse.bsr_mv(A, x, got, alpha=alpha, beta=beta)
+        assert torch.equal(got, want)
+        sparse.bsr_mv(A, x, got.copy_(y0), alpha=alpha, beta=beta)
+        assert torch.equal(got, want)

@@ -193,4 +193,147 @@ inline BsrShape default_bsr_shape(int nrow, int br, int bc, int64_t nnz_hint)
     return BsrShape{g, rows_per_group_for(br, bc)};
 }
 
+// ---------------------------------------------------------------------------
+// Scalar rows by wave tiles
+// ---------------------------------------------------------------------------
+//
+// A wavefront takes RW consecutive scalar rows: it loads their columns and
+// values in 16-byte pieces (four entries per lane, CH times), gathers x for
+// them, lays (value, x) out in LDS, and each lane adds one row from there, in
+// the order of group_row_product with G lanes (entry k into partial k % G, then
+// the butterfly), so the bits are the same.  What limits the lane-group kernel
+// on 7- and 9-entry rows is the rate of 4-byte requests (a plain copy at 4
+// bytes per lane reaches 3.7 TB/s here, at 16 bytes 6.5); no barrier is needed,
+// since a wave reads only what it wrote.  7-point rows, us per product with
+// alternating direction, lane groups / wave tiles: FP32 128^3 26.6 / 24.5,
+// 200^3 105 / 95, 256^3 241 / 200 (5.7 TB/s); FP64 128^3 41 / 33, 161^3 92 / 73,
+// 195^3 155 / 130.  FP64 tiles are half as long (RW = 32, CH = 1: their LDS
+// image is twice as large; 64 rows took 87 us at 161^3).  A tile whose entries
+// exceed the LDS image (rows far above the mean) is added from global memory.
+// Persistent workgroups that load the next tile ahead were slower (262 us at
+// 256^3), as were non-temporal matrix loads wherever consecutive products meet
+// in the memory-side cache (30 us at 128^3).
+//
+// The tiles are dealt to the XCDs in runs (xcd_run_block), so that the rows of
+// neighbouring tiles find their x in one L2 (FP32 256^3 214 -> 203 us; runs of
+// 32 or 64 gain 1 % more there and lose 4 % at 128^3).
+constexpr int kWaveTileEntries = 256;  // entries of one 16-byte piece per lane
+
+template <typename S, typename V, int CH> struct WaveTile {
+    V v[CH * kWaveTileEntries];
+    S x[CH * kWaveTileEntries];
+};
+
+// Workgroup b of `grid`, renumbered so that XCD b % 8 gets runs of consecutive
+// workgroups; a bijection for any grid.
+__device__ __forceinline__ int xcd_run_block(int b, int grid)
+{
+    constexpr int kXcd = 8, kRun = 8;
+    const int full = grid - grid % (kXcd * kRun);
+    if (b >= full)
+        return b;
+    const int i = b / kXcd;
+    return ((i / kRun) * kXcd + b % kXcd) * kRun + i % kRun;
+}
+
+// Sum of row row0 + lane (lane < RW and row < nrow, else 0).  STREAM: columns
+// and values are loaded past the caches.
+template <typename S, int G, int RW, int CH, bool STREAM = false, typename V, typename XF>
+__device__ __forceinline__ S wave_rows_product(int row0, int nrow, int lane, const int* __restrict__ offsets,
+                                               const int* __restrict__ columns, const V* __restrict__ values, XF x,
+                                               WaveTile<S, V, CH>& tile)
+{
+    typedef int I4 __attribute__((ext_vector_type(4)));
+    typedef V V4 __attribute__((ext_vector_type(4)));
+    typedef S S4 __attribute__((ext_vector_type(4)));
+    const int row = row0 + lane;
+    const bool on = lane < RW && row < nrow;
+    const int beg = on ? offsets[row] : 0;
+    const int end = on ? offsets[row + 1] : 0;
+    const int nnz = offsets[nrow];
+    const int last = (nrow - row0 < RW ? nrow - row0 : RW) - 1;
+    const int b0 = __builtin_amdgcn_readfirstlane(beg);
+    const int e0 = __builtin_amdgcn_readlane(end, last);
+    const int base = b0 & ~3;
+    S a[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+        a[g] = S(0);
+    if (e0 - base <= CH * kWaveTileEntries) {  // wave-uniform
+        I4 c[CH];
+        V4 v[CH];
+#pragma unroll
+        for (int u = 0; u < CH; ++u) {
+            const int k = base + (u * kWave + lane) * 4;
+            if (k < e0) {
+                if (k + 3 < nnz) {
+                    c[u] = stream_load<STREAM>(reinterpret_cast<const I4*>(columns + k));
+                    v[u] = stream_load<STREAM>(reinterpret_cast<const V4*>(values + k));
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        c[u][q] = k + q < nnz ? columns[k + q] : 0;
+                        v[u][q] = k + q < nnz ? values[k + q] : V(0);
+                    }
+                }
+            }
+        }
+        S4 xv[CH];
+#pragma unroll
+        for (int u = 0; u < CH; ++u) {
+            const int k = base + (u * kWave + lane) * 4;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                xv[u][q] = (k + q >= b0 && k + q < e0) ? x((size_t)c[u][q]) : S(0);
+        }
+#pragma unroll
+        for (int u = 0; u < CH; ++u) {
+            const int k = (u * kWave + lane) * 4;
+            if (base + k < e0) {
+                *reinterpret_cast<V4*>(tile.v + k) = v[u];
+                *reinterpret_cast<S4*>(tile.x + k) = xv[u];
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int k = beg; k < end; k += G) {
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const bool in = k + g < end;
+                const int i = (in ? k + g : beg) - base;
+                const S t = fma((S)tile.v[i], tile.x[i], a[g]);
+                a[g] = in ? t : a[g];
+            }
+        }
+    } else {
+        for (int k = beg; k < end; k += G) {
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+                if (k + g < end)
+                    a[g] = fma((S)values[k + g], x((size_t)columns[k + g]), a[g]);
+        }
+    }
+#pragma unroll
+    for (int off = G / 2; off > 0; off >>= 1)
+#pragma unroll
+        for (int g = 0; g < off; ++g)
+            a[g] = a[g] + a[g + off];
+    return a[0];
+}
+
+// Wave tiles take compact scalar matrices with 16-byte aligned columns and
+// values, 4 lanes per row (more than 4 entries per row on average) and at most
+// 7.25, so that nearly every tile of 32 or 64 rows fits its image of 8 entries
+// per row (9-entry rows, 24 to 48 of them per tile, were slower: FP64 60
+// against 48 us on 1400^2 nodes).  The smallest systems stay with the lane
+// groups, which have more waves in flight there: FP32 values and x below 2M
+// rows (100^3 15.5 / 16.3 us), otherwise below 2^18 (64^3 FP64 6.9 / 6.1 us,
+// 41^3 even).
+inline bool wave_rows_supported(int lanes, int nrow, int64_t nnz_hint, bool wide_x, const int* row_counts,
+                                const void* columns, const void* values)
+{
+    return lanes == 4 && nrow >= (wide_x ? 1 << 18 : 1 << 21) && 4 * nnz_hint <= (int64_t)29 * nrow && !row_counts &&
+           (((uintptr_t)columns | (uintptr_t)values) & 15) == 0;
+}
+
 }  // namespace wa

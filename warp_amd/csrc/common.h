@@ -159,6 +159,23 @@ template <typename T> __device__ __forceinline__ void store_agent(T* p, T v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Loads and stores that bypass the caches where STREAM is set: for data that
+// is not touched again before it would have been displaced.
+template <bool STREAM, typename T> __device__ __forceinline__ T stream_load(const T* p)
+{
+    if constexpr (STREAM)
+        return __builtin_nontemporal_load(p);
+    else
+        return *p;
+}
+template <bool STREAM, typename T> __device__ __forceinline__ void stream_store(T v, T* p)
+{
+    if constexpr (STREAM)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+
 // Block partial sums for a following finalize kernel: thread 0 of workgroup b
 // writes the NV workgroup sums to partials[v * gridDim.x + b] with plain
 // stores (the kernel boundary makes them visible; no per-workgroup fences,

@@ -335,6 +335,40 @@ __global__ __launch_bounds__(kBlock) void cg_spmv_kernel(
     write_block_partials<kBlock, 1>(acc, parts, lds);
 }
 
+// The unfused SpMV of large scalar systems by wave tiles (see
+// wave_rows_product; each row's sum as above), one workgroup of four tiles
+// each, their partials reduced as the wide grid's.  256^3 FP32: 250-261 ->
+// 220 us.
+template <typename S, int G, int RW, int CH, bool STREAM>
+__global__ __launch_bounds__(kBlock) void cg_spmv_wave_kernel(
+    int nrow, const int* __restrict__ offsets, const int* __restrict__ columns, const S* __restrict__ values,
+    S* __restrict__ Ap, CgWs ws, double* __restrict__ parts
+)
+{
+    __shared__ __attribute__((aligned(16))) WaveTile<S, S, CH> tiles[kBlock / kWave];
+    __shared__ double lds[kBlock / kWave];
+    const CgState* state = ws.state;
+    if (state->done)
+        return;
+    const S* __restrict__ p = static_cast<const S*>(ws.p);
+    int b = xcd_run_block((int)blockIdx.x, (int)gridDim.x);
+    if (state->iter & 1)  // odd iterations from the last tile, as above
+        b = (int)gridDim.x - 1 - b;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int64_t first = ((int64_t)b * (kBlock / kWave) + wave) * RW;
+    double acc[1] = {0.0};
+    if (first < nrow) {
+        const int row0 = (int)first;
+        const S v =
+            wave_rows_product<S, G, RW, CH, STREAM>(row0, nrow, lane, offsets, columns, values, LoadX<S>{p}, tiles[wave]);
+        if (lane < RW && row0 + lane < nrow) {
+            Ap[row0 + lane] = v;
+            acc[0] = (double)p[row0 + lane] * (double)v;
+        }
+    }
+    write_block_partials<kBlock, 1>(acc, parts, lds);
+}
+
 // Wide SpMV grids (one workgroup per tile, more than kMaxSpmvGrid): their
 // partials reduced to kWideParts, workgroup b summing the b-th contiguous
 // range in a fixed order into spmv_partials[b]; the update sums those.
@@ -431,12 +465,101 @@ __global__ __launch_bounds__(kBlock) void cg_update_kernel(
     write_block_partials<kBlock, 2>(acc, ws.upd_partials, lds);
 }
 
+// The same pass over scalars in 16-byte vectors, for a point preconditioner (or
+// none): each thread loads its next vectors while it stores the current ones.
+// Bound by its eight streams (5.5 TB/s at 256^3 FP32); 100^3 FP32 33.4 -> 32.0
+// us per iteration against one row per thread.  2048 workgroups, and vectors
+// skewed against each other in the workspace, measured the same.
+template <typename S, int PREC, bool STREAM>
+__global__ __launch_bounds__(kBlock) void cg_update_vec_kernel(
+    int64_t n, const S* __restrict__ prec, S* __restrict__ x, S* __restrict__ r, S* __restrict__ z,
+    const S* __restrict__ Ap, int spmv_parts, CgWs ws
+)
+{
+    constexpr int kV = 16 / (int)sizeof(S);
+    typedef S V __attribute__((ext_vector_type(kV)));
+    __shared__ double lds[kBlock / kWave];
+    CgState* state = ws.state;
+    const int done = state->done;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        state->rz_prev = state->rz;
+        state->done_prev = done;
+        if (!done)
+            state->iter = state->iter + 1;
+    }
+    if (done)
+        return;
+    const S* __restrict__ p = dir_buffer<S>(ws, 0);
+    const V* __restrict__ pv = reinterpret_cast<const V*>(p);
+    const V* __restrict__ av = reinterpret_cast<const V*>(Ap);
+    const V* __restrict__ mv = reinterpret_cast<const V*>(prec);
+    V* __restrict__ xv = reinterpret_cast<V*>(x);
+    V* __restrict__ rv = reinterpret_cast<V*>(r);
+    V* __restrict__ zv = reinterpret_cast<V*>(z);
+    const int64_t nv = n / kV;
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    V pc = {}, ac = {}, xc = {}, rc = {}, mc = {};
+    auto load = [&](int64_t k) {
+        pc = pv[k];
+        ac = stream_load<STREAM>(av + k);
+        xc = stream_load<STREAM>(xv + k);
+        rc = stream_load<STREAM>(rv + k);
+        if (PREC == kPrecDiag)
+            mc = stream_load<STREAM>(mv + k);
+    };
+    if (i < nv)
+        load(i);
+    double t[1];
+    sum_parts<1, kMaxSpmvGrid>(ws.spmv_partials, 0, spmv_parts, lds, t);
+    const double a = state->rr > state->atol_sq ? state->rz / t[0] : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        state->pAp = t[0];
+        state->alpha = a;
+    }
+    const S alpha = (S)a;
+    double acc[2] = {0.0, 0.0};
+    for (; i < nv; i += stride) {
+        V xn, rn, zn;
+#pragma unroll
+        for (int k = 0; k < kV; ++k) {
+            xn[k] = fma(alpha, pc[k], xc[k]);
+            rn[k] = fma(-alpha, ac[k], rc[k]);
+            zn[k] = PREC == kPrecDiag ? mc[k] * rn[k] : rn[k];
+        }
+        if (i + stride < nv)
+            load(i + stride);
+        stream_store<STREAM>(xn, xv + i);
+        stream_store<STREAM && PREC != kPrecNone>(rn, rv + i);  // r is the next direction without one
+        if (PREC != kPrecNone)
+            zv[i] = zn;
+#pragma unroll
+        for (int k = 0; k < kV; ++k) {
+            acc[0] += (double)rn[k] * (double)rn[k];
+            acc[1] += (double)rn[k] * (double)zn[k];
+        }
+    }
+    // the last n % kV entries
+    const int64_t j = nv * kV + threadIdx.x;
+    if (blockIdx.x == 0 && j < n) {
+        x[j] = fma(alpha, p[j], x[j]);
+        const S rj = fma(-alpha, Ap[j], r[j]);
+        r[j] = rj;
+        const S zj = PREC == kPrecDiag ? prec[j] * rj : rj;
+        if (PREC != kPrecNone)
+            z[j] = zj;
+        acc[0] += (double)rj * (double)rj;
+        acc[1] += (double)rj * (double)zj;
+    }
+    write_block_partials<kBlock, 2>(acc, ws.upd_partials, lds);
+}
+
 // p = z + beta p (unfused path).  The prologue sums the update's partials
 // into r.r and r.z of the new iterate, forms beta and `done`; workgroup 0
 // records them.  z and p are 256-byte aligned workspace slices, moved in
 // 16-byte vectors (the first ones loaded before the prologue, the next ones
 // while the current are stored); one fma per entry, as a scalar loop.
-template <typename S>
+template <typename S, bool STREAM>
 __global__ __launch_bounds__(kBlock) void cg_direction_kernel(int64_t n, const S* __restrict__ z, S* __restrict__ p,
                                                               int upd_parts, CgWs ws)
 {
@@ -453,7 +576,7 @@ __global__ __launch_bounds__(kBlock) void cg_direction_kernel(int64_t n, const S
     int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     V zc = {}, pc = {};
     if (i < nv) {
-        zc = zv[i];
+        zc = stream_load<STREAM>(zv + i);
         pc = pv[i];
     }
     double t[2];
@@ -470,7 +593,7 @@ __global__ __launch_bounds__(kBlock) void cg_direction_kernel(int64_t n, const S
     for (; i < nv; i += stride) {
         V zn = {}, pn = {};
         if (i + stride < nv) {
-            zn = zv[i + stride];
+            zn = stream_load<STREAM>(zv + i + stride);
             pn = pv[i + stride];
         }
         V o;
@@ -588,9 +711,37 @@ template <typename S> struct CgLauncher {
     // persistent workgroups whose partials the update sums in its prologue
     // (64^3 3x3 elasticity, 17,164 tiles: 66 us per iteration, 71 with the wide grid).
     static constexpr unsigned kWideSpmvTiles = 16u * kMaxSpmvGrid;
-    template <int BR, int G> bool wide_spmv() const { return !fused && rows_grid<BR, G>() > kWideSpmvTiles; }
+    template <int BR, int G> bool wide_spmv() const
+    {
+        return !fused && (rows_grid<BR, G>() > kWideSpmvTiles || wave_spmv<BR, G>());
+    }
+    static constexpr int kWaveRW = sizeof(S) == 4 ? 64 : 32, kWaveCH = sizeof(S) == 4 ? 2 : 1;
+    template <int BR, int G> bool wave_spmv() const
+    {
+        // 65^3 FP64 23.9 us per iteration, 24.9 by wave tiles (their partials take a
+        // launch more), 100^3 45.1 / 42.7, 128^3 84.9 / 70
+        return !fused && BR == 1 && G == 4 && pb.nrow >= (1 << 19) &&
+               wave_rows_supported(G, pb.nrow, pb.nnz_hint, sizeof(S) == 8, nullptr, pb.columns, pb.values);
+    }
+    // What bypasses the caches (256 MB memory-side).  The matrix, where it is
+    // twice that: a product cannot start on what the last one left, and p, Ap
+    // and z stay for the next pass (256^3 FP32 348 -> 337 us per iteration; a
+    // 420 MB FP64 matrix 194 -> 207, so not below).  x, r and the
+    // preconditioner, touched once per iteration, where an iteration's matrix
+    // and vectors exceed it and a vector its L2 (256^3 FP32 366 -> 337 us,
+    // 160^3 90 -> 84, 128^3 FP64 77 -> 73; 128^3 FP32, 167 MB in all, 49 -> 55,
+    // so not below).
+    int64_t matrix_bytes() const { return pb.nnz_hint * (int64_t)(sizeof(int) + pb.br * pb.br * sizeof(S)); }
+    int64_t vector_bytes() const { return (int64_t)pb.nrow * pb.br * (int64_t)sizeof(S); }
+    bool stream_matrix() const { return matrix_bytes() > ((int64_t)512 << 20); }
+    bool stream_vectors() const
+    {
+        return vector_bytes() > ((int64_t)8 << 20) && matrix_bytes() + 6 * vector_bytes() > ((int64_t)256 << 20);
+    }
     template <int BR, int G> unsigned spmv_grid() const
     {
+        if (wave_spmv<BR, G>())
+            return (unsigned)ceil_div(pb.nrow, (kBlock / kWave) * kWaveRW);
         return wide_spmv<BR, G>() ? rows_grid<BR, G>() : std::min<unsigned>(rows_grid<BR, G>(), (unsigned)kMaxSpmvGrid);
     }
     // partials the update reads
@@ -602,8 +753,17 @@ template <typename S> struct CgLauncher {
     {
         return (unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(count, kBlock), kMaxVecGrid));
     }
-    // workgroups (= partials) of the update pass: one thread per block row
-    unsigned upd_grid() const { return vec_grid(pb.nrow); }
+    // The update in 16-byte vectors: unfused, point preconditioner, x and the
+    // preconditioner aligned (the workspace vectors are).
+    bool vec_update() const
+    {
+        return !fused && pb.prec_kind != kPrecBlock && (((uintptr_t)pb.x | (uintptr_t)pb.prec) & 15) == 0;
+    }
+    // workgroups (= partials) of the update pass: one thread per vector or block row
+    unsigned upd_grid() const
+    {
+        return vec_update() ? vec_grid(ceil_div((int64_t)pb.nrow * pb.br, 16 / (int)sizeof(S))) : vec_grid(pb.nrow);
+    }
 
     template <int BR, int G, int PREC> int init_t(int first)
     {
@@ -633,6 +793,20 @@ template <typename S> struct CgLauncher {
         // the wide grid's partials go to the initial residual's partial buffer
         // (unused between restarts; it holds one per workgroup of any row grid)
         double* parts = wide_spmv<BR, G>() ? ws.init_partials : ws.spmv_partials;
+        if constexpr (BR == 1 && G == 4) {
+            if (wave_spmv<BR, G>()) {
+                if (stream_matrix())
+                    cg_spmv_wave_kernel<S, G, kWaveRW, kWaveCH, true><<<grid, kBlock, 0, stream>>>(
+                        pb.nrow, pb.offsets, pb.columns, (const S*)pb.values, (S*)ws.Ap, ws, parts);
+                else
+                    cg_spmv_wave_kernel<S, G, kWaveRW, kWaveCH, false><<<grid, kBlock, 0, stream>>>(
+                        pb.nrow, pb.offsets, pb.columns, (const S*)pb.values, (S*)ws.Ap, ws, parts);
+                WA_LAUNCH_CHECK();
+                cg_wide_spmv_finalize_kernel<<<kWideParts, kFinalizeBlock, 0, stream>>>(parts, (int)grid, ws);
+                WA_LAUNCH_CHECK();
+                return kOk;
+            }
+        }
         cg_spmv_kernel<S, BR, G, false><<<grid, kBlock, 0, stream>>>(
             pb.nrow, pb.offsets, pb.columns, (const S*)pb.values, nullptr, (S*)ws.Ap, (int)upd_grid(), ws, parts
         );
@@ -657,6 +831,19 @@ template <typename S> struct CgLauncher {
         default: WA_SPMV_PARTS(BR, 64)
         }
 #undef WA_SPMV_PARTS
+        if constexpr (PREC != kPrecBlock) {
+            if (vec_update()) {
+                const int64_t n = (int64_t)pb.nrow * BR;
+                if (stream_vectors())
+                    cg_update_vec_kernel<S, PREC, true><<<upd_grid(), kBlock, 0, stream>>>(
+                        n, (const S*)pb.prec, (S*)pb.x, (S*)ws.r, (S*)ws.z, (const S*)ws.Ap, (int)spmv_parts, ws);
+                else
+                    cg_update_vec_kernel<S, PREC, false><<<upd_grid(), kBlock, 0, stream>>>(
+                        n, (const S*)pb.prec, (S*)pb.x, (S*)ws.r, (S*)ws.z, (const S*)ws.Ap, (int)spmv_parts, ws);
+                WA_LAUNCH_CHECK();
+                return kOk;
+            }
+        }
         cg_update_kernel<S, BR, PREC><<<upd_grid(), kBlock, 0, stream>>>(
             pb.nrow, (const S*)pb.prec, (S*)pb.x, (S*)ws.r, (S*)ws.z, (const S*)ws.Ap, fused ? 1 : 0, (int)spmv_parts,
             ws
@@ -724,7 +911,10 @@ template <typename S> struct CgLauncher {
     int direction()
     {
         const int64_t n = (int64_t)pb.nrow * pb.br;
-        cg_direction_kernel<S><<<vec_grid(n), kBlock, 0, stream>>>(n, z_vec(), (S*)ws.p, (int)upd_grid(), ws);
+        if (stream_vectors() && pb.prec_kind != kPrecNone)
+            cg_direction_kernel<S, true><<<vec_grid(n), kBlock, 0, stream>>>(n, z_vec(), (S*)ws.p, (int)upd_grid(), ws);
+        else
+            cg_direction_kernel<S, false><<<vec_grid(n), kBlock, 0, stream>>>(n, z_vec(), (S*)ws.p, (int)upd_grid(), ws);
         WA_LAUNCH_CHECK();
         return kOk;
     }
