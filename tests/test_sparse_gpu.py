@@ -1553,3 +1553,37 @@ def test_bsr_mv_wave_tiles_equal_lane_groups(device, dtype, shift):
         assert torch.equal(got, want)
         sparse.bsr_mv(A, x, got.copy_(y0), alpha=alpha, beta=beta)
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("renumber", [False, True])
+@pytest.mark.parametrize("bs,n", [(3, 21), (1, 45)])
+def test_bsr_mv_transpose_gather_grid_numbering(device, bs, n, renumber):
+    """The gathered transpose where the mirror tried first is right (grid order)
+    and where it is not (random numbering), over more workgroups than one run of
+    them per XCD: the bits of bsr_mv of the explicit transpose."""
+    g = torch.Generator(device=device).manual_seed(n)
+    node = torch.arange(n**3, device=device)
+    x, y, z = node % n, (node // n) % n, node // (n * n)
+    rows, cols = [], []
+    for dz in (-1, 0, 1):
+        for dy in (-1, 0, 1):
+            for dx in (-1, 0, 1):
+                if bs == 1 and abs(dx) + abs(dy) + abs(dz) > 1:
+                    continue
+                ok = ((x + dx >= 0) & (x + dx < n) & (y + dy >= 0) & (y + dy < n) & (z + dz >= 0) & (z + dz < n))
+                rows.append(node[ok])
+                cols.append((node + dx + n * dy + n * n * dz)[ok])
+    rows, cols = torch.cat(rows), torch.cat(cols)
+    if renumber:
+        perm = torch.randperm(n**3, generator=g, device=device)
+        rows, cols = perm[rows], perm[cols]
+    vals = torch.randn((rows.numel(), bs, bs), generator=g, device=device)
+    A = sparse.bsr_zeros(n**3, n**3, wa.float32 if bs == 1 else wa.mat33, device=device)
+    sparse.bsr_set_from_triplets(A, rows.to(torch.int32), cols.to(torch.int32),
+                                 vals.reshape(-1) if bs == 1 else vals, prune_numerical_zeros=False)
+    A.nnz_sync()
+    u = torch.randn((n**3, bs) if bs > 1 else (n**3,), generator=g, device=device)
+    T = sparse.bsr_transposed(A)
+    T.nnz_sync()
+    assert sparse._mirror_symmetric(A)
+    assert torch.equal(sparse.bsr_mv(A, u, transpose=True), sparse.bsr_mv(T, u))

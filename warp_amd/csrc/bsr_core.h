@@ -226,9 +226,9 @@ template <typename S, typename V, int CH> struct WaveTile {
 
 // Workgroup b of `grid`, renumbered so that XCD b % 8 gets runs of consecutive
 // workgroups; a bijection for any grid.
-__device__ __forceinline__ int xcd_run_block(int b, int grid)
+template <int kRun = 8> __device__ __forceinline__ int xcd_run_block(int b, int grid)
 {
-    constexpr int kXcd = 8, kRun = 8;
+    constexpr int kXcd = 8;
     const int full = grid - grid % (kXcd * kRun);
     if (b >= full)
         return b;

@@ -406,46 +406,75 @@ __global__ __launch_bounds__(kBlock) void bsr_mv_transpose_kernel(
 // y = alpha A^T x + beta y without atomics, for a square compact matrix
 // whose pattern is structurally symmetric (every block (r, c) has a mirror
 // (c, r)): output block row c gathers, over row c's blocks (c, r) in storage
-// order, the mirror block (r, c) -- found by binary search in row r -- times
-// x[r].  G lanes per output row: lane g takes blocks g, g + G, ... with fused
-// multiply-adds, then an xor butterfly; the result depends only on G.
+// order, the mirror block (r, c) times x[r].  G lanes per output row: lane g
+// takes blocks g, g + G, ... with fused multiply-adds, then an xor butterfly;
+// the result depends only on G.
+//
+// Where the mirror is: bound by the chain of dependent loads, so the block as
+// far from the end of row r as (c, r) is from the start of row c is tried
+// first; on grids and meshes numbered along their axes that is the mirror for
+// all but the boundary rows.  Elsewhere the binary search in row r goes on from
+// what its column says.
+// Workgroups are dealt to the XCDs in runs, since neighbouring output rows read
+// the same lines of values.
+// us per product (lanes as in bsr_mv), search alone / mirror tried first:
+// elasticity 53^3 91 / 51, 64^3 181 / 107, 2D Poisson 400^2 18 / 8.8, FP64
+// 7-point 100^3 75 / 49; elasticity 53^3 in random numbering 354 / 352.  Runs of
+// 1 / 8 / 128 workgroups: 78 / 69 / 57 at 53^3.  Loading the values before the
+// column is known (random numbering: 460) or two or four rows per group (59 and
+// 73 at 53^3) were slower.
+constexpr int kTransposeRun = 128;
+
 template <typename S, int B, int G>
 __global__ __launch_bounds__(kBlock) void bsr_mv_transpose_gather_kernel(
     int nrow, const int* __restrict__ offsets, const int* __restrict__ columns, const S* __restrict__ values,
     const S* __restrict__ x, S* __restrict__ y, S alpha, S beta
 )
 {
-    const int c = blockIdx.x * (kBlock / G) + threadIdx.x / G;
+    const int64_t first = (int64_t)xcd_run_block<kTransposeRun>((int)blockIdx.x, (int)gridDim.x) * (kBlock / G) +
+                          threadIdx.x / G;
     const int lane = threadIdx.x % G;
-    if (c >= nrow)
+    if (first >= nrow)
         return;
+    const int c = (int)first;
     const int beg = offsets[c];
-    const int end = offsets[c + 1];
+    const int count = offsets[c + 1] - beg;
     S acc[B];
 #pragma unroll
     for (int j = 0; j < B; ++j)
         acc[j] = S(0);
-    for (int k = beg + lane; k < end; k += G) {
-        const int r = columns[k];
+    for (int k = lane; k < count; k += G) {
+        const int r = columns[beg + k];
         if (r < 0 || r >= nrow)
             continue;
-        const int rend = offsets[r + 1];
-        int lo = offsets[r], hi = rend;
-        while (lo < hi) {
-            const int mid = lo + (hi - lo) / 2;
-            if (columns[mid] < c)
-                lo = mid + 1;
-            else
-                hi = mid;
+        const int rbeg = offsets[r], rend = offsets[r + 1];
+        if (rbeg >= rend)
+            continue;
+        S xr[B];
+#pragma unroll
+        for (int i = 0; i < B; ++i)
+            xr[i] = x[(size_t)r * B + i];
+        int at = max(rbeg, rend - 1 - k);
+        const int found = columns[at];
+        if (found != c) {
+            int lo = found < c ? at + 1 : rbeg, hi = found < c ? rend : at;
+            while (lo < hi) {
+                const int mid = lo + (hi - lo) / 2;
+                if (columns[mid] < c)
+                    lo = mid + 1;
+                else
+                    hi = mid;
+            }
+            if (lo == rend || columns[lo] != c)
+                continue;  // no mirror block (the caller checks that there is always one)
+            at = lo;
         }
-        if (lo == rend || columns[lo] != c)
-            continue;  // no mirror block (the caller checks that there is always one)
-        const S* blk = values + (size_t)lo * (B * B);  // block (r, c): B x B, row-major
+        const S* blk = values + (size_t)at * (B * B);  // block (r, c): B x B, row-major
 #pragma unroll
         for (int j = 0; j < B; ++j)
 #pragma unroll
             for (int i = 0; i < B; ++i)
-                acc[j] = fma(blk[i * B + j], x[(size_t)r * B + i], acc[j]);
+                acc[j] = fma(blk[i * B + j], xr[i], acc[j]);
     }
 #pragma unroll
     for (int j = 0; j < B; ++j) {
