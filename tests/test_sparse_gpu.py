@@ -1587,3 +1587,33 @@ def test_bsr_mv_transpose_gather_grid_numbering(device, bs, n, renumber):
     T.nnz_sync()
     assert sparse._mirror_symmetric(A)
     assert torch.equal(sparse.bsr_mv(A, u, transpose=True), sparse.bsr_mv(T, u))
+
+
+@pytest.mark.parametrize("nrow", [1, 63, 1000, 16383, 16384, 16385, 40000])
+@pytest.mark.parametrize("order", ["sorted", "runs", "random"])
+def test_single_level_assembly_vs_unique(device, nrow, order):
+    """Few triplets (one-level bucketing: row ranks from runs of equal rows in a
+    wave, the one-workgroup scan up to 16,384 rows and the tiled one above),
+    invalid and all-zero triplets among them: topology of the sorted unique keys,
+    sums in ascending triplet order."""
+    g = torch.Generator().manual_seed(nrow)
+    T = 30_011
+    rows = torch.randint(-1, nrow + 1, (T,), generator=g)
+    if order == "sorted":
+        rows = rows.sort().values
+    elif order == "runs":
+        rows = rows[: T // 7 + 1].repeat_interleave(7)[:T]
+    cols = torch.randint(0, min(nrow, 40), (T,), generator=g)
+    vals = torch.randint(-3, 4, (T,), generator=g).float()  # exact sums, zeros pruned
+    A = sparse.bsr_zeros(nrow, nrow, wa.float32, device=device)
+    sparse.bsr_set_from_triplets(A, rows.to(torch.int32).to(device), cols.to(torch.int32).to(device), vals.to(device))
+    nnz = A.nnz_sync()
+    keep = (rows >= 0) & (rows < nrow) & (vals != 0)
+    key, inv = torch.unique(rows[keep] * nrow + cols[keep], sorted=True, return_inverse=True)
+    want = torch.zeros(key.numel()).index_add(0, inv, vals[keep])
+    off = torch.zeros(nrow + 1, dtype=torch.int64)
+    off[1:] = torch.cumsum(torch.bincount(key // nrow, minlength=nrow), 0)
+    assert nnz == key.numel()
+    assert torch.equal(A.offsets.cpu().long(), off)
+    assert torch.equal(A.columns[:nnz].cpu().long(), key % nrow)
+    assert torch.equal(A.values[:nnz].cpu(), want)

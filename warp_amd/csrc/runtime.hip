@@ -166,6 +166,70 @@ __global__ __launch_bounds__(kScanBlock) void scan_tile_kernel(
     }
 }
 
+// At most kScanOne items: one workgroup and one launch instead of two.  All
+// loads up front, transposed through LDS so that each thread sums 16
+// consecutive items; bound by that one workgroup's latency.
+constexpr int kScanOneThreads = 1024;
+constexpr int kScanOnePer = 16;
+constexpr int64_t kScanOne = (int64_t)kScanOneThreads * kScanOnePer;
+
+template <bool CLEAR>
+__global__ __launch_bounds__(kScanOneThreads) void scan_one_kernel(int* in, int* out, int n)
+{
+    __shared__ int items[kScanOneThreads * (kScanOnePer + 1)];  // item i at i + i / 16: no bank conflicts
+    __shared__ int totals[kScanOneThreads / kWave];
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+    int v[kScanOnePer];
+#pragma unroll
+    for (int k = 0; k < kScanOnePer; ++k) {
+        const int i = k * kScanOneThreads + tid;
+        v[k] = i < n ? in[i] : 0;
+    }
+#pragma unroll
+    for (int k = 0; k < kScanOnePer; ++k) {
+        const int i = k * kScanOneThreads + tid;
+        items[i + i / kScanOnePer] = v[k];
+    }
+    __syncthreads();
+    int* mine = items + tid * (kScanOnePer + 1);
+    int run = 0;
+#pragma unroll
+    for (int k = 0; k < kScanOnePer; ++k) {
+        v[k] = run;
+        run += mine[k];
+    }
+    int incl = run;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int t = __shfl_up(incl, off);
+        incl += lane >= off ? t : 0;
+    }
+    if (lane == kWave - 1)
+        totals[wave] = incl;
+    __syncthreads();
+    int prefix = incl - run, total = 0;
+#pragma unroll
+    for (int w = 0; w < kScanOneThreads / kWave; ++w) {
+        prefix += w < wave ? totals[w] : 0;
+        total += totals[w];
+    }
+#pragma unroll
+    for (int k = 0; k < kScanOnePer; ++k)
+        mine[k] = prefix + v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kScanOnePer; ++k) {
+        const int i = k * kScanOneThreads + tid;
+        if (i < n) {
+            out[i] = items[i + i / kScanOnePer];
+            if (CLEAR)
+                in[i] = 0;
+        }
+    }
+    if (tid == 0)
+        out[n] = total;
+}
+
 __global__ void scan_empty_kernel(int* out) { *out = 0; }
 
 __global__ __launch_bounds__(256) void fill_i32_kernel(int* p, int64_t n, int v)
@@ -204,6 +268,11 @@ int scan_i32(int* in, int* out, int64_t n, void* ws, hipStream_t stream)
         return kOk;
     }
     const int64_t tiles = ceil_div(n, kScanTile);
+    if (n <= kScanOne) {
+        scan_one_kernel<CLEAR><<<1, kScanOneThreads, 0, stream>>>(in, out, (int)n);
+        WA_LAUNCH_CHECK();
+        return kOk;
+    }
     int* partials = static_cast<int*>(ws);
     // The reduce pass reads `in` before the tile pass overwrites it, so in-place use is safe.
     scan_reduce_kernel<<<(unsigned)tiles, kScanBlock, 0, stream>>>(in, n, partials);

@@ -22,8 +22,8 @@
 //      ends (summed_block_offsets) when asked for, and per unique block
 //      values = v[i0] + v[i1] + ... sequentially in ascending triplet order
 //      (bit-identical to the reference CUDA order).
-// Matrices of more than 4096 * 4096 rows use a single-level row histogram and
-// scatter with global atomics for steps 1-4.
+// Few triplets, and matrices of more than 4096 * 4096 rows, use a single-level
+// row histogram with global atomics and a scatter for steps 1-4.
 #include "common.h"
 
 #include <algorithm>
@@ -59,6 +59,13 @@ constexpr int kMinTile = 16384;
 // contiguously (~kSubTile / buckets keys per run) instead of key by key.
 constexpr int kStagedBuckets = 256;
 constexpr int kSubTile = 4096;
+// At most this many triplets are bucketed at one level, by a row histogram of
+// global atomics (row_rank): there the latency of the two-level passes' few
+// workgroups and extra launches counts more than the atomics.  Whole assembly,
+// two levels / one, us: 16 K triplets 104 / 65, 262 K in element order 126 / 78,
+// shuffled 123 / 91, 512 K shuffled 129 / 121, 1.0 M shuffled 149 / 157 (in
+// element order 151 / 97, but the order is not known here).
+constexpr int kSingleLevelMax = 3 << 18;
 
 struct Partition {
     int shift = 0;
@@ -81,7 +88,7 @@ Partition partition_of(int nrow, int T)
     p.nb = (int)buckets(p.shift);
     if (p.nb < 1)
         p.nb = 1;
-    p.tiled = (1 << p.shift) <= kMaxBucketRows && T > 0 && nrow > 0;
+    p.tiled = (1 << p.shift) <= kMaxBucketRows && T > kSingleLevelMax && nrow > 0;
     p.staged = p.staged && p.tiled;
     const int64_t per = (T + kMaxTiles - 1) / kMaxTiles;
     p.tile = (int)(per > kMinTile ? (per + kBlock - 1) / kBlock * kBlock : kMinTile);
@@ -119,6 +126,7 @@ TripletWs carve_ws(void* base, size_t bytes, int nrow, int T, bool own_summed, s
     const int64_t ntile_hist = w.part.tiled ? (int64_t)w.part.nb * w.part.ntiles + 1 : 1;
     w.trow = c.take<int>((size_t)T);
     w.hist = c.take<int>((size_t)nrow + 1);
+    w.counters = c.take<int>(kListCounters);  // right after hist: one fill clears both
     w.row_start = c.take<int>((size_t)nrow + 1);
     w.keys = c.take<uint64_t>((size_t)T);
     w.alt = c.take<uint64_t>((size_t)T);
@@ -126,7 +134,6 @@ TripletWs carve_ws(void* base, size_t bytes, int nrow, int T, bool own_summed, s
     w.tile_offsets = c.take<int>((size_t)ntile_hist);
     w.large_rows = c.take<int>((size_t)nrow + 1);
     w.medium_rows = c.take<int>((size_t)nrow + 1);
-    w.counters = c.take<int>(kListCounters);
     w.scan_ws = c.take<char>(scan_workspace_bytes(std::max<int64_t>((int64_t)nrow + 1, ntile_hist)));
     w.summed_offsets = own_summed ? c.take<int>((size_t)T) : nullptr;
     w.summed_indices = own_summed ? c.take<int>((size_t)T) : nullptr;
@@ -167,41 +174,61 @@ __device__ __forceinline__ bool in_mask(int row, int col, const int* offsets, co
     return lo < end && columns[lo] == col;
 }
 
+// Position of the lane's triplet among those of row `key` (-1: none) counted
+// so far in hist: the first lane of every run of equal keys in the wave adds the
+// run's length with one atomic.  Element-ordered triplets repeat a row 4 to 8
+// times; shuffled ones pay one atomic each.
+__device__ __forceinline__ int row_rank(int key, int* hist)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int prev = __shfl_up(key, 1);
+    const uint64_t heads = __ballot(lane == 0 || prev != key);
+    const uint64_t upto = heads & (~uint64_t(0) >> (kWave - 1 - lane));
+    const int first = kWave - 1 - __clzll((long long)upto);
+    const uint64_t after = first < kWave - 1 ? heads >> (first + 1) : 0;
+    const int len = after ? __ffsll((long long)after) : kWave - first;
+    int base = 0;
+    if (lane == first && key >= 0)
+        base = atomicAdd(&hist[key], len);
+    return __shfl(base, first) + lane - first;
+}
+
 template <typename U>
 __global__ __launch_bounds__(kBlock) void classify_kernel(
     int T, const int* tpl_count, int nrow, int ncol, const int* rows, const int* cols, const U* values,
     int block_size, U zero_mask, const int* mask_offsets, const int* mask_row_counts, const int* mask_columns,
-    int* trow, int* hist
+    int* trow, int* hist, int* rank
 )
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= T)
-        return;
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const bool in = i < T;
     const int limit = tpl_count ? *tpl_count : T;
-    const int r = rows[i];
-    const int c = cols[i];
+    const int r = in ? rows[i] : -1;
+    const int c = in ? cols[i] : -1;
+    const U v0 = in && values ? values[(size_t)i * block_size] : U(0);
     bool valid = i < limit && r >= 0 && r < nrow && c >= 0 && c < ncol;
     if (valid && mask_offsets)
         valid = in_mask(r, c, mask_offsets, mask_row_counts, mask_columns);
-    if (valid && values)
+    if (valid && values && (v0 & zero_mask) == U(0))
         valid = !block_is_zero(values + (size_t)i * block_size, block_size, zero_mask);
-    trow[i] = valid ? r : -1;
-    if (valid)
-        atomicAdd(&hist[r], 1);
+    const int k = row_rank(valid ? r : -1, hist);
+    if (in) {
+        trow[i] = valid ? r : -1;
+        rank[i] = k;
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void scatter_kernel(
-    int T, const int* trow, const int* cols, const int* row_start, int* hist, uint64_t* keys
+    int T, const int* trow, const int* cols, const int* row_start, const int* rank, uint64_t* keys
 )
 {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= T)
         return;
     const int r = trow[i];
     if (r < 0)
         return;
-    const int pos = row_start[r] + atomicSub(&hist[r], 1) - 1;
-    keys[pos] = ((uint64_t)(uint32_t)cols[i] << 32) | (uint32_t)i;
+    keys[row_start[r] + rank[i]] = ((uint64_t)(uint32_t)cols[i] << 32) | (uint32_t)i;
 }
 
 // Tiled classification (one workgroup per tile): validity as classify_kernel,
@@ -1490,37 +1517,40 @@ int bucket_sort_rows(
         return sort_rows(nrow, RowRanges{w.row_start, nullptr}, w, summed_indices, urow, write_back, stream,
                          /*counters_zeroed=*/true);
     }
-    WA_TRY(launch_fill(w.hist, (int64_t)nrow + 1, 0, stream));
+    // one level: the row histogram (and the list counters after it) from global
+    // atomics, whose results place the keys within their rows
+    WA_TRY(launch_fill(w.hist, (int64_t)(w.counters - w.hist) + kListCounters, 0, stream));
+    int* rank = reinterpret_cast<int*>(w.alt);  // free until the longest rows are sorted
     if (T > 0) {
         const unsigned grid = (unsigned)ceil_div(T, kBlock);
         switch (prune ? scalar_size : 0) {
         case 1:
             classify_kernel<uint8_t><<<grid, kBlock, 0, stream>>>(
                 T, tpl_count, nrow, ncol, rows, cols, (const uint8_t*)tpl_values, block_size, (uint8_t)zero_mask, mo,
-                mrc, mc, w.trow, w.hist
+                mrc, mc, w.trow, w.hist, rank
             );
             break;
         case 2:
             classify_kernel<uint16_t><<<grid, kBlock, 0, stream>>>(
                 T, tpl_count, nrow, ncol, rows, cols, (const uint16_t*)tpl_values, block_size, (uint16_t)zero_mask, mo,
-                mrc, mc, w.trow, w.hist
+                mrc, mc, w.trow, w.hist, rank
             );
             break;
         case 4:
             classify_kernel<uint32_t><<<grid, kBlock, 0, stream>>>(
                 T, tpl_count, nrow, ncol, rows, cols, (const uint32_t*)tpl_values, block_size, (uint32_t)zero_mask, mo,
-                mrc, mc, w.trow, w.hist
+                mrc, mc, w.trow, w.hist, rank
             );
             break;
         case 8:
             classify_kernel<uint64_t><<<grid, kBlock, 0, stream>>>(
                 T, tpl_count, nrow, ncol, rows, cols, (const uint64_t*)tpl_values, block_size, (uint64_t)zero_mask, mo,
-                mrc, mc, w.trow, w.hist
+                mrc, mc, w.trow, w.hist, rank
             );
             break;
         default:
             classify_kernel<uint32_t><<<grid, kBlock, 0, stream>>>(
-                T, tpl_count, nrow, ncol, rows, cols, nullptr, block_size, 0u, mo, mrc, mc, w.trow, w.hist
+                T, tpl_count, nrow, ncol, rows, cols, nullptr, block_size, 0u, mo, mrc, mc, w.trow, w.hist, rank
             );
             break;
         }
@@ -1529,11 +1559,12 @@ int bucket_sort_rows(
     WA_TRY(exclusive_scan_i32(w.hist, w.row_start, nrow, w.scan_ws, stream));
     if (T > 0) {
         scatter_kernel<<<(unsigned)ceil_div(T, kBlock), kBlock, 0, stream>>>(
-            T, w.trow, cols, w.row_start, w.hist, w.keys
+            T, w.trow, cols, w.row_start, rank, w.keys
         );
         WA_LAUNCH_CHECK();
     }
-    return sort_rows(nrow, RowRanges{w.row_start, nullptr}, w, summed_indices, urow, write_back, stream);
+    return sort_rows(nrow, RowRanges{w.row_start, nullptr}, w, summed_indices, urow, write_back, stream,
+                     /*counters_zeroed=*/true);
 }
 
 // Triplets -> compact BSR.  `mo`, `mrc`, `mc` (offsets, row counts, columns of
