@@ -494,3 +494,87 @@ def test_cg_vector_update_and_wave_spmv(device, dtype, n, prec, shift):
         p = z + (rz / old) * p
     rel = float((x.double() - xs).norm() / xs.norm())
     assert rel < (2e-5 if dtype == torch.float32 else 1.3e-11), rel
+
+
+@pytest.mark.parametrize("prec", ["diag", "block_diag", "id"])
+@pytest.mark.parametrize("family,n,dtype", [
+    ("poisson", 3, torch.float32), ("poisson", 24, torch.float32), ("poisson", 200, torch.float32),
+    ("poisson", 90, torch.float64), ("elasticity", 3, torch.float32), ("elasticity", 9, torch.float64),
+    ("elasticity", 17, torch.float32), ("renumbered", 200, torch.float32)])
+def test_cg_one_launch_solve(device, family, n, dtype, prec):
+    """Small systems in one launch (one workgroup up to the most, rows that do
+    not divide, windows that do not fit: a random numbering) against the same
+    solve with a callback, which takes the general kernels: same iteration count
+    (whole groups of check_every, maxiter).  Only the order of the FP64 sums
+    differs.  Over 12 iterations the iterates agree to 1e-5 (FP32 rounds alpha and
+    beta once per iteration: 12 * 6e-8, grown by less than 10) and 1e-12 (FP64:
+    12 * 1e-16 and the same growth leave 1e-14); later ones part as Ritz values
+    converge, so a converged solve is held to the other's true residual."""
+    if family == "elasticity":
+        r, c, v, b, nn = problems.elasticity3d_q1(n, device=device)
+        A = sparse.bsr_zeros(nn, nn, wa.matrix((3, 3), wa.types.type_to_scalar(dtype)), device=device)
+        sparse.bsr_set_from_triplets(A, r, c, v.to(dtype), prune_numerical_zeros=False)
+    else:
+        r, c, v, b, nn = problems.poisson2d_q1(n, 1)
+        r, c, v, b = (torch.from_numpy(t).to(device) for t in (r, c, v, b))
+        if family == "renumbered":
+            perm = torch.randperm(nn, generator=torch.Generator().manual_seed(1)).to(device)
+            keep = (r >= 0) & (c >= 0)
+            r, c, v = perm[r[keep].long()].to(torch.int32), perm[c[keep].long()].to(torch.int32), v[keep]
+            b = torch.empty_like(b).index_copy_(0, perm, b)
+        A = sparse.bsr_zeros(nn, nn, wa.types.type_to_scalar(dtype), device=device)
+        sparse.bsr_set_from_triplets(A, r, c, v.to(dtype))
+    A.nnz_sync()
+    b = b.to(dtype)
+    M = linear.preconditioner(A, prec)
+    for kw in (dict(tol=1e-12, maxiter=12), dict(tol=1e-5, maxiter=600), dict(tol=1e-5, maxiter=600, check_every=7),
+               dict(tol=1e-12, maxiter=37), dict(tol=2.0, maxiter=50)):
+        x0, x1 = torch.full_like(b, 0.01), torch.full_like(b, 0.01)
+        seen = []
+        i0, _, a0 = linear.cg(A, b, x0, atol=0.0, M=M, callback=lambda *a: seen.append(a), **kw)
+        i1, e1, a1 = linear.cg(A, b, x1, atol=0.0, M=M, **kw)
+        assert i0 == i1 and a0 == a1 and len(seen) > 0
+        if kw["maxiter"] == 12:
+            tight = 1e-12 if dtype == torch.float64 else 1e-5
+            assert float((x0 - x1).norm()) <= tight * float(x0.norm())
+        elif e1 <= a1:
+            true = [float((b.double() - sparse.bsr_mv(A, x).double()).norm()) for x in (x0, x1)]
+            assert true[1] <= 2.0 * true[0] + a1  # the same attainable accuracy
+
+
+def test_cg_one_launch_nan_and_concurrent_streams(device):
+    """A right-hand side with a NaN runs to maxiter as the general kernels do, and
+    solves on several streams and threads at once give the serial result."""
+    import threading
+
+    r, c, v, b, nn = problems.poisson2d_q1(96, 1)
+    A = sparse.bsr_zeros(nn, nn, wa.float32, device=device)
+    sparse.bsr_set_from_triplets(A, *(torch.from_numpy(t).to(device) for t in (r, c, v)))
+    A.nnz_sync()
+    M = linear.preconditioner(A, "diag")
+    bt = torch.from_numpy(b).to(device)
+    bad = bt.clone()
+    bad[5] = float("nan")
+    it, err, _ = linear.cg(A, bad, torch.zeros_like(bt), tol=1e-5, maxiter=30, M=M)
+    assert it == 30 and math.isnan(err)
+    want = torch.zeros_like(bt)
+    i0, _, _ = linear.cg(A, bt, want, tol=1e-6, maxiter=200, M=M)
+    torch.cuda.synchronize()
+    results = [None] * 4
+
+    def work(k):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(5):
+                x = torch.zeros_like(bt)
+                i, _, _ = linear.cg(A, bt, x, tol=1e-6, maxiter=200, M=M)
+            s.synchronize()
+        results[k] = (i, x)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i, x in results:
+        assert i == i0 and torch.equal(x, want)

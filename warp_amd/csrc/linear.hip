@@ -58,6 +58,11 @@ struct CgState {
     int iter_copy;  // the SpMV's copy of iter (fused direction buffers), read by the update
     int done;       // r.r <= atol^2 for the current iterate
     int done_prev;  // `done` as the update saw it, read by the direction pass
+    // small systems (cg_small_kernel): largest column window and block count of
+    // a workgroup's rows, workgroups that finished
+    int small_window;
+    int small_blocks;
+    int small_done;
 };
 
 enum PrecKind { kPrecNone = 0, kPrecDiag = 1, kPrecBlock = 2 };
@@ -69,6 +74,8 @@ enum PrecKind { kPrecNone = 0, kPrecDiag = 1, kPrecBlock = 2 };
 // kMaxSpmvGrid workgroups, the update and direction passes grid-stride with
 // at most kMaxVecGrid.
 constexpr int kMaxSpmvGrid = 2048;
+constexpr int kSmallMaxGroups = 128;  // workgroups of cg_small_kernel
+constexpr int kSmallReplicas = 8;     // copies of its exchange slots
 constexpr int kMaxVecGrid = 1024;
 
 struct CgWs {
@@ -76,6 +83,7 @@ struct CgWs {
     double* init_partials;  // 3 * max_init_blocks (b.b, r.r, r.z of the initial residual)
     double* spmv_partials;  // kMaxSpmvGrid (p.Ap)
     double* upd_partials;   // 2 * kMaxVecGrid (r.r, r.z)
+    unsigned long long* small_slots;  // exchange slots of cg_small_kernel
     int max_init_blocks;
     void* r;
     void* z;
@@ -96,6 +104,7 @@ CgWs carve_cg(void* base, size_t bytes, int64_t nrow, int64_t n, size_t scalar_b
     w.init_partials = c.take<double>((size_t)3 * w.max_init_blocks);
     w.spmv_partials = c.take<double>((size_t)kMaxSpmvGrid);
     w.upd_partials = c.take<double>((size_t)2 * kMaxVecGrid);
+    w.small_slots = c.take<unsigned long long>((size_t)kSmallReplicas * 6 * kSmallMaxGroups);
     w.r = c.take<char>((size_t)n * scalar_bytes);
     w.z = c.take<char>((size_t)n * scalar_bytes);
     w.p = c.take<char>((size_t)n * scalar_bytes);
@@ -635,6 +644,382 @@ __global__ void cg_state_init_kernel(CgWs ws, double rtol, double atol)
     state->done_prev = 0;
     state->iter = 0;
     state->iter_copy = 0;
+    state->small_window = 0;
+    state->small_blocks = 0;
+    state->small_done = 0;
+}
+
+// ---------------------------------------------------------------------------
+// Small systems: all iterations of a solve in one launch
+// ---------------------------------------------------------------------------
+//
+// What bounds a small solve is the latency of two kernels per iteration (2D
+// Poisson, 16 K unknowns: 6.1 + 3.8 us and two gaps for 1.2 MB of data).  Here
+// N workgroups stay for the whole solve: each keeps its rows' matrix, the p
+// entries of the columns they touch (a window of the numbering), x, r and the
+// preconditioner in LDS and registers, and an iteration is two all-reductions
+// over the workgroups (p.Ap; r.r and r.z) and one exchange of z.  p = z + beta p
+// is evaluated by every workgroup for its whole window, so only z travels.  us
+// per iteration, two kernels (replayed as graphs) / this: 2D Poisson 128^2 11.3 /
+// 6.2, 250^2 12.1 / 8.6, elasticity 12^3 11.1 / 7.1, 7-point 40^3 12.1 / 9.5; what a
+// solve costs besides its iterations 230 / 83 us.  The two all-reductions are
+// most of what is left.
+//
+// All-reduction: each workgroup stores its FP64 partial in its own slot with a
+// device-scope store; one wave of every workgroup polls all slots until none
+// holds the sentinel and adds them in the same order, so all workgroups form
+// bit-identical alpha, beta and `done`.  Slots alternate between two sets by the
+// iteration's parity.  A workgroup clears its slots of the other set right after
+// the p.Ap reduction: there every workgroup has arrived, hence has read that set
+// for the last time, and the clear is ordered before the workgroup's r.r / r.z
+// partials by the release fence, hence before anyone polls that set again.  z is
+// overwritten only after the p.Ap reduction, by when all have read the old one.
+//
+// The launch is cooperative (all workgroups resident), and every wait is
+// bounded: a workgroup that polls kSmallSpins times leaves without finishing, x
+// is only written by cg_small_commit_kernel once all have finished, and the host
+// then solves by the kernels above.
+constexpr int kSmallThreads = 512;
+constexpr int kSmallPer = 2;       // scalars per thread
+constexpr int kSmallLds = 144 * 1024;
+constexpr int kSmallSpins = 1 << 21;
+constexpr unsigned long long kSlotEmpty = 0x7ff8dead00c0ffeeull;  // a NaN no sum stores
+
+// Slot set of quantity q (0 p.Ap, 1 r.r, 2 r.z) and parity.  Every partial is
+// stored in kSmallReplicas copies and workgroup w polls copy w % kSmallReplicas:
+// polls of one line by every workgroup queue at its memory channel.
+__device__ __forceinline__ unsigned long long* small_slots(const CgWs& ws, int replica, int q, int parity)
+{
+    return ws.small_slots + ((size_t)replica * 6 + q * 2 + parity) * kSmallMaxGroups;
+}
+
+// A sum's bits, any NaN as one NaN (never the sentinel).
+__device__ __forceinline__ unsigned long long slot_bits(double v)
+{
+    return v == v ? (unsigned long long)__double_as_longlong(v) : 0x7ff8000000000000ull;
+}
+
+// Column window and block count of each workgroup's rows (their maxima go to the
+// state, for the LDS the solve needs), and empty slots.
+__global__ __launch_bounds__(kBlock) void cg_small_plan_kernel(int nrow, int rows, const int* __restrict__ offsets,
+                                                              const int* __restrict__ columns, CgWs ws)
+{
+    __shared__ int s_lo, s_hi;
+    const int w = blockIdx.x;
+    if (threadIdx.x < 6 * kSmallReplicas)
+        small_slots(ws, threadIdx.x / 6, threadIdx.x % 6 / 2, threadIdx.x % 2)[w] = kSlotEmpty;
+    const int r0 = min(w * rows, nrow), r1 = min(r0 + rows, nrow);
+    if (threadIdx.x == 0) {
+        s_lo = r0;
+        s_hi = r1;
+    }
+    __syncthreads();
+    const int b0 = offsets[r0], b1 = offsets[r1];
+    int lo = r0, hi = r1;
+    for (int b = b0 + threadIdx.x; b < b1; b += kBlock) {
+        const int c = columns[b];
+        lo = min(lo, c);
+        hi = max(hi, c + 1);
+    }
+    atomicMin(&s_lo, lo);
+    atomicMax(&s_hi, hi);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        // columns outside the matrix: no window fits (the general kernels take the system as before)
+        const bool bad = s_lo < 0 || s_hi > nrow;
+        atomicMax(&ws.state->small_window, bad ? 0x7fffffff : s_hi - s_lo);
+        atomicMax(&ws.state->small_blocks, b1 - b0);
+    }
+}
+
+// Dynamic LDS of cg_small_kernel, in bytes: offsets, columns, values, p window,
+// Ap, r, reductions.
+template <typename S, int BR> struct SmallLds {
+    size_t off, col, val, p, ap, r, red, bytes;
+    __host__ __device__ SmallLds(int rows, int blocks, int window)
+    {
+        size_t at = 0;
+        const auto take = [&](size_t n) {
+            const size_t here = at;
+            at += (n + 15) / 16 * 16;
+            return here;
+        };
+        off = take(sizeof(int) * (size_t)(rows + 1));
+        col = take(sizeof(int) * (size_t)(blocks + 1));
+        val = take(sizeof(S) * (size_t)(blocks + 1) * BR * BR);
+        p = take(sizeof(S) * (size_t)window * BR);
+        ap = take(sizeof(S) * (size_t)rows * BR);
+        r = take(sizeof(S) * (size_t)rows * BR);
+        red = take(sizeof(double) * 2 * (kSmallThreads / kWave + 1));
+        bytes = at;
+    }
+};
+
+// Sum of each of NV values over all threads of all `n` workgroups, bit-identical
+// everywhere; false where a wait ran out.  ORDER: what the workgroup has stored
+// for others is visible to them once they return.
+template <int NV, bool ORDER>
+__device__ __forceinline__ bool small_all_reduce(double (&v)[NV], int q0, int parity, int n, const CgWs& ws, double* red)
+{
+    constexpr int kWaves = kSmallThreads / kWave;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        v[q] = wave_sum(v[q]);
+        if (lane == 0)
+            red[q * kWaves + wave] = v[q];
+    }
+    if (ORDER)
+        __builtin_amdgcn_s_waitcnt(0);  // this wave's exchanged stores have arrived
+    __syncthreads();
+    bool ok = true;
+    if (wave == 0) {
+#pragma unroll
+        for (int q = 0; q < NV; ++q) {
+            double t = 0.0;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w)
+                t += red[q * kWaves + w];
+            v[q] = t;
+        }
+        if (n > 1) {
+            if (ORDER)
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            if (lane < kSmallReplicas) {
+#pragma unroll
+                for (int q = 0; q < NV; ++q)
+                    store_agent(small_slots(ws, lane, q0 + q, parity) + blockIdx.x, slot_bits(v[q]));
+            }
+            const int replica = (int)blockIdx.x % kSmallReplicas;
+            constexpr int kPer = kSmallMaxGroups / kWave;
+            unsigned long long got[NV][kPer];
+            int spins = 0;
+            for (;;) {
+                bool ready = true;
+#pragma unroll
+                for (int q = 0; q < NV; ++q)
+#pragma unroll
+                    for (int u = 0; u < kPer; ++u) {
+                        const int w = lane + u * kWave;
+                        got[q][u] = w < n ? load_agent(small_slots(ws, replica, q0 + q, parity) + w) : 0ull;
+                        ready = ready && got[q][u] != kSlotEmpty;
+                    }
+                if (__all(ready))
+                    break;
+                if (++spins >= kSmallSpins) {
+                    ok = false;
+                    break;
+                }
+            }
+            if (ORDER)
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll
+            for (int q = 0; q < NV; ++q) {
+                double t = 0.0;
+#pragma unroll
+                for (int u = 0; u < kPer; ++u)
+                    t += lane + u * kWave < n ? __longlong_as_double((long long)got[q][u]) : 0.0;
+                v[q] = wave_sum(t);
+            }
+        }
+        if (lane == 0) {
+#pragma unroll
+            for (int q = 0; q < NV; ++q)
+                red[NV * kWaves + q] = __longlong_as_double((long long)(ok ? slot_bits(v[q]) : kSlotEmpty));
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        v[q] = red[NV * kWaves + q];
+        ok = (unsigned long long)__double_as_longlong(v[q]) != kSlotEmpty;
+    }
+    __syncthreads();
+    return ok;
+}
+
+template <typename S, int BR, int G, int PREC>
+__global__ __launch_bounds__(kSmallThreads) void cg_small_kernel(
+    int nrow, int rows, int max_blocks, int max_window, int maxiter, const int* __restrict__ offsets,
+    const int* __restrict__ columns, const S* __restrict__ values, const S* __restrict__ prec,
+    const S* __restrict__ x_in, CgWs ws
+)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char small_smem[];
+    const SmallLds<S, BR> lay(rows, max_blocks, max_window);
+    int* l_off = reinterpret_cast<int*>(small_smem + lay.off);
+    int* l_col = reinterpret_cast<int*>(small_smem + lay.col);
+    S* l_val = reinterpret_cast<S*>(small_smem + lay.val);
+    S* l_p = reinterpret_cast<S*>(small_smem + lay.p);
+    S* l_ap = reinterpret_cast<S*>(small_smem + lay.ap);
+    S* l_r = reinterpret_cast<S*>(small_smem + lay.r);
+    double* red = reinterpret_cast<double*>(small_smem + lay.red);
+    const int n = (int)gridDim.x, w = (int)blockIdx.x, tid = (int)threadIdx.x;
+    const int r0 = min(w * rows, nrow), r1 = min(r0 + rows, nrow), mine = r1 - r0;
+    const int b0 = offsets[r0], nb = offsets[r1] - b0;
+    S* zx = static_cast<S*>(ws.p2);  // z, exchanged
+
+    // the window of columns
+    int lo = r0, hi = r1;
+    for (int b = tid; b < nb; b += kSmallThreads) {
+        const int c = columns[b0 + b];
+        l_col[b] = c;
+        lo = min(lo, c);
+        hi = max(hi, c + 1);
+    }
+    int* span = reinterpret_cast<int*>(red);
+    if (tid == 0) {
+        span[0] = r0;
+        span[1] = r1;
+        l_off[0] = 0;
+        if (nb == 0) {  // inactive slots of the product read block 0
+            l_col[0] = r0;
+            for (int e = 0; e < BR * BR; ++e)
+                l_val[e] = S(0);
+        }
+    }
+    __syncthreads();
+    atomicMin(&span[0], lo);
+    atomicMax(&span[1], hi);
+    for (int i = tid; i < mine; i += kSmallThreads)
+        l_off[i + 1] = offsets[r0 + i + 1] - b0;
+    for (int i = tid; i < nb * BR * BR; i += kSmallThreads)
+        l_val[i] = values[(size_t)b0 * BR * BR + i];
+    __syncthreads();
+    lo = span[0];
+    const int window = (span[1] - lo) * BR;
+    for (int b = tid; b < max(nb, 1); b += kSmallThreads)
+        l_col[b] -= lo;
+    const S* p_in = static_cast<const S*>(ws.p);
+    for (int i = tid; i < window; i += kSmallThreads)
+        l_p[i] = p_in[(size_t)lo * BR + i];
+
+    // own scalars i = tid + u * kSmallThreads of rows r0 .. r1 - 1
+    const int own = mine * BR;
+    const S* r_in = static_cast<const S*>(ws.r);
+    S x[kSmallPer], r[kSmallPer], m[kSmallPer][PREC == kPrecBlock ? BR : 1];
+#pragma unroll
+    for (int u = 0; u < kSmallPer; ++u) {
+        const int i = tid + u * kSmallThreads;
+        const size_t g = (size_t)r0 * BR + i;
+        x[u] = i < own ? x_in[g] : S(0);
+        r[u] = i < own ? r_in[g] : S(0);
+        if (PREC == kPrecDiag)
+            m[u][0] = i < own ? prec[g] : S(0);
+        if constexpr (PREC == kPrecBlock)
+#pragma unroll
+            for (int c = 0; c < BR; ++c)
+                m[u][c] = i < own ? prec[g * BR + c] : S(0);
+    }
+    const double atol_sq = ws.state->atol_sq;
+    double rr = ws.state->rr, rz = ws.state->rz, alpha = 0.0, beta = 0.0, pap = 0.0;
+    const S* l_pown = l_p + (size_t)(r0 - lo) * BR;
+    int it = 0;
+    bool ok = true;
+    __syncthreads();
+    while (rr > atol_sq && it < maxiter) {
+        const int parity = it & 1;
+        // Ap
+        constexpr int RPG = rows_per_group_for(BR, BR);
+        for (int row = tid / G * RPG; row < mine; row += kSmallThreads / G * RPG) {
+            const RowAcc<S, BR * RPG> a = group_rows_product_f<S, BR, BR, G, RPG, S>(
+                row, mine, tid % G, l_off, nullptr, l_col, l_val, LoadX<S>{l_p});
+            for (int e = tid % G; e < BR * RPG && row + e / BR < mine; e += G)
+                l_ap[row * BR + e] = pick(a, e);
+        }
+        __syncthreads();
+        double s1[1] = {0.0};
+#pragma unroll
+        for (int u = 0; u < kSmallPer; ++u) {
+            const int i = tid + u * kSmallThreads;
+            if (i < own)
+                s1[0] += (double)l_pown[i] * (double)l_ap[i];
+        }
+        ok = small_all_reduce<1, false>(s1, 0, parity, n, ws, red);
+        if (!ok)
+            return;
+        if (tid < 3 * kSmallReplicas && n > 1)  // everyone has read the other set for the last time
+            store_agent(small_slots(ws, tid / 3, tid % 3, parity ^ 1) + w, kSlotEmpty);
+        pap = s1[0];
+        alpha = rz / pap;
+        const S al = (S)alpha;
+#pragma unroll
+        for (int u = 0; u < kSmallPer; ++u) {
+            const int i = tid + u * kSmallThreads;
+            if (i < own) {
+                x[u] = fma(al, l_pown[i], x[u]);
+                r[u] = fma(-al, l_ap[i], r[u]);
+                if constexpr (PREC == kPrecBlock)
+                    l_r[i] = r[u];
+            }
+        }
+        if constexpr (PREC == kPrecBlock)
+            __syncthreads();
+        double s2[2] = {0.0, 0.0};
+#pragma unroll
+        for (int u = 0; u < kSmallPer; ++u) {
+            const int i = tid + u * kSmallThreads;
+            if (i < own) {
+                S z = r[u];
+                if (PREC == kPrecDiag)
+                    z = m[u][0] * r[u];
+                if constexpr (PREC == kPrecBlock) {
+                    z = S(0);
+#pragma unroll
+                    for (int c = 0; c < BR; ++c)
+                        z = fma(m[u][c], l_r[i - i % BR + c], z);
+                }
+                store_agent(zx + (size_t)r0 * BR + i, z);
+                s2[0] += (double)r[u] * (double)r[u];
+                s2[1] += (double)r[u] * (double)z;
+            }
+        }
+        ok = small_all_reduce<2, true>(s2, 1, parity, n, ws, red);
+        if (!ok)
+            return;
+        rr = s2[0];
+        ++it;
+        if (!(rr > atol_sq) || it >= maxiter) {
+            rz = s2[1];
+            break;
+        }
+        beta = s2[1] / rz;
+        rz = s2[1];
+        const S be = (S)beta;
+        for (int i = tid; i < window; i += kSmallThreads)
+            l_p[i] = fma(be, l_p[i], load_agent(zx + (size_t)lo * BR + i));
+        __syncthreads();
+    }
+    S* out = static_cast<S*>(ws.Ap);
+#pragma unroll
+    for (int u = 0; u < kSmallPer; ++u) {
+        const int i = tid + u * kSmallThreads;
+        if (i < own)
+            out[(size_t)r0 * BR + i] = x[u];
+    }
+    if (tid == 0) {
+        if (w == 0) {
+            CgState* state = ws.state;
+            state->rr = rr;
+            state->rz = rz;
+            state->alpha = alpha;
+            state->beta = beta;
+            state->pAp = pap;
+            state->iter = it;
+            state->iter_copy = it;
+            state->done = !(rr > atol_sq);
+        }
+        atomicAdd(&ws.state->small_done, 1);
+    }
+}
+
+// x = the solution, if every workgroup of cg_small_kernel finished
+template <typename S>
+__global__ __launch_bounds__(kBlock) void cg_small_commit_kernel(int n, int groups, S* __restrict__ x, CgWs ws)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < n && ws.state->small_done == groups)
+        x[i] = static_cast<const S*>(ws.Ap)[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -1041,6 +1426,102 @@ struct CycleRunner {
     }
 };
 
+// Number of workgroups of cg_small_kernel for a system (a power of two; 0: not
+// small): 32 KB of matrix each until there are 128, then up to 96 KB.  us per
+// iteration at 24 / 32 / 48 KB: 2D Poisson 128^2 6.20 / 6.18 / 6.76, 64^2 5.4 / 5.4 /
+// 6.2, 12^3 elasticity 7.9 / 7.1 / 7.2; 128 workgroups against 256: 2D Poisson
+// 250^2 8.6 / 10.8, 18^3 elasticity 9.7 / 11.6 (the all-reductions grow with their
+// number).
+template <typename S> int small_groups(const CgProblem& pb)
+{
+    const int64_t n = (int64_t)pb.nrow * pb.br;
+    const int64_t matrix = pb.nnz_hint * (int64_t)(sizeof(int) + pb.br * pb.br * sizeof(S));
+    if (n * (int64_t)sizeof(S) > (int64_t)kFusedDirectionMaxBytes || matrix > (int64_t)kSmallMaxGroups * 96 * 1024)
+        return 0;
+    int g = 1;
+    while (g < kSmallMaxGroups && ((int64_t)g * 32 * 1024 < matrix || (int64_t)g * kSmallThreads < n))
+        g *= 2;
+    return ceil_div(pb.nrow, g) * pb.br <= kSmallThreads * kSmallPer ? g : 0;
+}
+
+template <typename S> const void* small_kernel(int br, int lanes, int prec)
+{
+#define WA_SMALL_PREC(BR, G)                                                                                          \
+    if (br == BR && lanes == G) {                                                                                     \
+        if (prec == kPrecNone)                                                                                        \
+            return (const void*)cg_small_kernel<S, BR, G, kPrecNone>;                                                 \
+        if (prec == kPrecDiag || BR == 1) /* a 1x1 block is a point */                                                \
+            return (const void*)cg_small_kernel<S, BR, G, kPrecDiag>;                                                 \
+        return (const void*)cg_small_kernel<S, BR, G, BR == 1 ? kPrecDiag : kPrecBlock>;                              \
+    }
+    WA_SMALL_PREC(1, 2)
+    WA_SMALL_PREC(1, 4)
+    WA_SMALL_PREC(1, 8)
+    WA_SMALL_PREC(1, 16)
+    WA_SMALL_PREC(3, 8)
+    WA_SMALL_PREC(3, 16)
+    WA_SMALL_PREC(3, 32)
+#undef WA_SMALL_PREC
+    return nullptr;
+}
+
+// Solves by cg_small_kernel where the system fits; *solved = 0 with x untouched
+// otherwise.  The caller's stream is not capturing (the state is read back).
+template <typename S>
+int cg_solve_small(CgLauncher<S>& L, double rtol, double atol, int maxiter, int check_every, CgState* h, int* cur_iter,
+                   int* solved)
+{
+    *solved = 0;
+    const CgProblem& pb = L.pb;
+    const int groups = small_groups<S>(pb);
+    const void* kernel = groups ? small_kernel<S>(pb.br, L.g(), pb.prec_kind) : nullptr;
+    if (!kernel)
+        return kOk;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(L.stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return kOk;
+    }
+    int rows = (int)ceil_div(pb.nrow, groups);
+    cg_state_init_kernel<<<1, 1, 0, L.stream>>>(L.ws, rtol, atol);
+    WA_LAUNCH_CHECK();
+    WA_TRY(L.init(1));
+    cg_small_plan_kernel<<<groups, kBlock, 0, L.stream>>>(pb.nrow, rows, pb.offsets, pb.columns, L.ws);
+    WA_LAUNCH_CHECK();
+    WA_TRY(read_state(L.ws.state, h, L.stream));
+    *cur_iter = 0;
+    if (h->rr <= h->atol_sq) {
+        *solved = 1;
+        return kOk;
+    }
+    if (h->small_window > kSmallLds / (int)sizeof(S))
+        return kOk;
+    const size_t lds = pb.br == 1 ? SmallLds<S, 1>(rows, h->small_blocks, h->small_window).bytes
+                                  : SmallLds<S, 3>(rows, h->small_blocks, h->small_window).bytes;
+    if (lds > (size_t)kSmallLds)
+        return kOk;
+    const int n = pb.nrow * pb.br;
+    int nrow = pb.nrow, blocks = h->small_blocks, window = h->small_window;
+    const S *values = (const S*)pb.values, *prec = (const S*)pb.prec, *x = (const S*)pb.x;
+    const int *offsets = pb.offsets, *columns = pb.columns;
+    void* args[] = {&nrow, &rows, &blocks, &window, &maxiter, &offsets, &columns, &values, &prec, &x, &L.ws};
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLds) != hipSuccess ||
+        hipLaunchCooperativeKernel(kernel, dim3((unsigned)groups), dim3(kSmallThreads), args, (unsigned)lds, L.stream) !=
+        hipSuccess) {
+        (void)hipGetLastError();  // does not fit this device: the general kernels
+        return kOk;
+    }
+    cg_small_commit_kernel<S><<<(unsigned)ceil_div(n, kBlock), kBlock, 0, L.stream>>>(n, groups, (S*)pb.x, L.ws);
+    WA_LAUNCH_CHECK();
+    WA_TRY(read_state(L.ws.state, h, L.stream));
+    if (h->small_done != groups)
+        return kOk;
+    // as the host loop counts: whole groups of check_every, and to the end on NaN
+    *cur_iter = h->rr <= h->atol_sq ? (int)std::min<int64_t>(maxiter, ceil_div(h->iter, check_every) * check_every) : maxiter;
+    *solved = 1;
+    return kOk;
+}
+
 template <typename S>
 int cg_solve_impl(
     const CgProblem& pb, double tol, double atol, int maxiter, int check_every, int restart, int use_graph,
@@ -1061,6 +1542,25 @@ int cg_solve_impl(
     WA_REQUIRE((uintptr_t)workspace % 16 == 0, "cg_solve: workspace must be 16-byte aligned");
     if (maxiter <= 0)
         maxiter = (int)n;
+
+    if (check_every > 0 && restart <= 0 && !cb) {
+        double rtol_v, atol_v;
+        get_tolerances(sizeof(S) == 8, tol, atol, &rtol_v, &atol_v);
+        CgLauncher<S> small{pb, ws, caller_stream};
+        small.fused = true;
+        CgState h;
+        int cur_iter = 0, solved = 0;
+        WA_TRY(cg_solve_small(small, rtol_v, atol_v, maxiter, check_every, &h, &cur_iter, &solved));
+        if (solved) {
+            if (iters_out)
+                *iters_out = cur_iter;
+            if (rnorm_out)
+                *rnorm_out = std::sqrt(h.rr);
+            if (atol_out)
+                *atol_out = std::sqrt(h.atol_sq);
+            return kOk;
+        }
+    }
 
     // graphs only where launches bound the iteration: measured on MI355X,
     // replaying the cycles between two checks as one graph gave 2D Poisson
