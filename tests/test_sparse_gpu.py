@@ -1617,3 +1617,31 @@ def test_single_level_assembly_vs_unique(device, nrow, order):
     assert torch.equal(A.offsets.cpu().long(), off)
     assert torch.equal(A.columns[:nnz].cpu().long(), key % nrow)
     assert torch.equal(A.values[:nnz].cpu(), want)
+
+
+@pytest.mark.parametrize("bs,dtype,wdtype", [(3, torch.float32, wa.float32), (2, torch.float64, wa.float64)])
+def test_assembly_of_values_beyond_the_caches(device, bs, dtype, wdtype):
+    """More than 256 MB of values (classified past the caches), sub-tiles and
+    chunks with remainders: zero blocks of both signs are pruned, blocks whose
+    only nonzero is the last scalar are kept, invalid rows dropped; whole
+    numbers, so the sums are exact in any order."""
+    size = bs * bs * (4 if dtype == torch.float32 else 8)
+    T = (256 << 20) // size + 1013
+    nrow = T // 60
+    g = torch.Generator(device=device).manual_seed(bs)
+    rows = torch.randint(-1, nrow + 1, (T,), generator=g, device=device)
+    cols = (rows + torch.randint(0, 30, (T,), generator=g, device=device)).clamp(0, nrow - 1)
+    vals = torch.randint(-3, 4, (T, bs, bs), generator=g, device=device).to(dtype)
+    vals[::5] = 0.0
+    vals[1::10] = -0.0
+    vals[5::20, -1, -1] = 1.0
+    A = sparse.bsr_zeros(nrow, nrow, wa.matrix((bs, bs), wdtype), device=device)
+    sparse.bsr_set_from_triplets(A, rows.to(torch.int32), cols.to(torch.int32), vals)
+    nnz = A.nnz_sync()
+    keep = (rows >= 0) & (rows < nrow) & (vals != 0).flatten(1).any(1)
+    key, inv = torch.unique(rows[keep] * nrow + cols[keep], sorted=True, return_inverse=True)
+    want = torch.zeros((key.numel(), bs, bs), dtype=dtype, device=device).index_add(0, inv, vals[keep])
+    assert nnz == key.numel()
+    assert torch.equal(A.columns[:nnz].long(), key % nrow)
+    assert torch.equal(A.offsets[1:].long(), torch.cumsum(torch.bincount(key // nrow, minlength=nrow), 0))
+    assert torch.equal(A.values[:nnz].view(nnz, bs, bs), want)
