@@ -119,8 +119,13 @@ enum OutFlags {
     kOutPool = 2,
     kOutF32 = 4,
     kOutAccumulate = 8,
-    kOutF32x4 = 16,  // with kOutF32: yf takes 16-byte stores (set by launch_conv from yf's alignment)
 };
+// The form of the output, compiled in (launch_conv): BF16, FP32 in 16-byte
+// stores, FP32 at any alignment.  As run-time flags the FP32 branches
+// lengthen the BF16 epilogue: layers of the 128^3 forward pass, flags
+// / compiled in, us: 32 -> 16 19.2 / 17.8, 64 -> 32 16.6 / 15.7, 16 -> 32 15.9 /
+// 15.2, 32 -> 64 13.4 / 12.8, 2 -> 16 27.9 / 27.3.
+enum OutForm { kFormBf16 = 0, kFormF32x4 = 1, kFormF32 = 2 };
 
 // Persistent tile loops: workgroup b is dispatched to XCD b % kXcds (the
 // MI355X command processor deals workgroups to its 8 XCDs round-robin), so
@@ -248,7 +253,7 @@ template <int CI, int IN> struct HaloStage {
 // as the compiler chooses (a bound of 3 on the 16 -> 32 layer measured the same).
 template <int CI, int CO> constexpr int conv_min_waves() { return (CI == 2 && CO == 16) ? 6 : 1; }
 
-template <int CI, int CO, int IN, int CBG>
+template <int CI, int CO, int IN, int CBG, int FORM>
 __global__ __launch_bounds__(kBlock, (conv_min_waves<CI, CO>())) void conv3_mfma_kernel(
     int m, const unsigned short* __restrict__ x, const unsigned short* __restrict__ coarse,
     const bf16x8* __restrict__ wsw, const float* __restrict__ bias, int flags, unsigned short* __restrict__ y,
@@ -408,14 +413,14 @@ __global__ __launch_bounds__(kBlock, (conv_min_waves<CI, CO>())) void conv3_mfma
                 if (relu)
                     val[i] = fmaxf(val[i], 0.0f);
             }
-            if (CO % 16 == 0 && (flags & kOutF32x4)) {
+            if constexpr (FORM == kFormF32x4) {
                 // the lane's four channels in one 16-byte store: the 1 -> 16 layer at
                 // 128^3 (134 MB written) 70 -> 27 us against four 4-byte stores, which
                 // remain for an output that is not 16-byte aligned
                 f32x4* d = reinterpret_cast<f32x4*>(yf + v * CO + o0);
                 const f32x4 o = {val[0], val[1], val[2], val[3]};
                 *d = (flags & kOutAccumulate) ? *d + o : o;
-            } else if (flags & kOutF32) {
+            } else if constexpr (FORM == kFormF32) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     if (o0 + i < CO) {
@@ -427,14 +432,14 @@ __global__ __launch_bounds__(kBlock, (conv_min_waves<CI, CO>())) void conv3_mfma
 #pragma unroll
                 for (int i = 0; i < 4; ++i)  // pool what was stored
                     val[i] = bf2f((unsigned short)(st[i / 2] >> (16 * (i % 2))));
-                if constexpr (CO % 16 == 0)
-                    *reinterpret_cast<bf16x4*>(y + v * CO + o0) = __builtin_bit_cast(bf16x4, st);
+                static_assert(FORM != kFormBf16 || CO % 16 == 0, "BF16 outputs store four channels at once");
+                *reinterpret_cast<bf16x4*>(y + v * CO + o0) = __builtin_bit_cast(bf16x4, st);
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 psum[g / 2][i] = (g % 2) ? psum[g / 2][i] + val[i] : val[i];
         }
-        if (flags & kOutPool) {
+        if (FORM == kFormBf16 && (flags & kOutPool)) {
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 float sv[4];
@@ -664,12 +669,12 @@ int launch_co1(int m, int in_mode, const unsigned short* x, const unsigned short
     return kOk;
 }
 
-template <int CI, int CO, int IN, int CBG>
+template <int CI, int CO, int IN, int CBG, int FORM>
 void launch_conv_groups(int m, int tiles, const unsigned short* x, const unsigned short* coarse, const bf16x8* w,
                         const float* bias, int flags, unsigned short* y, float* yf, unsigned short* pooled,
                         hipStream_t s)
 {
-    constexpr auto kernel = conv3_mfma_kernel<CI, CO, IN, CBG>;
+    constexpr auto kernel = conv3_mfma_kernel<CI, CO, IN, CBG, FORM>;
     constexpr int nsplit = c_blocks(CO) / CBG;
     static const int per_cu = [] {
         int nb = 0;
@@ -687,7 +692,7 @@ void launch_conv_groups(int m, int tiles, const unsigned short* x, const unsigne
     kernel<<<(unsigned)grid, kBlock, 0, s>>>(m, x, coarse, w, bias, flags, y, yf, pooled);
 }
 
-template <int CI, int CO, int IN>
+template <int CI, int CO, int IN, int FORM>
 void launch_conv_mode(int m, const unsigned short* x, const unsigned short* coarse, const bf16x8* w,
                       const float* bias, int flags, unsigned short* y, float* yf, unsigned short* pooled, hipStream_t s)
 {
@@ -699,11 +704,11 @@ void launch_conv_mode(int m, const unsigned short* x, const unsigned short* coar
     constexpr bool kCanGroup = CB > 1 && ConvLds<CI, CB>::kBytes <= 160 * 1024;
     if constexpr (kCanGroup) {
         if (tiles >= 1024) {
-            launch_conv_groups<CI, CO, IN, CB>(m, tiles, x, coarse, w, bias, flags, y, yf, pooled, s);
+            launch_conv_groups<CI, CO, IN, CB, FORM>(m, tiles, x, coarse, w, bias, flags, y, yf, pooled, s);
             return;
         }
     }
-    launch_conv_groups<CI, CO, IN, 1>(m, tiles, x, coarse, w, bias, flags, y, yf, pooled, s);
+    launch_conv_groups<CI, CO, IN, 1, FORM>(m, tiles, x, coarse, w, bias, flags, y, yf, pooled, s);
 }
 
 template <int CI, int CO>
@@ -711,14 +716,24 @@ int launch_conv(int m, int in_mode, const unsigned short* x, const unsigned shor
                 const float* bias, int flags, unsigned short* y, float* yf, unsigned short* pooled, hipStream_t s)
 {
     const bf16x8* w = static_cast<const bf16x8*>(wsw);
-    flags &= kOutRelu | kOutPool | kOutF32 | kOutAccumulate;
-    if (CO % 16 == 0 && (flags & kOutF32) && (uintptr_t)yf % 16 == 0)
-        flags |= kOutF32x4;
-    if (in_mode == kInUpAdd) {
-        if constexpr (CI > 2)
-            launch_conv_mode<CI, CO, kInUpAdd>(m, x, coarse, w, bias, flags, y, yf, pooled, s);
+    const auto launch = [&](auto form) {
+        constexpr int FORM = decltype(form)::value;
+        if (in_mode == kInUpAdd) {
+            if constexpr (CI > 2)
+                launch_conv_mode<CI, CO, kInUpAdd, FORM>(m, x, coarse, w, bias, flags, y, yf, pooled, s);
+        } else {
+            launch_conv_mode<CI, CO, kInPlain, FORM>(m, x, coarse, w, bias, flags, y, yf, pooled, s);
+        }
+    };
+    if constexpr (CO % 16 == 0) {
+        if (!(flags & kOutF32))
+            launch(std::integral_constant<int, kFormBf16>());
+        else if ((uintptr_t)yf % 16 == 0)
+            launch(std::integral_constant<int, kFormF32x4>());
+        else
+            launch(std::integral_constant<int, kFormF32>());
     } else {
-        launch_conv_mode<CI, CO, kInPlain>(m, x, coarse, w, bias, flags, y, yf, pooled, s);
+        launch(std::integral_constant<int, kFormF32>());
     }
     WA_LAUNCH_CHECK();
     return kOk;
