@@ -1645,3 +1645,8 @@ def test_assembly_of_values_beyond_the_caches(device, bs, dtype, wdtype):
     assert torch.equal(A.columns[:nnz].long(), key % nrow)
     assert torch.equal(A.offsets[1:].long(), torch.cumsum(torch.bincount(key // nrow, minlength=nrow), 0))
     assert torch.equal(A.values[:nnz].view(nnz, bs, bs), want)
+
+
+def test_triplets_row_size_classes_scalar_f64(device, oracle_mod):
+    """FP64 scalars (block size compiled in) over the same row lengths."""
+    test_triplets_row_size_classes(device, oracle_mod, (), np.float64)
