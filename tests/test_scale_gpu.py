@@ -247,3 +247,39 @@ def test_cg_wide_spmv_grid_vs_oracle(device, oracle_mod):
     assert it == it_o == iters
     assert abs(err - err_o) <= 1e-3 * err_o
     assert dx <= 1e-4
+
+
+def test_offsets_up_to_the_largest_int(device):
+    """2^31 - 1 entries (five a row, seven in the last): the wave tiles of the
+    product and the in-place projection step past the last entry without leaving
+    the arrays.  The entries ahead of the last rows are ones of column 0 and x is
+    whole numbers there, so every sum is exact."""
+    from warp_amd.fem import dirichlet
+
+    nrow, nnz = (2**31 - 3) // 5, 2**31 - 1
+    A = sparse.bsr_zeros(nrow, nrow, wa.float32, device=device)
+    off = torch.arange(0, nnz, 5, dtype=torch.int32, device=device)
+    assert off.numel() == nrow + 1
+    off[-1] = nnz
+    A.offsets, A.nnz = off, nnz
+    A.columns = torch.zeros(nnz, dtype=torch.int32, device=device)
+    A.values = torch.ones(nnz, dtype=torch.float32, device=device)
+    tail = torch.tensor([0, 1, 2, 3, 4, 5, nrow - 1], dtype=torch.int32, device=device)
+    A.columns[-7:] = tail
+    A.values[-7:] = torch.arange(2.0, 9.0, device=device)
+    x = torch.zeros(nrow, dtype=torch.float32, device=device)
+    x[:6] = torch.arange(1.0, 7.0, device=device)
+    x[-1] = 10.0
+    last = float((A.values[-7:] * x[tail.long()]).sum())
+    for _ in range(2):  # both traversal directions
+        y = sparse.bsr_mv(A, x)
+        assert float(y[-1]) == last and bool((y[:-1] == 5.0).all())
+        del y
+    P = sparse.bsr_zeros(nrow, nrow, wa.float32, device=device)
+    P.offsets = torch.zeros(nrow + 1, dtype=torch.int32, device=device)
+    P.offsets[-1] = 1
+    P.columns = tail[-1:].clone()
+    P.values, P.nnz = torch.ones(1, dtype=torch.float32, device=device), 1
+    assert dirichlet._project_in_place(A, P)
+    assert A.values[-7:].tolist() == [0.0] * 6 + [1.0]
+    assert bool((A.values[:-7] == 1.0).all())

@@ -250,6 +250,7 @@ __device__ __forceinline__ S wave_rows_product(int row0, int nrow, int lane, con
     const bool on = lane < RW && row < nrow;
     const int beg = on ? offsets[row] : 0;
     const int end = on ? offsets[row + 1] : 0;
+    const int len = end - beg;
     const int nnz = offsets[nrow];
     const int last = (nrow - row0 < RW ? nrow - row0 : RW) - 1;
     const int b0 = __builtin_amdgcn_readfirstlane(beg);
@@ -264,16 +265,17 @@ __device__ __forceinline__ S wave_rows_product(int row0, int nrow, int lane, con
         V4 v[CH];
 #pragma unroll
         for (int u = 0; u < CH; ++u) {
-            const int k = base + (u * kWave + lane) * 4;
-            if (k < e0) {
-                if (k + 3 < nnz) {
+            // unsigned: a piece of the last tile may start past the largest int
+            const unsigned k = (unsigned)base + (u * kWave + lane) * 4;
+            if (k < (unsigned)e0) {
+                if (k + 3 < (unsigned)nnz) {
                     c[u] = stream_load<STREAM>(reinterpret_cast<const I4*>(columns + k));
                     v[u] = stream_load<STREAM>(reinterpret_cast<const V4*>(values + k));
                 } else {
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        c[u][q] = k + q < nnz ? columns[k + q] : 0;
-                        v[u][q] = k + q < nnz ? values[k + q] : V(0);
+                        c[u][q] = k + q < (unsigned)nnz ? columns[k + q] : 0;
+                        v[u][q] = k + q < (unsigned)nnz ? values[k + q] : V(0);
                     }
                 }
             }
@@ -281,36 +283,36 @@ __device__ __forceinline__ S wave_rows_product(int row0, int nrow, int lane, con
         S4 xv[CH];
 #pragma unroll
         for (int u = 0; u < CH; ++u) {
-            const int k = base + (u * kWave + lane) * 4;
+            const unsigned k = (unsigned)base + (u * kWave + lane) * 4;
 #pragma unroll
             for (int q = 0; q < 4; ++q)
-                xv[u][q] = (k + q >= b0 && k + q < e0) ? x((size_t)c[u][q]) : S(0);
+                xv[u][q] = (k + q >= (unsigned)b0 && k + q < (unsigned)e0) ? x((size_t)c[u][q]) : S(0);
         }
 #pragma unroll
         for (int u = 0; u < CH; ++u) {
             const int k = (u * kWave + lane) * 4;
-            if (base + k < e0) {
+            if (k < e0 - base) {
                 *reinterpret_cast<V4*>(tile.v + k) = v[u];
                 *reinterpret_cast<S4*>(tile.x + k) = xv[u];
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        for (int k = beg; k < end; k += G) {
+        for (int k = 0; k < len; k += G) {
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const bool in = k + g < end;
-                const int i = (in ? k + g : beg) - base;
+                const bool in = k + g < len;
+                const int i = beg - base + (in ? k + g : 0);
                 const S t = fma((S)tile.v[i], tile.x[i], a[g]);
                 a[g] = in ? t : a[g];
             }
         }
     } else {
-        for (int k = beg; k < end; k += G) {
+        for (int k = 0; k < len; k += G) {
 #pragma unroll
             for (int g = 0; g < G; ++g)
-                if (k + g < end)
-                    a[g] = fma((S)values[k + g], x((size_t)columns[k + g]), a[g]);
+                if (k + g < len)
+                    a[g] = fma((S)values[beg + k + g], x((size_t)columns[beg + k + g]), a[g]);
         }
     }
 #pragma unroll

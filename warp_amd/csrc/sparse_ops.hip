@@ -945,8 +945,9 @@ __global__ __launch_bounds__(kBlock) void project_blocks_kernel(int nrow, const 
     const int lane = threadIdx.x % G;
     const int pr = p_offsets[r];
     const bool has_r = p_offsets[r + 1] > pr;
-    const int end = a_offsets[r + 1];
-    for (int b = a_offsets[r] + lane; b < end; b += G) {
+    const int beg = a_offsets[r], count = a_offsets[r + 1] - beg;
+    for (int k = lane; k < count; k += G) {  // from the row's start: a step past the end stays an int
+        const int b = beg + k;
         const int c = a_columns[b];
         if (c < 0 || c >= nrow)
             continue;
