@@ -700,8 +700,11 @@ __device__ __forceinline__ unsigned long long slot_bits(double v)
 }
 
 // Column window and block count of each workgroup's rows (their maxima go to the
-// state, for the LDS the solve needs), and empty slots.
-__global__ __launch_bounds__(kBlock) void cg_small_plan_kernel(int nrow, int rows, const int* __restrict__ offsets,
+// state, for the LDS the solve needs), and empty slots.  Bound by the latency of
+// its column loads, hence 1024 threads with four in flight each.
+constexpr int kPlanThreads = 1024;
+
+__global__ __launch_bounds__(kPlanThreads) void cg_small_plan_kernel(int nrow, int rows, const int* __restrict__ offsets,
                                                               const int* __restrict__ columns, CgWs ws)
 {
     __shared__ int s_lo, s_hi;
@@ -711,23 +714,36 @@ __global__ __launch_bounds__(kBlock) void cg_small_plan_kernel(int nrow, int row
     const int r0 = min(w * rows, nrow), r1 = min(r0 + rows, nrow);
     if (threadIdx.x == 0) {
         s_lo = r0;
-        s_hi = r1;
+        s_hi = r1 - 1;  // the last column
     }
     __syncthreads();
     const int b0 = offsets[r0], b1 = offsets[r1];
-    int lo = r0, hi = r1;
-    for (int b = b0 + threadIdx.x; b < b1; b += kBlock) {
-        const int c = columns[b];
-        lo = min(lo, c);
-        hi = max(hi, c + 1);
+    int lo = r0, hi = r1 - 1;
+    for (int k = threadIdx.x; k < b1 - b0; k += 4 * kPlanThreads) {
+        int c[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            c[u] = k + u * kPlanThreads < b1 - b0 ? columns[b0 + k + u * kPlanThreads] : lo;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            lo = min(lo, c[u]);
+            hi = max(hi, c[u]);
+        }
     }
-    atomicMin(&s_lo, lo);
-    atomicMax(&s_hi, hi);
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        lo = min(lo, __shfl_xor(lo, off));
+        hi = max(hi, __shfl_xor(hi, off));
+    }
+    if (threadIdx.x % kWave == 0) {
+        atomicMin(&s_lo, lo);
+        atomicMax(&s_hi, hi);
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         // columns outside the matrix: no window fits (the general kernels take the system as before)
-        const bool bad = s_lo < 0 || s_hi > nrow;
-        atomicMax(&ws.state->small_window, bad ? 0x7fffffff : s_hi - s_lo);
+        const bool bad = s_lo < 0 || s_hi >= nrow;
+        atomicMax(&ws.state->small_window, bad ? 0x7fffffff : s_hi + 1 - s_lo);
         atomicMax(&ws.state->small_blocks, b1 - b0);
     }
 }
@@ -1466,12 +1482,18 @@ template <typename S> const void* small_kernel(int br, int lanes, int prec)
 }
 
 // Solves by cg_small_kernel where the system fits; *solved = 0 with x untouched
-// otherwise.  The caller's stream is not capturing (the state is read back).
+// otherwise.  *initial then says whether the workspace holds the solve's initial
+// state (read back into *h) for the general kernels to go on from: so it is
+// where only the columns' window did not fit, and the one thing such a solve
+// pays is cg_small_plan_kernel (2D Poisson 250^2 in random numbering, 10
+// iterations: 383 us by the general kernels alone, 386 now; 412 against 347
+// when they began again).  The caller's stream is not capturing (the state is
+// read back).
 template <typename S>
 int cg_solve_small(CgLauncher<S>& L, double rtol, double atol, int maxiter, int check_every, CgState* h, int* cur_iter,
-                   int* solved)
+                   int* solved, int* initial)
 {
-    *solved = 0;
+    *solved = *initial = 0;
     const CgProblem& pb = L.pb;
     const int groups = small_groups<S>(pb);
     const void* kernel = groups ? small_kernel<S>(pb.br, L.g(), pb.prec_kind) : nullptr;
@@ -1486,9 +1508,10 @@ int cg_solve_small(CgLauncher<S>& L, double rtol, double atol, int maxiter, int 
     cg_state_init_kernel<<<1, 1, 0, L.stream>>>(L.ws, rtol, atol);
     WA_LAUNCH_CHECK();
     WA_TRY(L.init(1));
-    cg_small_plan_kernel<<<groups, kBlock, 0, L.stream>>>(pb.nrow, rows, pb.offsets, pb.columns, L.ws);
+    cg_small_plan_kernel<<<groups, kPlanThreads, 0, L.stream>>>(pb.nrow, rows, pb.offsets, pb.columns, L.ws);
     WA_LAUNCH_CHECK();
     WA_TRY(read_state(L.ws.state, h, L.stream));
+    *initial = 1;
     *cur_iter = 0;
     if (h->rr <= h->atol_sq) {
         *solved = 1;
@@ -1511,6 +1534,7 @@ int cg_solve_small(CgLauncher<S>& L, double rtol, double atol, int maxiter, int 
         (void)hipGetLastError();  // does not fit this device: the general kernels
         return kOk;
     }
+    *initial = 0;  // z, Ap and the state are written from here on
     cg_small_commit_kernel<S><<<(unsigned)ceil_div(n, kBlock), kBlock, 0, L.stream>>>(n, groups, (S*)pb.x, L.ws);
     WA_LAUNCH_CHECK();
     WA_TRY(read_state(L.ws.state, h, L.stream));
@@ -1543,14 +1567,15 @@ int cg_solve_impl(
     if (maxiter <= 0)
         maxiter = (int)n;
 
+    double rtol_v, atol_v;
+    get_tolerances(sizeof(S) == 8, tol, atol, &rtol_v, &atol_v);
+    CgState h;
+    int initial = 0;  // the state, r, z and p of the initial residual are there, and h holds the state
     if (check_every > 0 && restart <= 0 && !cb) {
-        double rtol_v, atol_v;
-        get_tolerances(sizeof(S) == 8, tol, atol, &rtol_v, &atol_v);
         CgLauncher<S> small{pb, ws, caller_stream};
         small.fused = true;
-        CgState h;
         int cur_iter = 0, solved = 0;
-        WA_TRY(cg_solve_small(small, rtol_v, atol_v, maxiter, check_every, &h, &cur_iter, &solved));
+        WA_TRY(cg_solve_small(small, rtol_v, atol_v, maxiter, check_every, &h, &cur_iter, &solved, &initial));
         if (solved) {
             if (iters_out)
                 *iters_out = cur_iter;
@@ -1578,11 +1603,11 @@ int cg_solve_impl(
             check_every = std::max(check_every, cycle);
     }
 
-    double rtol_v, atol_v;
-    get_tolerances(sizeof(S) == 8, tol, atol, &rtol_v, &atol_v);
-    cg_state_init_kernel<<<1, 1, 0, stream>>>(ws, rtol_v, atol_v);
-    WA_LAUNCH_CHECK();
-    WA_TRY(L.init(1));
+    if (!initial) {
+        cg_state_init_kernel<<<1, 1, 0, stream>>>(ws, rtol_v, atol_v);
+        WA_LAUNCH_CHECK();
+        WA_TRY(L.init(1));
+    }
 
     auto cycle_body = [&]() -> int {
         for (int k = 0; k < cycle; ++k)
@@ -1611,7 +1636,6 @@ int cg_solve_impl(
             WA_TRY(runner.run(group_of(k), 1, k == kDeviceGroup));
         }
         if (iters_out || rnorm_out || atol_out) {
-            CgState h;
             WA_TRY(read_state(ws.state, &h, stream));
             if (iters_out)
                 *iters_out = h.iter;
@@ -1623,8 +1647,8 @@ int cg_solve_impl(
         return kOk;
     }
 
-    CgState h;
-    WA_TRY(read_state(ws.state, &h, stream));
+    if (!initial)
+        WA_TRY(read_state(ws.state, &h, stream));
     const double atol_out_v = std::sqrt(h.atol_sq);
     int cur_iter = 0;
     if (cb)
