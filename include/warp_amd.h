@@ -487,7 +487,10 @@ typedef int (*warp_amd_cg_callback)(int iteration, double residual_norm, double 
 
 size_t warp_amd_cg_workspace_size(int64_t n, int scalar_size);
 /* byte offset inside the CG workspace of: 0 the iteration count (int32),
- * 1 r.r (double), 2 atol^2 (double) -- the device results of check_every == 0 */
+ * 1 r.r (double), 2 atol^2 (double) -- the device results of check_every == 0;
+ * 3 (int32) the largest column window that the plan of a one-launch solve found
+ * (0: no plan since the state was initialised) and 4 (int32) the workgroups of a
+ * one-launch solve that finished (0: the general kernels solved) */
 size_t warp_amd_cg_state_offset(int which);
 
 /* Preconditioned CG on a compact BSR matrix with 1x1 or 3x3 blocks.

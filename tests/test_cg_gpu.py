@@ -580,28 +580,41 @@ def test_cg_one_launch_nan_and_concurrent_streams(device):
         assert i == i0 and torch.equal(x, want)
 
 
-def test_cg_window_misfit_starts_once(device):
-    """A small system whose columns' window does not fit one launch (a random
-    numbering) goes on from the initial residual it has: one state and one
-    residual kernel, no more than with a callback, and the same bits."""
-    from torch.profiler import ProfilerActivity, profile
+def _solve_with_route(A, b, x, **kw):
+    """(results of cg, the plan's column window, finished workgroups of a one-launch solve)."""
+    from warp_amd import _native
 
-    r, c, v, b, nn = problems.poisson2d_q1(200, 1)
+    solver = linear.cg(A, b, x, run=False, **kw)
+    res = solver()
+    off = [_native.lib().warp_amd_cg_state_offset(k) for k in (3, 4)]
+    window, finished = (int(solver._ws[o:o + 4].view(torch.int32)) for o in off)
+    return res, window, finished
+
+
+def _renumbered_poisson(n, device):
+    r, c, v, b, nn = problems.poisson2d_q1(n, 1)
     r, c, v, b = (torch.from_numpy(t).to(device) for t in (r, c, v, b))
     perm = torch.randperm(nn, generator=torch.Generator().manual_seed(1)).to(device)
     keep = (r >= 0) & (c >= 0)
     A = sparse.bsr_zeros(nn, nn, wa.float32, device=device)
     sparse.bsr_set_from_triplets(A, perm[r[keep].long()].to(torch.int32), perm[c[keep].long()].to(torch.int32), v[keep])
     A.nnz_sync()
-    b = torch.empty_like(b).index_copy_(0, perm, b)
+    return A, torch.empty_like(b).index_copy_(0, perm, b)
+
+
+@pytest.mark.parametrize("n", [200])
+def test_cg_window_misfit_starts_once(device, n):
+    """A small system whose columns' window does not fit one launch (a random
+    numbering) goes on from the state and residual it has (the plan's window is
+    still in the state, which initialising again would clear), with the bits of
+    the general kernels."""
+    A, b = _renumbered_poisson(n, device)
     M = linear.preconditioner(A, "diag")
     runs = []
     for kw in (dict(), dict(callback=lambda *a: None)):
         x = torch.full_like(b, 0.01)
-        with profile(activities=[ProfilerActivity.CUDA]) as prof:
-            it, err, atol = linear.cg(A, b, x, tol=1e-5, atol=0.0, maxiter=60, M=M, **kw)
-        names = [e.name for e in prof.events()]
-        starts = [sum(k in n for n in names) for k in ("cg_state_init_kernel", "cg_init_kernel", "cg_small_kernel")]
-        runs.append((it, err, atol, x.cpu().numpy().tobytes(), starts))
+        res, window, finished = _solve_with_route(A, b, x, tol=1e-5, atol=0.0, maxiter=60, M=M, **kw)
+        runs.append((res, x.cpu().numpy().tobytes()))
+        assert finished == 0
+        assert (window > 0) == (not kw)
     assert runs[0] == runs[1]
-    assert runs[0][-1] == [1, 1, 0]

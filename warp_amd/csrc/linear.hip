@@ -1958,13 +1958,18 @@ WA_API size_t warp_amd_cg_workspace_size(int64_t n, int scalar_size)
 
 // Byte offsets of the device-resident scalars inside the CG workspace, so
 // callers can read them without a host copy of the layout:
-// 0 iterations (int32), 1 r.r (double), 2 atol^2 (double).
+// 0 iterations (int32), 1 r.r (double), 2 atol^2 (double); and what says which
+// kernels solved (int32): 3 the largest column window of the one-launch solve's
+// plan (0: no plan since the state was last initialised), 4 its workgroups that
+// finished (0: the general kernels solved).
 WA_API size_t warp_amd_cg_state_offset(int which)
 {
     switch (which) {
     case 0: return offsetof(wa::CgState, iter);
     case 1: return offsetof(wa::CgState, rr);
     case 2: return offsetof(wa::CgState, atol_sq);
+    case 3: return offsetof(wa::CgState, small_window);
+    case 4: return offsetof(wa::CgState, small_done);
     default: return 0;
     }
 }
