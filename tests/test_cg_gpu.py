@@ -602,10 +602,10 @@ def _renumbered_poisson(n, device):
     return A, torch.empty_like(b).index_copy_(0, perm, b)
 
 
-@pytest.mark.parametrize("n", [200])
+@pytest.mark.parametrize("n", [128, 200])
 def test_cg_window_misfit_starts_once(device, n):
-    """A small system whose columns' window does not fit one launch (a random
-    numbering) goes on from the state and residual it has (the plan's window is
+    """A small system whose columns' window is too large for one launch (a random
+    numbering; at 128 it fits the LDS, but is slower so) goes on from the state and residual it has (the plan's window is
     still in the state, which initialising again would clear), with the bits of
     the general kernels."""
     A, b = _renumbered_poisson(n, device)

@@ -683,6 +683,12 @@ constexpr int kSmallThreads = 512;
 constexpr int kSmallPer = 2;       // scalars per thread
 constexpr int kSmallLds = 144 * 1024;
 constexpr int kSmallSpins = 1 << 21;
+// Scalars of p that a workgroup's columns may span: it reads z for all of them
+// once an iteration.  Random numbering, us per iteration, two kernels / one
+// launch: 96^2 FP32 11.5 / 10.3, FP64 12.2 / 10.6; 112^2 12.2 / 12.2, 12.7 / 12.5;
+// 128^2 12.2 / 13.9, 12.8 / 12.9.  Systems numbered along their axes span half
+// of this at most.
+constexpr int kSmallMaxWindow = 12 * 1024;
 constexpr unsigned long long kSlotEmpty = 0x7ff8dead00c0ffeeull;  // a NaN no sum stores
 
 // Slot set of quantity q (0 p.Ap, 1 r.r, 2 r.z) and parity.  Every partial is
@@ -1517,7 +1523,7 @@ int cg_solve_small(CgLauncher<S>& L, double rtol, double atol, int maxiter, int 
         *solved = 1;
         return kOk;
     }
-    if (h->small_window > kSmallLds / (int)sizeof(S))
+    if ((int64_t)h->small_window * pb.br > kSmallMaxWindow)
         return kOk;
     const size_t lds = pb.br == 1 ? SmallLds<S, 1>(rows, h->small_blocks, h->small_window).bytes
                                   : SmallLds<S, 3>(rows, h->small_blocks, h->small_window).bytes;
