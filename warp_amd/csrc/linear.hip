@@ -35,6 +35,8 @@
 #include "bsr_core.h"
 
 #include <cmath>
+#include <condition_variable>
+#include <mutex>
 #include <vector>
 
 namespace wa {
@@ -675,10 +677,10 @@ __global__ void cg_state_init_kernel(CgWs ws, double rtol, double atol)
 // partials by the release fence, hence before anyone polls that set again.  z is
 // overwritten only after the p.Ap reduction, by when all have read the old one.
 //
-// The launch is cooperative (all workgroups resident), and every wait is
-// bounded: a workgroup that polls kSmallSpins times leaves without finishing, x
-// is only written by cg_small_commit_kernel once all have finished, and the host
-// then solves by the kernels above.
+// All workgroups are resident (SmallShare), and every wait is bounded: a
+// workgroup that polls kSmallSpins times leaves without finishing, x is only
+// written by cg_small_commit_kernel once all have finished, and the host then
+// solves by the kernels above.
 constexpr int kSmallThreads = 512;
 constexpr int kSmallPer = 2;       // scalars per thread
 constexpr int kSmallLds = 144 * 1024;
@@ -1487,6 +1489,86 @@ template <typename S> const void* small_kernel(int br, int lanes, int prec)
     return nullptr;
 }
 
+// What the one-launch solves in flight hold of a device.  Cooperative launches
+// of one process run one after another, whatever their streams (2D Poisson 128^2,
+// 80 iterations, eight threads: 511 us a solve, 332 by the general kernels, whose
+// launches overlap).  So only a solve with no other in flight is launched
+// cooperatively; the others are ordinary launches, resident all the same because
+// of what may be in flight at once: one workgroup for each compute unit, or two
+// where every workgroup in flight is one of which three fit (a unit that holds
+// one of them has room for another, wherever in its LDS and registers the first
+// lies).  Launches are dealt evenly to the XCDs, and any other kernel on the
+// device ends by itself, after which its units are free.  Further solves wait
+// here, in order of arrival; those inside entered with their streams drained, so
+// they always end.  us a solve of 80 iterations with 1 / 2 / 4 / 8 threads, by the
+// general kernels: 64^2 1113 / 667 / 381 / 310, 128^2 1108 / 656 / 381 / 321,
+// 250^2 1236 / 704 / 441 / 398; all cooperative: 535 / 454 / 444 / 440, 593 / 520 /
+// 511 / 511, 799 / 721 / 712 / 711; so: 570 / 287 / 193 / 179, 577 / 432 / 256 /
+// 250, 801 / 489 / 395 / 393.
+class SmallShare {
+    struct Device {
+        std::mutex lock;
+        std::condition_variable left;
+        uint64_t arrived = 0, entered = 0;
+        int held = 0;   // workgroups in flight
+        int whole = 0;  // those of which fewer than three fit a compute unit
+    };
+    static constexpr int kMaxDevices = 64;
+    static Device& device(int id)
+    {
+        static Device devices[kMaxDevices];
+        return devices[id];
+    }
+    Device* dev = nullptr;
+    int share = 0, whole = 0;
+
+public:
+    bool alone = false;
+
+    // false: not on this device (the caller takes the general kernels)
+    bool enter(int groups, const void* kernel, size_t lds)
+    {
+        int id = 0, units = 0, per_unit = 0;
+        if (hipGetDevice(&id) != hipSuccess || id < 0 || id >= kMaxDevices ||
+            hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, id) != hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_unit, kernel, kSmallThreads, lds) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        // whole eighths: the workgroups of a launch are dealt to 8 XCDs
+        const int need = (groups + 7) / 8 * 8;
+        if (need > units || per_unit < 1)
+            return false;
+        Device& d = device(id);
+        std::unique_lock<std::mutex> hold(d.lock);
+        const uint64_t ticket = d.arrived++;
+        d.left.wait(hold, [&] {
+            return ticket == d.entered && d.held + need <= (per_unit > 2 && d.whole == 0 ? 2 * units : units);
+        });
+        ++d.entered;
+        alone = d.held == 0;
+        dev = &d;
+        share = need;
+        whole = per_unit > 2 ? 0 : need;
+        d.held += share;
+        d.whole += whole;
+        d.left.notify_all();
+        return true;
+    }
+    SmallShare() = default;
+    SmallShare(const SmallShare&) = delete;
+    SmallShare& operator=(const SmallShare&) = delete;
+    ~SmallShare()
+    {
+        if (!dev)
+            return;
+        std::lock_guard<std::mutex> hold(dev->lock);
+        dev->held -= share;
+        dev->whole -= whole;
+        dev->left.notify_all();
+    }
+};
+
 // Solves by cg_small_kernel where the system fits; *solved = 0 with x untouched
 // otherwise.  *initial then says whether the workspace holds the solve's initial
 // state (read back into *h) for the general kernels to go on from: so it is
@@ -1534,9 +1616,12 @@ int cg_solve_small(CgLauncher<S>& L, double rtol, double atol, int maxiter, int 
     const S *values = (const S*)pb.values, *prec = (const S*)pb.prec, *x = (const S*)pb.x;
     const int *offsets = pb.offsets, *columns = pb.columns;
     void* args[] = {&nrow, &rows, &blocks, &window, &maxiter, &offsets, &columns, &values, &prec, &x, &L.ws};
+    SmallShare share;  // until the solve has ended (read_state below)
+    const dim3 grid((unsigned)groups), block(kSmallThreads);
     if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLds) != hipSuccess ||
-        hipLaunchCooperativeKernel(kernel, dim3((unsigned)groups), dim3(kSmallThreads), args, (unsigned)lds, L.stream) !=
-        hipSuccess) {
+        !share.enter(groups, kernel, lds) ||
+        (share.alone ? hipLaunchCooperativeKernel(kernel, grid, block, args, (unsigned)lds, L.stream)
+                     : hipLaunchKernel(kernel, grid, block, args, lds, L.stream)) != hipSuccess) {
         (void)hipGetLastError();  // does not fit this device: the general kernels
         return kOk;
     }
