@@ -524,6 +524,21 @@ int warp_amd_cg_solve_f64(
     void* workspace, size_t workspace_bytes, int* iterations, double* residual_norm, double* abs_tolerance,
     void* stream);
 
+/* The same without restart, graph and callback, with a limit on a small system's
+ * one-launch solve: a workgroup that has looked `polls` times for the others'
+ * sums leaves, x stays as it was, and the general kernels solve.  The functions
+ * above use 2^21 (seconds); 0 always takes the general kernels in the end. */
+int warp_amd_cg_solve_polls_f32(
+    int nrow, int block_size, const int* offsets, const int* columns, const float* values, int64_t nnz_hint,
+    int prec_kind, const float* prec, const float* b, float* x, double tol, double atol, int maxiter,
+    int check_every, int polls, void* workspace, size_t workspace_bytes, int* iterations, double* residual_norm,
+    double* abs_tolerance, void* stream);
+int warp_amd_cg_solve_polls_f64(
+    int nrow, int block_size, const int* offsets, const int* columns, const double* values, int64_t nnz_hint,
+    int prec_kind, const double* prec, const double* b, double* x, double tol, double atol, int maxiter,
+    int check_every, int polls, void* workspace, size_t workspace_bytes, int* iterations, double* residual_norm,
+    double* abs_tolerance, void* stream);
+
 /* Generic CG building blocks for caller-supplied operators.
  * *out = sum a[i] b[i] accumulated in FP64, deterministic (replaces TiledDot
  * block_dot_kernel / block_sum_kernel, linear.py:580-612); the workspace

@@ -683,3 +683,49 @@ def test_cg_one_launch_solves_overlap(device):
         took[threads] = min(took.get(threads, math.inf), time.perf_counter() - t)
     print(f"[cg one-launch] 40 solves each: 1 stream {took[1] * 1e3:.1f} ms, 4 streams {took[4] * 1e3:.1f} ms")
     assert took[4] < 2.6 * took[1]
+
+
+@pytest.mark.parametrize("polls,maxiter", [(0, 1), (0, 60), (1, 1), (1, 60), (3, 60)])
+@pytest.mark.parametrize("family,n,dtype", [("poisson", 90, torch.float32), ("elasticity", 9, torch.float64)])
+def test_cg_one_launch_falls_back(device, family, n, dtype, polls, maxiter):
+    """A one-launch solve whose waits run out (a limit of a few looks at the
+    others' sums: every workgroup leaves by itself, some after iterations of
+    their own) leaves x alone, and the general kernels give the bits they give
+    with a callback; if all looks succeeded, the one-launch solve's."""
+    import ctypes
+
+    from warp_amd import _native
+
+    if family == "elasticity":
+        r, c, v, b, nn = problems.elasticity3d_q1(n, device=device)
+        btype = wa.matrix((3, 3), wa.types.type_to_scalar(dtype))
+    else:
+        r, c, v, b, nn = problems.poisson2d_q1(n, 1)
+        r, c, v, b = (torch.from_numpy(t).to(device) for t in (r, c, v, b))
+        btype = wa.types.type_to_scalar(dtype)
+    A = sparse.bsr_zeros(nn, nn, btype, device=device)
+    sparse.bsr_set_from_triplets(A, r, c, v.to(dtype))
+    A.nnz_sync()
+    b = b.to(dtype)
+    M = linear.preconditioner(A, "diag")
+    want = []
+    for kw in (dict(), dict(callback=lambda *a: None)):
+        x = torch.full_like(b, 0.01)
+        res, _, finished = _solve_with_route(A, b, x, tol=1e-30, atol=0.0, maxiter=maxiter, M=M, **kw)
+        want.append((finished, res, x))
+    assert want[0][0] > 1 and want[1][0] == 0
+    lib = _native.lib()
+    x = torch.full_like(b, 0.01)
+    ws = torch.empty(lib.warp_amd_cg_workspace_size(x.numel(), x.element_size()), dtype=torch.uint8, device=device)
+    it, err, atol = ctypes.c_int(0), ctypes.c_double(0.0), ctypes.c_double(0.0)
+    _native.call("warp_amd_cg_solve_polls_f64" if dtype == torch.float64 else "warp_amd_cg_solve_polls_f32", nn,
+                 A.block_shape[0], A.offsets.data_ptr(), A.columns.data_ptr(), A.values.data_ptr(), int(A.nnz),
+                 linear.PREC_DIAG, M._prec_data.data_ptr(), b.data_ptr(), x.data_ptr(), 1e-30, 0.0, maxiter, 10, polls,
+                 ws.data_ptr(), ws.numel(), ctypes.byref(it), ctypes.byref(err), ctypes.byref(atol),
+                 _native.stream_of(device))
+    o = lib.warp_amd_cg_state_offset(4)
+    finished = int(ws[o:o + 4].view(torch.int32))
+    print(f"[cg fallback] {family} polls {polls}: {finished} workgroups finished after the solve's last start")
+    assert finished in (0, want[0][0]) and (polls > 0 or finished == 0)
+    _, res, xw = want[0] if finished else want[1]
+    assert (it.value, err.value, atol.value) == res and torch.equal(x, xw)

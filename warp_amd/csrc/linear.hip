@@ -678,13 +678,13 @@ __global__ void cg_state_init_kernel(CgWs ws, double rtol, double atol)
 // overwritten only after the p.Ap reduction, by when all have read the old one.
 //
 // All workgroups are resident (SmallShare), and every wait is bounded: a
-// workgroup that polls kSmallSpins times leaves without finishing, x is only
+// workgroup that polls kSmallPolls times leaves without finishing, x is only
 // written by cg_small_commit_kernel once all have finished, and the host then
 // solves by the kernels above.
 constexpr int kSmallThreads = 512;
 constexpr int kSmallPer = 2;       // scalars per thread
 constexpr int kSmallLds = 144 * 1024;
-constexpr int kSmallSpins = 1 << 21;
+constexpr int kSmallPolls = 1 << 21;
 // Scalars of p that a workgroup's columns may span: it reads z for all of them
 // once an iteration.  Random numbering, us per iteration, two kernels / one
 // launch: 96^2 FP32 11.5 / 10.3, FP64 12.2 / 10.6; 112^2 12.2 / 12.2, 12.7 / 12.5;
@@ -780,10 +780,12 @@ template <typename S, int BR> struct SmallLds {
 };
 
 // Sum of each of NV values over all threads of all `n` workgroups, bit-identical
-// everywhere; false where a wait ran out.  ORDER: what the workgroup has stored
+// everywhere; false where `polls` looks at the others' slots did not find them
+// all.  ORDER: what the workgroup has stored
 // for others is visible to them once they return.
 template <int NV, bool ORDER>
-__device__ __forceinline__ bool small_all_reduce(double (&v)[NV], int q0, int parity, int n, const CgWs& ws, double* red)
+__device__ __forceinline__ bool small_all_reduce(double (&v)[NV], int q0, int parity, int n, int polls, const CgWs& ws,
+                                                 double* red)
 {
     constexpr int kWaves = kSmallThreads / kWave;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
@@ -816,9 +818,12 @@ __device__ __forceinline__ bool small_all_reduce(double (&v)[NV], int q0, int pa
             }
             const int replica = (int)blockIdx.x % kSmallReplicas;
             constexpr int kPer = kSmallMaxGroups / kWave;
-            unsigned long long got[NV][kPer];
-            int spins = 0;
-            for (;;) {
+            unsigned long long got[NV][kPer] = {};
+            for (int look = 0;; ++look) {
+                if (look >= polls) {
+                    ok = false;
+                    break;
+                }
                 bool ready = true;
 #pragma unroll
                 for (int q = 0; q < NV; ++q)
@@ -830,10 +835,6 @@ __device__ __forceinline__ bool small_all_reduce(double (&v)[NV], int q0, int pa
                     }
                 if (__all(ready))
                     break;
-                if (++spins >= kSmallSpins) {
-                    ok = false;
-                    break;
-                }
             }
             if (ORDER)
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -864,7 +865,7 @@ __device__ __forceinline__ bool small_all_reduce(double (&v)[NV], int q0, int pa
 
 template <typename S, int BR, int G, int PREC>
 __global__ __launch_bounds__(kSmallThreads) void cg_small_kernel(
-    int nrow, int rows, int max_blocks, int max_window, int maxiter, const int* __restrict__ offsets,
+    int nrow, int rows, int max_blocks, int max_window, int maxiter, int polls, const int* __restrict__ offsets,
     const int* __restrict__ columns, const S* __restrict__ values, const S* __restrict__ prec,
     const S* __restrict__ x_in, CgWs ws
 )
@@ -959,7 +960,7 @@ __global__ __launch_bounds__(kSmallThreads) void cg_small_kernel(
             if (i < own)
                 s1[0] += (double)l_pown[i] * (double)l_ap[i];
         }
-        ok = small_all_reduce<1, false>(s1, 0, parity, n, ws, red);
+        ok = small_all_reduce<1, false>(s1, 0, parity, n, polls, ws, red);
         if (!ok)
             return;
         if (tid < 3 * kSmallReplicas && n > 1)  // everyone has read the other set for the last time
@@ -998,7 +999,7 @@ __global__ __launch_bounds__(kSmallThreads) void cg_small_kernel(
                 s2[1] += (double)r[u] * (double)z;
             }
         }
-        ok = small_all_reduce<2, true>(s2, 1, parity, n, ws, red);
+        ok = small_all_reduce<2, true>(s2, 1, parity, n, polls, ws, red);
         if (!ok)
             return;
         rr = s2[0];
@@ -1578,8 +1579,8 @@ public:
 // when they began again).  The caller's stream is not capturing (the state is
 // read back).
 template <typename S>
-int cg_solve_small(CgLauncher<S>& L, double rtol, double atol, int maxiter, int check_every, CgState* h, int* cur_iter,
-                   int* solved, int* initial)
+int cg_solve_small(CgLauncher<S>& L, double rtol, double atol, int maxiter, int check_every, int polls, CgState* h,
+                   int* cur_iter, int* solved, int* initial)
 {
     *solved = *initial = 0;
     const CgProblem& pb = L.pb;
@@ -1615,7 +1616,7 @@ int cg_solve_small(CgLauncher<S>& L, double rtol, double atol, int maxiter, int 
     int nrow = pb.nrow, blocks = h->small_blocks, window = h->small_window;
     const S *values = (const S*)pb.values, *prec = (const S*)pb.prec, *x = (const S*)pb.x;
     const int *offsets = pb.offsets, *columns = pb.columns;
-    void* args[] = {&nrow, &rows, &blocks, &window, &maxiter, &offsets, &columns, &values, &prec, &x, &L.ws};
+    void* args[] = {&nrow, &rows, &blocks, &window, &maxiter, &polls, &offsets, &columns, &values, &prec, &x, &L.ws};
     SmallShare share;  // until the solve has ended (read_state below)
     const dim3 grid((unsigned)groups), block(kSmallThreads);
     if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kSmallLds) != hipSuccess ||
@@ -1641,7 +1642,7 @@ template <typename S>
 int cg_solve_impl(
     const CgProblem& pb, double tol, double atol, int maxiter, int check_every, int restart, int use_graph,
     CgCallback cb, void* cb_user, void* workspace, size_t workspace_bytes, int* iters_out, double* rnorm_out,
-    double* atol_out, hipStream_t caller_stream
+    double* atol_out, hipStream_t caller_stream, int polls = kSmallPolls
 )
 {
     WA_REQUIRE(pb.br == 1 || pb.br == 3, "cg_solve: block size must be 1 or 3, got %d", pb.br);
@@ -1666,7 +1667,7 @@ int cg_solve_impl(
         CgLauncher<S> small{pb, ws, caller_stream};
         small.fused = true;
         int cur_iter = 0, solved = 0;
-        WA_TRY(cg_solve_small(small, rtol_v, atol_v, maxiter, check_every, &h, &cur_iter, &solved, &initial));
+        WA_TRY(cg_solve_small(small, rtol_v, atol_v, maxiter, check_every, polls, &h, &cur_iter, &solved, &initial));
         if (solved) {
             if (iters_out)
                 *iters_out = cur_iter;
@@ -2079,6 +2080,18 @@ WA_API size_t warp_amd_cg_state_offset(int which)
             pb, tol, atol, maxiter, check_every, restart, use_graph, callback, callback_user, workspace,              \
             workspace_bytes, iterations, residual_norm, abs_tolerance, wa::as_stream(stream)                          \
         );                                                                                                            \
+    }                                                                                                                 \
+    WA_API int warp_amd_cg_solve_polls_##SUFFIX(                                                                      \
+        int nrow, int block_size, const int* offsets, const int* columns, const S* values, int64_t nnz_hint,          \
+        int prec_kind, const S* prec, const S* b, S* x, double tol, double atol, int maxiter, int check_every,        \
+        int polls, void* workspace, size_t workspace_bytes, int* iterations, double* residual_norm,                   \
+        double* abs_tolerance, void* stream                                                                           \
+    )                                                                                                                 \
+    {                                                                                                                 \
+        wa::CgProblem pb{nrow, block_size, offsets, columns, values, nnz_hint, prec_kind, prec, b, x};                \
+        return wa::cg_solve_impl<S>(pb, tol, atol, maxiter, check_every, 0, 0, nullptr, nullptr, workspace,           \
+                                    workspace_bytes, iterations, residual_norm, abs_tolerance,                        \
+                                    wa::as_stream(stream), polls);                                                    \
     }                                                                                                                 \
     WA_API int warp_amd_dot_##SUFFIX(                                                                                 \
         int64_t n, const S* a, const S* b, double* out, void* workspace, size_t workspace_bytes, void* stream         \
