@@ -52,6 +52,20 @@ def test_host_only_queries():
     assert len(set(offs)) == 3
 
 
+def test_triplet_workspace_covers_both_bucketings():
+    """The workspace of an assembly has room for the two-level passes also where
+    one level is taken (32 bytes a triplet: row, two keys, bucket row and two
+    summed positions), so one sized for a problem serves the same rows or triplets
+    with fewer of the other."""
+    from warp_amd import _native
+
+    size = _native.lib().warp_amd_bsr_from_triplets_workspace_size
+    counts = (4096, 65_536, 65_537, 100_000, 786_432, 786_433, 2_000_000)
+    for rows in (1, 100, 512, 6144, 6145, 300_000, 33_000_000):
+        assert all(size(rows, t) >= 32 * t for t in counts), rows
+        assert all(size(rows, a) <= size(rows, b) for a, b in zip(counts, counts[1:])), rows
+
+
 def test_error_reporting_without_gpu():
     """Argument errors are reported before any device work."""
     from warp_amd import _native

@@ -1650,3 +1650,36 @@ def test_assembly_of_values_beyond_the_caches(device, bs, dtype, wdtype):
 def test_triplets_row_size_classes_scalar_f64(device, oracle_mod):
     """FP64 scalars (block size compiled in) over the same row lengths."""
     test_triplets_row_size_classes(device, oracle_mod, (), np.float64)
+
+
+def _check_assembly_vs_unique(A, rows, cols, vals):
+    """A against the sorted unique keys of the valid, nonzero triplets; whole-number values, so exact sums."""
+    nnz = A.nnz_sync()
+    keep = (rows >= 0) & (rows < A.nrow) & (cols >= 0) & (cols < A.ncol) & (vals != 0)
+    key, inv = torch.unique(rows[keep].long() * A.ncol + cols[keep].long(), sorted=True, return_inverse=True)
+    want = torch.zeros(key.numel(), dtype=vals.dtype, device=vals.device).index_add(0, inv, vals[keep])
+    assert nnz == key.numel()
+    assert int(A.offsets[0]) == 0
+    assert torch.equal(A.offsets[1:A.nrow + 1].long(), torch.cumsum(torch.bincount(key // A.ncol, minlength=A.nrow), 0))
+    assert torch.equal(A.columns[:nnz].long(), key % A.ncol)
+    assert torch.equal(A.values[:nnz], want)
+
+
+@pytest.mark.parametrize("T,nrow,dense", [
+    (1, 1, 0), (65_536, 1, 0), (65_537, 1, 0), (65_536, 3, 0), (65_537, 3, 0), (128 * 600, 600, 0),
+    (128 * 600 + 1, 600, 0), (65_537, 5000, 3), (200_000, 70_000, 1), (200_000, 70_000, 300), (786_432, 6144, 0),
+    (786_433, 6144, 0), (786_432 + 4097, 20_000, 7)])
+def test_assembly_bucketing_edges(device, T, nrow, dense):
+    """Either side of each line between one-level and two-level bucketing, few
+    rows, and rows that hold half of all triplets (the LDS row table: one row, a
+    few, more than a workgroup has slots to spare)."""
+    g = torch.Generator(device=device).manual_seed(T + nrow)
+    rows = torch.randint(-1, nrow + 1, (T,), generator=g, device=device)
+    if dense:
+        heavy = torch.randint(0, dense, (T,), generator=g, device=device) * (nrow // dense)
+        rows = torch.where(torch.rand(T, generator=g, device=device) < 0.5, heavy, rows)
+    cols = torch.randint(-1, 200, (T,), generator=g, device=device)
+    vals = torch.randint(-3, 4, (T,), generator=g, device=device).float()
+    A = sparse.bsr_zeros(nrow, 199, wa.float32, device=device)
+    sparse.bsr_set_from_triplets(A, rows.to(torch.int32), cols.to(torch.int32), vals)
+    _check_assembly_vs_unique(A, rows, cols, vals)

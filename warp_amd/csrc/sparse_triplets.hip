@@ -60,20 +60,28 @@ constexpr int kMinTile = 16384;
 // contiguously (~kSubTile / buckets keys per run) instead of key by key.
 constexpr int kStagedBuckets = 256;
 constexpr int kSubTile = 4096;
-// At most this many triplets are bucketed at one level, by a row histogram of
-// global atomics (row_rank): there the latency of the two-level passes' few
-// workgroups and extra launches counts more than the atomics.  Whole assembly,
-// two levels / one, us: 16 K triplets 104 / 65, 262 K in element order 126 / 78,
-// shuffled 123 / 91, 512 K shuffled 129 / 121, 1.0 M shuffled 149 / 157 (in
-// element order 151 / 97, but the order is not known here).
-constexpr int kSingleLevelMax = 3 << 18;
+// Triplets bucketed at one level, by a row histogram of global atomics
+// (row_rank): there the latency of the two-level passes' few workgroups and extra
+// launches counts more than the atomics.  Whole assembly, two levels / one, us:
+// 16 K triplets 104 / 65, 262 K in element order 126 / 78, shuffled 123 / 91,
+// 512 K shuffled 129 / 121, 1.0 M shuffled 149 / 157 (in element order 151 / 97,
+// but the order is not known here).  In few rows the atomics queue, and the
+// two-level passes count in LDS; shuffled, two levels / one: 786 K triplets at 128
+// a row 116 / 109, at 256 117 / 145, at 512 155 / 239; 262 K at 128 101 / 83, at 256
+// 107 / 113, in 128 rows 231 / 313; 64 K in any number of rows as fast or faster (in
+// 128 rows 152 / 124, in 2 2252 / 2207).
+inline bool single_level(int nrow, int T)
+{
+    return T <= (1 << 16) || (T <= (3 << 18) && T <= (int64_t)128 * nrow);
+}
 
 struct Partition {
     int shift = 0;
     int nb = 1;       // coarse buckets
     int tile = kMinTile;
     int ntiles = 1;
-    bool tiled = false;   // false: single-level bucketing with global atomics
+    bool tileable = false;  // the two-level passes can take the row count
+    bool tiled = false;   // they do; false: single-level bucketing with global atomics
     bool staged = false;  // LDS-staged, run-contiguous scatter (nb <= kStagedBuckets)
 };
 
@@ -89,7 +97,8 @@ Partition partition_of(int nrow, int T)
     p.nb = (int)buckets(p.shift);
     if (p.nb < 1)
         p.nb = 1;
-    p.tiled = (1 << p.shift) <= kMaxBucketRows && T > kSingleLevelMax && nrow > 0;
+    p.tileable = (1 << p.shift) <= kMaxBucketRows && T > 0 && nrow > 0;
+    p.tiled = p.tileable && !single_level(nrow, T);
     p.staged = p.staged && p.tiled;
     const int64_t per = (T + kMaxTiles - 1) / kMaxTiles;
     p.tile = (int)(per > kMinTile ? (per + kBlock - 1) / kBlock * kBlock : kMinTile);
@@ -124,14 +133,15 @@ TripletWs carve_ws(void* base, size_t bytes, int nrow, int T, bool own_summed, s
     Carve c(base, bytes);
     TripletWs w;
     w.part = partition_of(nrow, T);
-    const int64_t ntile_hist = w.part.tiled ? (int64_t)w.part.nb * w.part.ntiles + 1 : 1;
+    // room for both routes, so that a workspace serves smaller problems too
+    const int64_t ntile_hist = w.part.tileable ? (int64_t)w.part.nb * w.part.ntiles + 1 : 1;
     w.trow = c.take<int>((size_t)T);
     w.hist = c.take<int>((size_t)nrow + 1);
     w.counters = c.take<int>(kListCounters);  // right after hist: one fill clears both
     w.row_start = c.take<int>((size_t)nrow + 1);
     w.keys = c.take<uint64_t>((size_t)T);
     w.alt = c.take<uint64_t>((size_t)T);
-    w.brow = w.part.tiled ? c.take<int>((size_t)T) : nullptr;
+    w.brow = w.part.tileable ? c.take<int>((size_t)T) : nullptr;
     w.tile_offsets = c.take<int>((size_t)ntile_hist);
     w.large_rows = c.take<int>((size_t)nrow + 1);
     w.medium_rows = c.take<int>((size_t)nrow + 1);
@@ -175,12 +185,29 @@ __device__ __forceinline__ bool in_mask(int row, int col, const int* offsets, co
     return lo < end && columns[lo] == col;
 }
 
-// Position of the lane's triplet among those of row `key` (-1: none) counted
-// so far in hist: the first lane of every run of equal keys in the wave adds the
-// run's length with one atomic.  Element-ordered triplets repeat a row 4 to 8
-// times; shuffled ones pay one atomic each.
-__device__ __forceinline__ int row_rank(int key, int* hist)
+// Position of the thread's triplet among those of row `key` (-1: none) counted
+// so far in hist.  The first lane of every run of equal keys in the wave adds the
+// run's length (element-ordered triplets repeat a row 4 to 8 times) to the row's
+// count in an LDS hash table, and the table's rows go to hist with one atomic
+// each.  Without the table the triplets of dense rows queue at those rows'
+// counters.  Whole assembly of 786 K shuffled triplets in 65,536 rows, a share of
+// them in a few dense ones, us by two levels / one without / with the table: half
+// in 4 rows 8848 / 9760 / 8823, in 16 1890 / 2096 / 1872, a tenth in 4 1487 / 1657 /
+// 1493, all rows alike 119 / 104 / 107.
+constexpr int kRankSlots = 2 * kBlock;
+
+struct RankTable {
+    int row[kRankSlots];    // -1: free
+    int count[kRankSlots];  // triplets of the row, then where they start in it
+};
+
+__device__ __forceinline__ int row_rank(int key, int* hist, RankTable& table)
 {
+    for (int s = threadIdx.x; s < kRankSlots; s += kBlock) {
+        table.row[s] = -1;
+        table.count[s] = 0;
+    }
+    __syncthreads();
     const int lane = threadIdx.x & (kWave - 1);
     const int prev = __shfl_up(key, 1);
     const uint64_t heads = __ballot(lane == 0 || prev != key);
@@ -188,9 +215,25 @@ __device__ __forceinline__ int row_rank(int key, int* hist)
     const int first = kWave - 1 - __clzll((long long)upto);
     const uint64_t after = first < kWave - 1 ? heads >> (first + 1) : 0;
     const int len = after ? __ffsll((long long)after) : kWave - first;
-    int base = 0;
+    int slot = 0, base = 0;
+    if (lane == first && key >= 0) {
+        slot = (int)(((unsigned)key * 2654435769u) >> (32 - 9));
+        static_assert(kRankSlots == 1 << 9, "the hash gives 9 bits");
+        for (;;) {  // ends: at most kBlock rows in kRankSlots slots
+            const int old = atomicCAS(&table.row[slot], -1, key);
+            if (old == -1 || old == key)
+                break;
+            slot = (slot + 1) % kRankSlots;
+        }
+        base = atomicAdd(&table.count[slot], len);
+    }
+    __syncthreads();
+    for (int s = threadIdx.x; s < kRankSlots; s += kBlock)
+        if (table.row[s] >= 0)
+            table.count[s] = atomicAdd(&hist[table.row[s]], table.count[s]);
+    __syncthreads();
     if (lane == first && key >= 0)
-        base = atomicAdd(&hist[key], len);
+        base += table.count[slot];
     return __shfl(base, first) + lane - first;
 }
 
@@ -201,6 +244,7 @@ __global__ __launch_bounds__(kBlock) void classify_kernel(
     int* trow, int* hist, int* rank
 )
 {
+    __shared__ RankTable table;
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     const bool in = i < T;
     const int limit = tpl_count ? *tpl_count : T;
@@ -212,7 +256,7 @@ __global__ __launch_bounds__(kBlock) void classify_kernel(
         valid = in_mask(r, c, mask_offsets, mask_row_counts, mask_columns);
     if (valid && values && (v0 & zero_mask) == U(0))
         valid = !block_is_zero(values + (size_t)i * block_size, block_size, zero_mask);
-    const int k = row_rank(valid ? r : -1, hist);
+    const int k = row_rank(valid ? r : -1, hist, table);
     if (in) {
         trow[i] = valid ? r : -1;
         rank[i] = k;
