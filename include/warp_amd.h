@@ -764,9 +764,11 @@ int warp_amd_relu_pool2_bwd_bf16(int n, int ch, const float* d, const float* dp,
  * reference counterpart; training of the learned preconditioner):
  * dW[27][cin][cout] = sum_v x~[v + d_t][ci] dy[v][co], db[cout] = sum_v dy[v][co],
  * both overwritten.  x: the layer's BF16 input (in_mode 1: x + upsample(coarse),
- * rounded as the forward rounds it); dy: [m^3][cout], BF16 (_bf16) or FP32 and
- * rounded to BF16 in the workspace; FP32 accumulation; per-workgroup partials in the workspace added in a fixed order.
- * Channel pairs: 2-16, 16-32, 32-64, 64-64, 64-32, 32-16, 16-1. */
+ * rounded as the forward rounds it); dy: [m^3][cout], BF16 (_bf16; x, coarse and
+ * dy 16-byte aligned, of 2 channels or one to a voxel, anything else is refused)
+ * or FP32 and rounded to BF16 in the workspace; FP32 accumulation; per-workgroup
+ * partials in the workspace added in a fixed order.  Channel pairs: 2-16, 16-32,
+ * 32-64, 64-64, 64-32, 32-16, 16-1. */
 size_t warp_amd_conv3_mfma_wgrad_bf16_workspace_size(int m, int cin, int cout);
 int warp_amd_conv3_mfma_wgrad_bf16(int m, int cin, int cout, int in_mode, const void* x, const void* coarse,
                                    const void* dy, float* dW, float* db, void* workspace, size_t workspace_bytes,

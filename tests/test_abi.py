@@ -104,3 +104,24 @@ def test_cg_rejects_misaligned_workspace_without_gpu():
     assert st == -2
     assert b"16-byte aligned" in lib.warp_amd_last_error()
     lib.warp_amd_clear_error()
+
+
+@pytest.mark.parametrize("cin,cout,which,shift", [
+    (16, 32, "x", 8), (16, 32, "dy", 2), (32, 16, "coarse", 4), (16, 1, "x", 2), (16, 1, "coarse", 8), (16, 1, "dy", 1),
+    (2, 16, "x", 2), (2, 16, "dy", 8)])
+def test_wgrad_rejects_misaligned_operands_without_gpu(cin, cout, which, shift):
+    """The BF16 weight gradients read 16-byte vectors (one voxel where it has
+    fewer than 8 channels): other addresses are an argument error, raised before
+    any device work (the pointers are never dereferenced)."""
+    from warp_amd import _native
+
+    lib = _native.lib()
+    m, fake = 8, 1 << 20
+    ptr = {"x": fake, "coarse": fake, "dy": fake}
+    ptr[which] += shift
+    ws = lib.warp_amd_conv3_mfma_wgrad_bf16_workspace_size(m, cin, cout)
+    st = lib.warp_amd_conv3_mfma_wgrad_bf16(m, cin, cout, 1 if cin >= 16 else 0, ptr["x"], ptr["coarse"], ptr["dy"], fake,
+                                            fake, fake, ws, None)
+    assert st == -2
+    assert b"16-byte aligned" in lib.warp_amd_last_error()
+    lib.warp_amd_clear_error()

@@ -1521,6 +1521,28 @@ WA_API int warp_amd_unet_pack_input_bf16(int64_t nvox, const double* r, const fl
 }
 
 namespace {
+// Arguments checked: the weight gradients of the pair (cin, cout) from a BF16 dy.
+int wgrad_pair(int m, int cin, int cout, int in_mode, const void* x, const void* coarse, const void* dy, float* dW,
+               float* db, void* workspace, hipStream_t s)
+{
+    const unsigned short* xi = static_cast<const unsigned short*>(x);
+    const unsigned short* ci = static_cast<const unsigned short*>(coarse);
+    const unsigned short* di = static_cast<const unsigned short*>(dy);
+    float* pw = static_cast<float*>(workspace);
+#define WA_WGRAD_CASE(A, B)                                                                                      \
+    if (cin == A && cout == B)                                                                                   \
+        return wa::launch_wgrad<A, B>(m, in_mode, xi, ci, di, dW, db, pw, s);
+    WA_WGRAD_CASE(2, 16)
+    WA_WGRAD_CASE(16, 32)
+    WA_WGRAD_CASE(32, 64)
+    WA_WGRAD_CASE(64, 64)
+    WA_WGRAD_CASE(64, 32)
+    WA_WGRAD_CASE(32, 16)
+    WA_WGRAD_CASE(16, 1)
+#undef WA_WGRAD_CASE
+    return wa::kErrUnsupported;
+}
+
 bool wgrad_pair_supported(int ci, int co)
 {
     static const int pairs[][2] = {{2, 16}, {16, 32}, {32, 64}, {64, 64}, {64, 32}, {32, 16}, {16, 1}};
@@ -1552,7 +1574,8 @@ WA_API size_t warp_amd_conv3_mfma_wgrad_workspace_size(int m, int cin, int cout)
 // dy[v][co], db[cout] = sum_v dy[v][co], both overwritten.  x: BF16 layer
 // input [m^3][cin] (in_mode 1: x + upsample(coarse), as the forward formed
 // it); dy: BF16 [m^3][cout]; FP32 accumulation, partial sums per workgroup
-// added in a fixed order (deterministic).  x, coarse and dy 16-byte aligned.
+// added in a fixed order (deterministic).  x, coarse and dy 16-byte aligned (of 2
+// channels or one: to a voxel).
 WA_API int warp_amd_conv3_mfma_wgrad_bf16(int m, int cin, int cout, int in_mode, const void* x, const void* coarse,
                                           const void* dy, float* dW, float* db, void* workspace,
                                           size_t workspace_bytes, void* stream)
@@ -1563,23 +1586,13 @@ WA_API int warp_amd_conv3_mfma_wgrad_bf16(int m, int cin, int cout, int in_mode,
     WA_REQUIRE(x && dy && dW && db, "conv3_mfma_wgrad: null array");
     WA_REQUIRE(workspace && workspace_bytes >= warp_amd_conv3_mfma_wgrad_bf16_workspace_size(m, cin, cout),
                "conv3_mfma_wgrad: workspace too small");
-    const unsigned short* xi = static_cast<const unsigned short*>(x);
-    const unsigned short* ci = static_cast<const unsigned short*>(coarse);
-    const unsigned short* di = static_cast<const unsigned short*>(dy);
-    float* pw = static_cast<float*>(workspace);
-    hipStream_t s = wa::as_stream(stream);
-#define WA_WGRAD_CASE(A, B)                                                                                      \
-    if (cin == A && cout == B)                                                                                   \
-        return wa::launch_wgrad<A, B>(m, in_mode, xi, ci, di, dW, db, pw, s);
-    WA_WGRAD_CASE(2, 16)
-    WA_WGRAD_CASE(16, 32)
-    WA_WGRAD_CASE(32, 64)
-    WA_WGRAD_CASE(64, 64)
-    WA_WGRAD_CASE(64, 32)
-    WA_WGRAD_CASE(32, 16)
-    WA_WGRAD_CASE(16, 1)
-#undef WA_WGRAD_CASE
-    return wa::kErrUnsupported;
+    // vectors of 8 BF16 channels, or one voxel where there are fewer
+    const auto misaligned = [](const void* p, int channels) {
+        return (uintptr_t)p % (channels >= 8 ? 16 : 2 * channels) != 0;
+    };
+    WA_REQUIRE(!misaligned(x, cin) && !misaligned(dy, cout) && (in_mode == 0 || !misaligned(coarse, cin)),
+               "conv3_mfma_wgrad: x, coarse and dy must be 16-byte aligned (fewer than 8 channels: to a voxel)");
+    return wgrad_pair(m, cin, cout, in_mode, x, coarse, dy, dW, db, workspace, wa::as_stream(stream));
 }
 
 // The same with dy FP32 [m^3][cout], rounded to BF16 in the workspace first.
@@ -1592,10 +1605,11 @@ WA_API int warp_amd_conv3_mfma_wgrad(int m, int cin, int cout, int in_mode, cons
     WA_REQUIRE(x && dy && dW && db, "conv3_mfma_wgrad: null array");
     WA_REQUIRE(workspace && workspace_bytes >= warp_amd_conv3_mfma_wgrad_workspace_size(m, cin, cout),
                "conv3_mfma_wgrad: workspace too small");
+    WA_REQUIRE(in_mode == 0 || (in_mode == 1 && cin >= 16 && coarse), "conv3_mfma_wgrad: bad input mode");
     const size_t parts = warp_amd_conv3_mfma_wgrad_bf16_workspace_size(m, cin, cout);
     void* h = reinterpret_cast<void*>(wa::align_up((uintptr_t)workspace + parts, 16));
     WA_TRY(warp_amd_f32_to_bf16((int64_t)m * m * m * cout, dy, h, stream));
-    return warp_amd_conv3_mfma_wgrad_bf16(m, cin, cout, in_mode, x, coarse, h, dW, db, workspace, parts, stream);
+    return wgrad_pair(m, cin, cout, in_mode, x, coarse, h, dW, db, workspace, wa::as_stream(stream));
 }
 
 // out = y > 0 ? dy : 0 with y BF16 (the ReLU of a BF16 forward), dy and out FP32
