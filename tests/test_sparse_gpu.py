@@ -1683,3 +1683,58 @@ def test_assembly_bucketing_edges(device, T, nrow, dense):
     A = sparse.bsr_zeros(nrow, 199, wa.float32, device=device)
     sparse.bsr_set_from_triplets(A, rows.to(torch.int32), cols.to(torch.int32), vals)
     _check_assembly_vs_unique(A, rows, cols, vals)
+
+
+@pytest.mark.parametrize("T,nrow", [(786_433, 6000), (786_432 + 4096 * 3 + 17, 300_000), (1_000_003, 3_000_000),
+                                    (1_000_003, 12_000_000), (900_001, 30_000_000)])
+@pytest.mark.parametrize("form", ["count", "masked", "bytes1", "bytes2"])
+def test_two_level_assembly_forms(device, T, nrow, form):
+    """The two-level passes from just above their line (staged and unstaged
+    scatters, remainders of tiles and chunks, rows so sparse that a chunk of keys
+    spans far more than its window of rows) with a device count below T, a masked
+    destination, and 1- and 2-byte scalars pruned through the C entry."""
+    from warp_amd import _native
+
+    g = torch.Generator(device=device).manual_seed(T + nrow)
+    ncol = 5000
+    rows = torch.randint(-1, nrow + 1, (T,), generator=g, device=device)
+    cols = torch.randint(-1, ncol + 1, (T,), generator=g, device=device)
+    cols[::3] = 7  # repeated blocks also where rows are sparse
+    rows[::3] = rows[::3] // 2000 * 2000
+    r32, c32 = rows.to(torch.int32), cols.to(torch.int32)
+    vals = torch.randint(-3, 4, (T,), generator=g, device=device).float()
+    if form == "count":
+        n = T - 70_001
+        A = sparse.bsr_zeros(nrow, ncol, wa.float32, device=device)
+        sparse.bsr_set_from_triplets(A, r32, c32, vals, count=torch.tensor([n], dtype=torch.int32, device=device))
+        _check_assembly_vs_unique(A, rows[:n], cols[:n], vals[:n])
+    elif form == "masked":
+        A = sparse.bsr_zeros(nrow, ncol, wa.float32, device=device)
+        sparse.bsr_set_from_triplets(A, r32[: T // 2], c32[: T // 2], torch.ones(T // 2, device=device))
+        nnz = A.nnz_sync()
+        off, col = A.offsets.clone(), A.columns[:nnz].clone()
+        sparse.bsr_set_from_triplets(A, r32, c32, vals, topology="masked")
+        assert torch.equal(A.offsets, off) and torch.equal(A.columns[:nnz], col)
+        key = torch.repeat_interleave(torch.arange(nrow, device=device), (off[1:] - off[:-1]).long()) * ncol + col
+        ok = (rows >= 0) & (rows < nrow) & (cols >= 0) & (cols < ncol)
+        mine = rows[ok] * ncol + cols[ok]
+        at = torch.searchsorted(key, mine).clamp(max=nnz - 1)
+        hit = key[at] == mine
+        want = torch.zeros(nnz, device=device).index_add(0, at[hit], vals[ok][hit])
+        assert torch.equal(A.values[:nnz], want)
+    else:
+        size = int(form[-1])
+        v = torch.randint(0, 3, (T, 2), generator=g, device=device).to(torch.int8 if size == 1 else torch.int16)
+        mask = (1 << (8 * size)) - 1
+        off = torch.empty(nrow + 1, dtype=torch.int32, device=device)
+        col = torch.empty(T, dtype=torch.int32, device=device)
+        lib = _native.lib()
+        ws = torch.empty(lib.warp_amd_bsr_from_triplets_workspace_size(nrow, T), dtype=torch.uint8, device=device)
+        _native.call("warp_amd_bsr_from_triplets", 2, size, nrow, ncol, T, None, _native.ptr(r32), _native.ptr(c32),
+                     _native.ptr(v), mask, 0, None, None, _native.ptr(off), None, _native.ptr(col), None, None,
+                     _native.ptr(ws), ws.numel(), _native.stream_of(device))
+        ok = (rows >= 0) & (rows < nrow) & (cols >= 0) & (cols < ncol) & (v != 0).any(1)
+        key = torch.unique(rows[ok] * ncol + cols[ok], sorted=True)
+        assert int(off[-1]) == key.numel()
+        assert torch.equal(col[: key.numel()].long(), key % ncol)
+        assert torch.equal(off[1:].long(), torch.cumsum(torch.bincount(key // ncol, minlength=nrow), 0))
