@@ -160,6 +160,8 @@ def test_projection_in_place_equals_general_route(device, br, dtype, case, monke
             assert dirichlet._project_in_place(probe, P) == (case == "diagonal")
         fem.project_system_matrix(A, P)
         nnz = A.nnz_sync()
+        if case == "diagonal":  # zeros past the blocks on either route
+            assert A.values.shape[0] > nnz and not bool(A.values[nnz:].any())
         results.append((A.offsets.cpu(), A.columns[:nnz].cpu(), A.values[:nnz].cpu(), A.nnz))
     (o0, c0, v0, n0), (o1, c1, v1, n1) = results
     assert n0 == n1 and torch.equal(o0, o1) and torch.equal(c0, c1)

@@ -361,3 +361,21 @@ def test_fused_output_gradients_vs_torch(device, n, ch):
     up = dp.repeat_interleave(2, 0).repeat_interleave(2, 1).repeat_interleave(2, 2)
     total = skip + 0.125 * up
     assert torch.equal(out, torch.where(y.float() > 0, total, torch.zeros_like(total)).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("count", [1, 255, 257, 4099])
+def test_relu_mask_bf16_vs_torch(device, count):
+    """out = y > 0 ? dy : 0 with a BF16 y: zeros of both signs, NaN and infinities of y and dy included."""
+    g = torch.Generator(device=device).manual_seed(count)
+    y = torch.randn(count, generator=g, device=device).to(torch.bfloat16)
+    dy = torch.randn(count, generator=g, device=device)
+    special = torch.tensor([0.0, -0.0, float("nan"), float("inf"), -float("inf")], device=device)
+    n = min(count, 25)
+    y[:n] = special.repeat(5)[:n].to(torch.bfloat16)
+    dy[:n] = special.repeat_interleave(5)[:n]
+    out = torch.full((count + 1,), 7.0, device=device)
+    _native.call("warp_amd_relu_mask_bf16", count, _native.ptr(y), _native.ptr(dy), _native.ptr(out),
+                 _native.stream_of(device))
+    want = torch.where(y.float() > 0, dy, torch.zeros_like(dy))
+    torch.testing.assert_close(out[:count], want, rtol=0, atol=0, equal_nan=True)
+    assert float(out[count]) == 7.0

@@ -70,7 +70,8 @@ def project_system_rhs(system_matrix: BsrMatrix, system_rhs: torch.Tensor, proje
 
 def _project_in_place(A: BsrMatrix, P: BsrMatrix) -> bool:
     """The projection of a compact ``A`` by a block-diagonal ``P`` whose blocks all lie on ``A``'s diagonal: the
-    topology stays, and only the blocks of constrained rows and columns are read and written.  False, with nothing
+    topology stays, and only the blocks of constrained rows and columns are read and written (the others keep the
+    sign of their zeros, where the sums of the general route make every zero positive).  False, with nothing
     done, where that does not hold; the check reads two counts back, so never under graph capture."""
     if (
         A is P
@@ -99,7 +100,7 @@ def _project_in_place(A: BsrMatrix, P: BsrMatrix) -> bool:
     if foreign or nnz > min(A.columns.numel(), A.values.shape[0]):
         return False
     A.nnz, A._nnz_pending = nnz, False
-    A.values[nnz:].zero_()
+    A.values[nnz:].zero_()  # as bsr_assign leaves it: values of a matrix straight from its triplets reach past nnz
     _native.call("warp_amd_bsr_project_blocks", A.scalar_type.size, A.block_shape[0], A.nrow, nnz, a_off, a_col,
                  _native.ptr(A.values), p_off, _native.ptr(P.values), stream)
     return True
