@@ -1738,3 +1738,44 @@ def test_two_level_assembly_forms(device, T, nrow, form):
         assert int(off[-1]) == key.numel()
         assert torch.equal(col[: key.numel()].long(), key % ncol)
         assert torch.equal(off[1:].long(), torch.cumsum(torch.bincount(key // ncol, minlength=nrow), 0))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_bsr_mv_wave_tiles_of_long_rows(device, dtype):
+    """Large scalar matrices whose long rows lie together, so that whole tiles
+    exceed their LDS image, ragged last tile included: the bits of four lanes a
+    row, and no more than 1.6 times their time (measured 0.85; adding such tiles
+    with one lane a row took 4 times as long)."""
+    nrow = (1 << 21) + 11
+    g = torch.Generator(device=device).manual_seed(9)
+    counts = torch.randint(0, 4, (nrow,), generator=g, device=device)
+    counts[: nrow // 16] = 36
+    counts[-(nrow // 16):] = 36
+    off = torch.zeros(nrow + 1, dtype=torch.int64, device=device)
+    off[1:] = torch.cumsum(counts, 0)
+    nnz = int(off[-1])
+    assert 4 < nnz / nrow < 7.25
+    rows = torch.repeat_interleave(torch.arange(nrow, device=device), counts)
+    cols = (rows + torch.randint(-2000, 2000, (nnz,), generator=g, device=device)).clamp(0, nrow - 1)
+    A = sparse.bsr_zeros(nrow, nrow, wa.types.type_to_scalar(dtype), device=device)
+    A.offsets, A.columns, A.nnz = off.to(torch.int32), cols.to(torch.int32), nnz
+    A.values = torch.randn(nnz, generator=g, device=device, dtype=dtype)
+    x = torch.randn(nrow, generator=g, device=device, dtype=dtype)
+    y = torch.empty_like(x)
+    took = []
+    for kw in (dict(tile_size=4), dict()):
+        runs = []
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(10):
+                sparse.bsr_mv(A, x, y, **kw)
+            end.record()
+            end.synchronize()
+            runs.append(start.elapsed_time(end) * 100.0)
+        took.append(min(runs))
+        if kw:
+            want = y.clone()
+    assert torch.equal(y, want)
+    print(f"[long rows] {dtype}: four lanes a row {took[0]:.0f} us, chosen {took[1]:.0f} us")
+    assert took[1] < 1.6 * took[0]

@@ -209,7 +209,8 @@ inline BsrShape default_bsr_shape(int nrow, int br, int bc, int64_t nnz_hint)
 // 200^3 105 / 95, 256^3 241 / 200 (5.7 TB/s); FP64 128^3 41 / 33, 161^3 92 / 73,
 // 195^3 155 / 130.  FP64 tiles are half as long (RW = 32, CH = 1: their LDS
 // image is twice as large; 64 rows took 87 us at 161^3).  A tile whose entries
-// exceed the LDS image (rows far above the mean) is added from global memory.
+// exceed the LDS image (rows far above the mean) is added by lane groups: FP32,
+// 2^21 rows, one eighth of them of 36 entries 80 / 68 us, by one lane a row 338.
 // Persistent workgroups that load the next tile ahead were slower (262 us at
 // 256^3), as were non-temporal matrix loads wherever consecutive products meet
 // in the memory-side cache (30 us at 128^3).
@@ -308,12 +309,16 @@ __device__ __forceinline__ S wave_rows_product(int row0, int nrow, int lane, con
             }
         }
     } else {
-        for (int k = 0; k < len; k += G) {
+        constexpr int RPG = RW * G / kWave;
+        const RowAcc<S, RPG> acc = group_rows_product_f<S, 1, 1, G, RPG, V>(row0 + lane / G * RPG, nrow, lane % G,
+                                                                          offsets, nullptr, columns, values, x);
+        S v = S(0);
 #pragma unroll
-            for (int g = 0; g < G; ++g)
-                if (k + g < len)
-                    a[g] = fma((S)values[beg + k + g], x((size_t)columns[beg + k + g]), a[g]);
+        for (int e = 0; e < RPG; ++e) {
+            const S t = __shfl(acc.v[e], lane / RPG * G);
+            v = lane % RPG == e ? t : v;
         }
+        return on ? v : S(0);
     }
 #pragma unroll
     for (int off = G / 2; off > 0; off >>= 1)
