@@ -170,9 +170,10 @@ def test_projection_in_place_equals_general_route(device, br, dtype, case, monke
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("shift", [0, 1])
-@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1029])
+@pytest.mark.parametrize("n", [1, 3, 4, 1023, 1029, (32 << 20) + 3])
 def test_copy_and_rescale_vector_tails(device, n, shift, dtype):
-    """Value copies at the remainders of the 16-byte pass and at storage that is not 16-byte aligned."""
+    """Value copies at the remainders of the 16-byte pass, past the caches (more than 128 MB) and at storage that is
+    not 16-byte aligned."""
     btype = wa.types.type_to_scalar(dtype)
     A = sparse.bsr_identity(n, btype, device=device)
     store = torch.randn(n + shift + 5, dtype=dtype, device=device)

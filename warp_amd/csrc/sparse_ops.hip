@@ -839,14 +839,13 @@ template <typename S> __global__ __launch_bounds__(kBlock) void rescale_kernel(i
 // what limits a 4-byte-per-lane pass is the request rate.  On the 64.7M
 // scalars of the 64^3 elasticity matrix (518 MB moved): 139 us at 4 bytes per
 // lane, 87 with plain 16-byte accesses (8 vectors per thread: 130), 79 us
-// (6.5 TB/s) with non-temporal ones, which keep the once-touched stream from
-// displacing what the next kernel reads.
+// (6.5 TB/s) with non-temporal ones (past_caches).
 template <typename S> struct Vec16 {
     static constexpr int kV = 16 / (int)sizeof(S);
     typedef S type __attribute__((ext_vector_type(16 / sizeof(S))));
 };
 
-template <typename S>
+template <typename S, bool STREAM>
 __global__ __launch_bounds__(kBlock) void copy_scaled_vec_kernel(int64_t n, const S* __restrict__ src, S scale,
                                                                 S* __restrict__ dst)
 {
@@ -855,17 +854,17 @@ __global__ __launch_bounds__(kBlock) void copy_scaled_vec_kernel(int64_t n, cons
     const int64_t nv = n / kV;
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i < nv) {
-        V v = __builtin_nontemporal_load(reinterpret_cast<const V*>(src) + i);
+        V v = stream_load<STREAM>(reinterpret_cast<const V*>(src) + i);
 #pragma unroll
         for (int k = 0; k < kV; ++k)
             v[k] = scale * v[k];
-        __builtin_nontemporal_store(v, reinterpret_cast<V*>(dst) + i);
+        stream_store<STREAM>(v, reinterpret_cast<V*>(dst) + i);
     }
     if (i < n - nv * kV)
         dst[nv * kV + i] = scale * src[nv * kV + i];
 }
 
-template <typename S>
+template <typename S, bool STREAM>
 __global__ __launch_bounds__(kBlock) void rescale_vec_kernel(int64_t n, S* __restrict__ x, S beta)
 {
 #pragma clang fp contract(off)
@@ -875,20 +874,45 @@ __global__ __launch_bounds__(kBlock) void rescale_vec_kernel(int64_t n, S* __res
     const int64_t nv = n / kV;
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i < nv) {
-        V v = __builtin_nontemporal_load(reinterpret_cast<const V*>(x) + i);
+        V v = stream_load<STREAM>(reinterpret_cast<const V*>(x) + i);
 #pragma unroll
         for (int k = 0; k < kV; ++k)
             v[k] = zero + beta * v[k];
-        __builtin_nontemporal_store(v, reinterpret_cast<V*>(x) + i);
+        stream_store<STREAM>(v, reinterpret_cast<V*>(x) + i);
     }
     if (i < n - nv * kV)
         x[nv * kV + i] = zero + beta * x[nv * kV + i];
 }
 
+// Past the caches where source and destination together exceed the 256 MB
+// memory-side cache: below, the next kernel finds the values there.  Copy of the
+// values and a product with them, us at 4 bytes per lane / plain / non-temporal:
+// 36 MB of scalars 50 / 46 / 52, 70 MB 108 / 92 / 90, 108 MB of 3x3 blocks 76 / 63 /
+// 70, 144 MB of scalars 228 / 195 / 193, 259 MB of blocks 216 / 161 / 150.
+template <typename S> bool past_caches(int64_t n) { return 2 * n * (int64_t)sizeof(S) > ((int64_t)256 << 20); }
+
 // Workgroups of a vector pass over n scalars (at least one, for the tail).
 template <typename S> unsigned vec_blocks(int64_t n)
 {
     return (unsigned)std::max<int64_t>(1, ceil_div(n / Vec16<S>::kV, kBlock));
+}
+
+template <typename S> void launch_copy_scaled(int64_t n, const void* src, double scale, void* dst, hipStream_t s)
+{
+    if (past_caches<S>(n))
+        copy_scaled_vec_kernel<S, true><<<vec_blocks<S>(n), kBlock, 0, s>>>(n, static_cast<const S*>(src), (S)scale,
+                                                                           static_cast<S*>(dst));
+    else
+        copy_scaled_vec_kernel<S, false><<<vec_blocks<S>(n), kBlock, 0, s>>>(n, static_cast<const S*>(src), (S)scale,
+                                                                            static_cast<S*>(dst));
+}
+
+template <typename S> void launch_rescale(int64_t n, void* x, double beta, hipStream_t s)
+{
+    if (past_caches<S>(n))
+        rescale_vec_kernel<S, true><<<vec_blocks<S>(n), kBlock, 0, s>>>(n, static_cast<S*>(x), (S)beta);
+    else
+        rescale_vec_kernel<S, false><<<vec_blocks<S>(n), kBlock, 0, s>>>(n, static_cast<S*>(x), (S)beta);
 }
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
@@ -1238,11 +1262,9 @@ WA_API int warp_amd_copy_scaled_values(int src_scalar_size, int dst_scalar_size,
     hipStream_t s = wa::as_stream(stream);
     if (src_scalar_size == dst_scalar_size && wa::aligned16(src) && wa::aligned16(dst)) {
         if (src_scalar_size == 4)
-            wa::copy_scaled_vec_kernel<float><<<wa::vec_blocks<float>(n), wa::kBlock, 0, s>>>(
-                n, static_cast<const float*>(src), (float)scale, static_cast<float*>(dst));
+            wa::launch_copy_scaled<float>(n, src, scale, dst, s);
         else
-            wa::copy_scaled_vec_kernel<double><<<wa::vec_blocks<double>(n), wa::kBlock, 0, s>>>(
-                n, static_cast<const double*>(src), scale, static_cast<double*>(dst));
+            wa::launch_copy_scaled<double>(n, src, scale, dst, s);
         WA_LAUNCH_CHECK();
         return wa::kOk;
     }
@@ -1273,11 +1295,9 @@ WA_API int warp_amd_rescale_values(int scalar_size, int64_t n, void* x, double b
     hipStream_t s = wa::as_stream(stream);
     if (wa::aligned16(x)) {
         if (scalar_size == 4)
-            wa::rescale_vec_kernel<float><<<wa::vec_blocks<float>(n), wa::kBlock, 0, s>>>(n, static_cast<float*>(x),
-                                                                                       (float)beta);
+            wa::launch_rescale<float>(n, x, beta, s);
         else
-            wa::rescale_vec_kernel<double><<<wa::vec_blocks<double>(n), wa::kBlock, 0, s>>>(
-                n, static_cast<double*>(x), beta);
+            wa::launch_rescale<double>(n, x, beta, s);
         WA_LAUNCH_CHECK();
         return wa::kOk;
     }
