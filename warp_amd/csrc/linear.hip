@@ -1469,6 +1469,11 @@ template <typename S> int small_groups(const CgProblem& pb)
     return ceil_div(pb.nrow, g) * pb.br <= kSmallThreads * kSmallPer ? g : 0;
 }
 
+// The kernel of a block size, lanes per row and preconditioner; null where it is
+// not compiled: each form is a kernel of its own, so only the rows that grids and
+// meshes give have one (means above 2 and up to 32 entries of scalar rows, above 4
+// and up to 32 blocks of 3x3 rows); nearly diagonal and nearly dense systems stay
+// with the general kernels.
 template <typename S> const void* small_kernel(int br, int lanes, int prec)
 {
 #define WA_SMALL_PREC(BR, G)                                                                                          \

@@ -22,8 +22,8 @@
 //      ends (summed_block_offsets) when asked for, and per unique block
 //      values = v[i0] + v[i1] + ... sequentially in ascending triplet order
 //      (bit-identical to the reference CUDA order).
-// Few triplets, and matrices of more than 4096 * 4096 rows, use a single-level
-// row histogram with global atomics and a scatter for steps 1-4.
+// Few triplets (single_level), and matrices of more than 4096 * 8192 rows, use a
+// single-level row histogram with global atomics and a scatter for steps 1-4.
 #include "common.h"
 
 #include <algorithm>
