@@ -510,7 +510,12 @@ size_t warp_amd_cg_state_offset(int which);
  * iterations are launch-bound, run on a private stream and replay the cycles
  * between two residual checks as one HIP graph; larger systems and callers
  * whose stream is being captured launch directly (same iterates either
- * way).  x: initial guess in, solution out. */
+ * way).  Small systems (matrix within the LDS of 128 workgroups) with
+ * check_every > 0, no restart, callback or capture are solved in one launch
+ * instead: the same iteration with the FP64 sums in another order.  Solves on
+ * several streams run side by side as far as the device has room for their
+ * workgroups; the call waits for its turn beyond that.  x: initial guess in,
+ * solution out. */
 int warp_amd_cg_solve_f32(
     int nrow, int block_size, const int* offsets, const int* columns, const float* values, int64_t nnz_hint,
     int prec_kind, const float* prec, const float* b, float* x, double tol, double atol, int maxiter,

@@ -7,7 +7,8 @@ and loop semantics.  Two execution routes, both on the gfx950 library:
 
 * native: a compact BSR matrix with 1x1 or 3x3 blocks and no / Jacobi /
   block-Jacobi preconditioner is solved by the library's own host loop over
-  three fused kernels per iteration (``warp_amd_cg_solve_*``);
+  three fused kernels per iteration, small systems in one launch
+  (``warp_amd_cg_solve_*``);
 * generic: any other ``LinearOperator`` (dense, diagonal, user ``matvec``)
   is driven from Python with the library's dot / update primitives.
 
