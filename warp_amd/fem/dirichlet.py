@@ -97,9 +97,12 @@ def _project_in_place(A: BsrMatrix, P: BsrMatrix) -> bool:
     _native.call("warp_amd_bsr_project_check", A.nrow, a_off, a_col, p_off, _native.ptr(P.columns),
                  _native.ptr(out), stream)
     foreign, nnz = out.tolist()
-    if foreign or nnz > min(A.columns.numel(), A.values.shape[0]):
+    if nnz == 0 or nnz > min(A.columns.numel(), A.values.shape[0]):
         return False
     A.nnz, A._nnz_pending = nnz, False
+    if foreign:
+        A._nnz_read = nnz
+        return False
     A.values[nnz:].zero_()  # as bsr_assign leaves it: values of a matrix straight from its triplets reach past nnz
     _native.call("warp_amd_bsr_project_blocks", A.scalar_type.size, A.block_shape[0], A.nrow, nnz, a_off, a_col,
                  _native.ptr(A.values), p_off, _native.ptr(P.values), stream)
@@ -110,7 +113,10 @@ def project_system_matrix(system_matrix: BsrMatrix, projector_matrix: BsrMatrix)
     """``A = (I - P) A (I - P) + P`` in place (dirichlet.py:93-104)."""
     if _project_in_place(system_matrix, projector_matrix):
         return
+    read = system_matrix.__dict__.pop("_nnz_read", None)
     complement_system = bsr_copy(system_matrix)
+    if read is not None:
+        complement_system._nnz_read = read  # the check's read-back stands in for the first product's
     bsr_mm(x=projector_matrix, y=system_matrix, z=complement_system, alpha=-1.0, beta=1.0)
     bsr_assign(dest=system_matrix, src=complement_system)
     bsr_axpy(x=projector_matrix, y=system_matrix)

@@ -168,6 +168,10 @@ class BsrMatrix:
 
     def nnz_sync(self) -> int:
         """Wait for the pending ``offsets[nrow]`` transfer (or start one) and return the exact nnz."""
+        read = self.__dict__.pop("_nnz_read", None)
+        if read is not None:  # just read back by the caller that made this matrix
+            self.nnz, self._nnz_pending = read, False
+            return read
         if self._nnz_event is None or not getattr(self, "_nnz_pending", False):
             self._copy_nnz_async()
         if self._nnz_event is not None:
