@@ -419,7 +419,10 @@ __global__ __launch_bounds__(kBlock) void bsr_mv_transpose_kernel(
 // the same lines of values.
 // us per product (lanes as in bsr_mv), search alone / mirror tried first:
 // elasticity 53^3 91 / 51, 64^3 181 / 107, 2D Poisson 400^2 18 / 8.8, FP64
-// 7-point 100^3 75 / 49; elasticity 53^3 in random numbering 354 / 352.  Runs of
+// 7-point 100^3 75 / 49; elasticity 53^3 in random numbering 354 / 352.  Scalar
+// rows of some 13 random entries: 50 K rows FP64 31.3 / 32.3, 300 K 225 / 221;
+// trying the mirror only where both rows are equally long gave 32.0 and 219, but
+// lost what the dense row of an arrow matrix gains (20 K rows 5.1 / 3.3 ms).  Runs of
 // 1 / 8 / 128 workgroups: 78 / 69 / 57 at 53^3.  Loading the values before the
 // column is known (random numbering: 460) or two or four rows per group (59 and
 // 73 at 53^3) were slower.
