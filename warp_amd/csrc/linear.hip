@@ -1522,7 +1522,7 @@ class SmallShare {
     static constexpr int kMaxDevices = 64;
     static Device& device(int id)
     {
-        static Device devices[kMaxDevices];
+        static Device* devices = new Device[kMaxDevices];  // never freed: threads may still solve at exit
         return devices[id];
     }
     Device* dev = nullptr;
